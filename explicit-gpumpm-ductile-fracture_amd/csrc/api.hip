@@ -432,7 +432,7 @@ static void free_particles(mpmx_ctx* c) {
         dfree(m.mass); dfree(m.id);
     }
     dfree(c->sigma); dfree(c->FP); dfree(c->vol); dfree(c->cg_col); dfree(c->payload); dfree(c->pbound); dfree(c->cbound);
-    dfree(c->keys); dfree(c->keys_alt); dfree(c->keys_next); dfree(c->vals); dfree(c->vals_alt); dfree(c->hist);
+    dfree(c->keys); dfree(c->keys_alt); dfree(c->keys_next); dfree(c->vals); dfree(c->vals_alt); dfree(c->hist); dfree(c->hist2);
     dfree(c->mv_tcount); dfree(c->mv_toff); dfree(c->mv_old); dfree(c->mv_slot);
     dfree(c->mv_tbound); dfree(c->mv_cpre); dfree(c->mv_cmask);
     for (int b = 0; b < 2; ++b) { dfree(c->mv_key[b]); dfree(c->mv_val[b]); }
@@ -808,6 +808,7 @@ static mpmx_status upload_particles(mpmx_ctx* c, const int64_t* counts, const st
     HIPCHK(c, dalloc(&c->vals_alt, n));
     c->sort_tiles = (int)((n + 2047) / 2048);
     HIPCHK(c, dalloc(&c->hist, (int64_t)256 * c->sort_tiles));
+    HIPCHK(c, dalloc(&c->hist2, (int64_t)256 * c->sort_tiles));
     HIPCHK(c, dalloc(&c->mv_tcount, c->sort_tiles));
     HIPCHK(c, dalloc(&c->mv_toff, c->sort_tiles));
     HIPCHK(c, dalloc(&c->mv_old, n));
@@ -874,6 +875,7 @@ static mpmx_status upload_particles(mpmx_ctx* c, const int64_t* counts, const st
     else k_upload_fp32<<<(int)((n + 255) / 256), 256, 0, c->stream>>>(c->ps[0], dx_, dv_, dm_, (int)n);
     HIPCHK(c, hipGetLastError());
     std::memset(c->hc, 0, sizeof(DevCounts));
+    c->hc->movers = -1;   // not counted yet
     HIPCHK(c, hipMemcpyAsync(c->dc, c->hc, sizeof(DevCounts), hipMemcpyHostToDevice, c->stream));
     // keys, first canonical sort, first tables (with the bound as capacity)
     HIPCHK(c, compute_keys(c));
@@ -1018,6 +1020,7 @@ static mpmx_status capture_substep(mpmx_ctx* c, double dt, int iters) {
     const int p = c->cur;
     choose_sort_path(c);
     const bool by_movers = c->sort_by_movers && c->old_keys_sorted;   // the path sort_keys takes
+    const bool few_movers = c->few_movers;
     uint32_t* const keys0 = c->keys;
     uint32_t* const keys1 = c->keys_alt;
     auto& G = c->graphs[p];
@@ -1067,6 +1070,7 @@ static mpmx_status capture_substep(mpmx_ctx* c, double dt, int iters) {
     G.dt = (float)dt;
     G.iters = iters;
     G.by_movers = by_movers;
+    G.few_movers = few_movers;
     G.blocks = c->hc->num_blocks;
     return MPMX_OK;
 }
@@ -1081,7 +1085,7 @@ static mpmx_status substep_graph(mpmx_ctx* c, double dt) {
     choose_sort_path(c);
     const bool by_movers = c->sort_by_movers && c->old_keys_sorted;
     if (!G.valid || G.dt != (float)dt || G.iters != want || c->hc->num_blocks > G.blocks + G.blocks / 4 + 64 ||
-        G.by_movers != by_movers) {
+        G.by_movers != by_movers || (by_movers && G.few_movers != c->few_movers)) {
         mpmx_status s = capture_substep(c, dt, want);
         if (s != MPMX_OK) return s;
     }

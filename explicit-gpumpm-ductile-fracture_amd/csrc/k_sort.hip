@@ -153,6 +153,37 @@ hipError_t scan_exclusive(mpmx_ctx* c, const int* in, int* out, int64_t n_cap, c
     return hipGetLastError();
 }
 
+// One launch, out of place, for a device count of some hundred tiles at most:
+// every tile adds up all entries before it itself (coalesced loads, a few
+// hundred per thread for the last tile) instead of waiting for a launch of
+// tile sums.
+__global__ __launch_bounds__(256) void k_scan_direct(const int* __restrict__ in, int* __restrict__ out,
+                                                     const int* __restrict__ n_dev, int64_t cap) {
+    __shared__ int lds4[4];
+    int64_t n = *n_dev;
+    n = n < cap ? n : cap;
+    const int64_t base = (int64_t)blockIdx.x * kScanTile;
+    if (base >= n) return;
+    int pre = 0;
+    for (int64_t i = threadIdx.x; i < base; i += 256) pre += in[i];
+    int offset, total;
+    (void)block_excl_scan256(pre, offset, lds4);
+    int v[kScanPer], local = 0;
+#pragma unroll
+    for (int q = 0; q < kScanPer; ++q) {
+        const int64_t i = base + (int64_t)threadIdx.x * kScanPer + q;
+        v[q] = (i < n) ? in[i] : 0;
+        local += v[q];
+    }
+    int off = block_excl_scan256(local, total, lds4) + offset;
+#pragma unroll
+    for (int q = 0; q < kScanPer; ++q) {
+        const int64_t i = base + (int64_t)threadIdx.x * kScanPer + q;
+        if (i < n) out[i] = off;
+        off += v[q];
+    }
+}
+
 // up to three scans of n entries each in the same two launches (in place
 // allowed); array y uses the tile sums at sums + y * tiles
 __global__ __launch_bounds__(256) void k_scan_reduce3(ScanSet3 a, int* sums, int64_t n) {
@@ -411,21 +442,31 @@ __device__ __forceinline__ uint64_t spread4(uint64_t x) {
     return x;
 }
 
-// the movers in slot order: new key, previous key, slot (toff: the tiles'
-// exclusive mover offsets); per 64 slots, the movers before them (cpre) and
-// which of them move (cmask), so that the movers before any slot s are
-// cpre[s / 64] + popcount(cmask[s / 64] below bit s % 64)
+// the movers in slot order: new key, previous key, slot; per 64 slots, the
+// movers before them (cpre) and which of them move (cmask), so that the movers
+// before any slot s are cpre[s / 64] + popcount(cmask[s / 64] below bit s %
+// 64).  Each tile adds up the counts of the tiles before it itself (toff keeps
+// the sum; a few loads per thread even at 13 M particles) instead of waiting
+// for two scan launches; the last tile leaves the total in *m_dev.
 __global__ __launch_bounds__(kRsThreads) void k_mover_list(const uint32_t* __restrict__ old,
                                                            const uint32_t* __restrict__ cur, int n,
-                                                           const int* __restrict__ toff, uint32_t* __restrict__ mkey,
+                                                           const int* __restrict__ tcount, int* __restrict__ toff,
+                                                           int* __restrict__ m_dev, uint32_t* __restrict__ mkey,
                                                            uint32_t* __restrict__ mold, uint32_t* __restrict__ mslot,
                                                            int* __restrict__ cpre, uint64_t* __restrict__ cmask) {
     __shared__ int lds4[4];
     uint32_t ko[kRsItems], kn[kRsItems];
     const int base = blockIdx.x * kRsTile;
     const unsigned bits = mover_bits(old, cur, base, n, ko, kn);
+    int pre = 0, before;
+    for (int t = threadIdx.x; t < (int)blockIdx.x; t += kRsThreads) pre += tcount[t];
+    (void)block_excl_scan256(pre, before, lds4);
     int mr[2], total;
-    half_ranks(bits, toff[blockIdx.x], mr, total, lds4);
+    half_ranks(bits, before, mr, total, lds4);
+    if (threadIdx.x == 0) {
+        toff[blockIdx.x] = before;
+        if (blockIdx.x == gridDim.x - 1) *m_dev = before + total;
+    }
     const int lane = threadIdx.x & 63;
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
@@ -536,48 +577,60 @@ __device__ __forceinline__ int table_bound(const OldTables& t, uint32_t k, bool 
 // of them after i), for K < P the slots up to the last previous key <= K
 // (all before i); with the tables of the previous sort (tb set) it comes
 // from the cell starts, else from a search of the previous keys.  Threads
-// 0 .. tiles also give each tile of slots the sorted movers that precede its
-// first slot (tbound, for k_place_stayers).
-__global__ __launch_bounds__(kRsThreads) void k_place_movers(const uint32_t* __restrict__ old, int n,
-                                                             const uint32_t* __restrict__ skey,
-                                                             const uint32_t* __restrict__ sr0,
-                                                             const uint32_t* __restrict__ mold,
-                                                             const uint32_t* __restrict__ mslot, const int* m_dev,
-                                                             const int* __restrict__ cpre,
-                                                             const uint64_t* __restrict__ cmask,
-                                                             const int* __restrict__ toff, int tiles,
-                                                             int* __restrict__ tbound, OldTables tb, bool use_tables,
-                                                             uint32_t* __restrict__ okeys, uint32_t* __restrict__ perm) {
-    int m = *m_dev;
-    m = m < n ? m : n;
-    const int gid = blockIdx.x * blockDim.x + threadIdx.x;
-    // the tile bounds go to the last threads of the grid, which mostly hold
-    // no mover: their searches then run beside the movers' own
-    const int tq = gid - (int)(gridDim.x * blockDim.x - (tiles + 1));
-    if (tq >= 0 && tq < tiles) {
-        const int t0 = toff[tq];
-        tbound[tq] = search_near<kPair>(skey, sr0, m, old[tq * kRsTile], (uint32_t)t0, t0);
-    } else if (tq == tiles) {
-        tbound[tiles] = m;
-    }
+// gid, gid + threads, ... of the movers.
+struct MoverSet {
+    const uint32_t* old;     // previous sort's keys
+    int n;
+    const uint32_t* skey;    // sorted movers: new key, list index
+    const uint32_t* sr0;
+    const uint32_t* mold;    // by list index: previous key, slot
+    const uint32_t* mslot;
+    const int* cpre;
+    const uint64_t* cmask;
+};
+__device__ __forceinline__ void place_movers(const MoverSet& M, int m, int gid, int threads, const OldTables& tb,
+                                             bool use_tables, uint32_t* __restrict__ okeys,
+                                             uint32_t* __restrict__ perm) {
+    const int n = M.n;
     if (use_tables) {
         const int np = *tb.num_page;
         use_tables = np <= tb.cap_p;   // truncated tables (a capacity error) are not used
     }
-    for (int r = gid; r < m; r += gridDim.x * blockDim.x) {
-        const uint32_t K = skey[r];
-        const int r0 = (int)sr0[r];
-        const int i = (int)mslot[r0];
-        const bool up = K > mold[r0];
+    for (int r = gid; r < m; r += threads) {
+        const uint32_t K = M.skey[r];
+        const int r0 = (int)M.sr0[r];
+        const int i = (int)M.mslot[r0];
+        const bool up = K > M.mold[r0];
         int all;
         if (use_tables) all = table_bound(tb, K, !up);
-        else all = up ? search_near<kLower>(old, nullptr, n, K, 0u, i + 1) : search_near<kUpper>(old, nullptr, n, K, 0u, i - 1);
+        else all = up ? search_near<kLower>(M.old, nullptr, n, K, 0u, i + 1) : search_near<kUpper>(M.old, nullptr, n, K, 0u, i - 1);
         all = all < 0 ? 0 : (all > n ? n : all);
-        const int pos = r + all - movers_before(cpre, cmask, all, n, m);
+        const int pos = r + all - movers_before(M.cpre, M.cmask, all, n, m);
         if (pos < 0 || pos >= n) continue;   // only if the previous keys were not sorted
         okeys[pos] = K;
         perm[pos] = (uint32_t)i;
     }
+}
+
+// the movers' places; the last threads of the grid, which mostly hold no
+// mover, also give each tile of slots the sorted movers that precede its
+// first slot (tbound, for the stayers), so that their searches run beside the
+// movers' own
+__global__ __launch_bounds__(kRsThreads) void k_place_movers(MoverSet M, const int* m_dev,
+                                                             const int* __restrict__ toff, int tiles,
+                                                             int* __restrict__ tbound, OldTables tb, bool use_tables,
+                                                             uint32_t* __restrict__ okeys, uint32_t* __restrict__ perm) {
+    int m = *m_dev;
+    m = m < M.n ? m : M.n;
+    const int gid = blockIdx.x * blockDim.x + threadIdx.x;
+    const int tq = gid - (int)(gridDim.x * blockDim.x - (tiles + 1));
+    if (tq >= 0 && tq < tiles) {
+        const int t0 = toff[tq];
+        tbound[tq] = search_near<kPair>(M.skey, M.sr0, m, M.old[tq * kRsTile], (uint32_t)t0, t0);
+    } else if (tq == tiles) {
+        tbound[tiles] = m;
+    }
+    place_movers(M, m, gid, gridDim.x * blockDim.x, tb, use_tables, okeys, perm);
 }
 
 // The stayers' places: stayer i (key k, m_i movers in slots before it) comes
@@ -587,36 +640,37 @@ __global__ __launch_bounds__(kRsThreads) void k_place_movers(const uint32_t* __r
 // when they fit; in each run of 4 slots of a thread the stayers come in
 // order, so each one's c continues from the last.
 constexpr int kPlaceStage = 1024;
-__global__ __launch_bounds__(kRsThreads) void k_place_stayers(const uint32_t* __restrict__ old,
-                                                              const uint32_t* __restrict__ cur, int n,
-                                                              const int* __restrict__ toff,
-                                                              const int* __restrict__ tbound,
-                                                              const uint32_t* __restrict__ skey,
-                                                              const uint32_t* __restrict__ sr0, const int* m_dev,
-                                                              uint32_t* __restrict__ okeys, uint32_t* __restrict__ perm) {
-    __shared__ int lds4[4];
-    __shared__ uint32_t stk[kPlaceStage], stv[kPlaceStage];
-    int m = *m_dev;
-    m = m < n ? m : n;
+struct StayerLds {
+    int lds4[4];
+    uint32_t stk[kPlaceStage], stv[kPlaceStage];
+};
+__device__ __forceinline__ void place_stayers(const MoverSet& M, const uint32_t* __restrict__ cur, int m, int tile,
+                                              const int* __restrict__ toff, const int* __restrict__ tbound,
+                                              uint32_t* __restrict__ okeys, uint32_t* __restrict__ perm,
+                                              StayerLds& sm) {
+    const int n = M.n;
+    int* const lds4 = sm.lds4;
+    uint32_t* const stk = sm.stk;
+    uint32_t* const stv = sm.stv;
     uint32_t ko[kRsItems], kn[kRsItems];
-    const int base = blockIdx.x * kRsTile;
-    const unsigned bits = mover_bits(old, cur, base, n, ko, kn);
+    const int base = tile * kRsTile;
+    const unsigned bits = mover_bits(M.old, cur, base, n, ko, kn);
     int mr[2], total;
-    half_ranks(bits, toff[blockIdx.x], mr, total, lds4);
+    half_ranks(bits, toff[tile], mr, total, lds4);
     // the tile's stayers lie between the bounds of its first slot and the
     // next tile's (k_place_movers found them)
-    const int lo = tbound[blockIdx.x];
-    int hi = tbound[blockIdx.x + 1];
+    const int lo = tbound[tile];
+    int hi = tbound[tile + 1];
     hi = hi > lo ? (hi < m ? hi : m) : lo;
     const bool staged = hi - lo <= kPlaceStage;
     if (staged)
         for (int q = threadIdx.x; q < hi - lo; q += kRsThreads) {
-            stk[q] = skey[lo + q];
-            stv[q] = sr0[lo + q];
+            stk[q] = M.skey[lo + q];
+            stv[q] = M.sr0[lo + q];
         }
     __syncthreads();
-    const uint32_t* ck = staged ? stk : skey + lo;
-    const uint32_t* cv = staged ? stv : sr0 + lo;
+    const uint32_t* ck = staged ? stk : M.skey + lo;
+    const uint32_t* cv = staged ? stv : M.sr0 + lo;
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
         int mrh = mr[h];
@@ -646,6 +700,222 @@ __global__ __launch_bounds__(kRsThreads) void k_place_stayers(const uint32_t* __
             okeys[pos] = ko[j];
             perm[pos] = (uint32_t)i;
         }
+    }
+}
+__global__ __launch_bounds__(kRsThreads) void k_place_stayers(MoverSet M, const uint32_t* __restrict__ cur,
+                                                              const int* m_dev, const int* __restrict__ toff,
+                                                              const int* __restrict__ tbound,
+                                                              uint32_t* __restrict__ okeys, uint32_t* __restrict__ perm) {
+    __shared__ StayerLds sm;
+    int m = *m_dev;
+    m = m < M.n ? m : M.n;
+    place_stayers(M, cur, m, (int)blockIdx.x, toff, tbound, okeys, perm, sm);
+}
+// both placements in one launch, where the tiles' bounds came with the sort
+// of the movers (k_mover_sort): workgroups [0, tiles) the stayers' tiles, the
+// rest the movers
+__global__ __launch_bounds__(kRsThreads) void k_place(MoverSet M, const uint32_t* __restrict__ cur, const int* m_dev,
+                                                      const int* __restrict__ toff, const int* __restrict__ tbound,
+                                                      int tiles, OldTables tb, bool use_tables,
+                                                      uint32_t* __restrict__ okeys, uint32_t* __restrict__ perm) {
+    __shared__ StayerLds sm;
+    int m = *m_dev;
+    m = m < M.n ? m : M.n;
+    if ((int)blockIdx.x < tiles)
+        place_stayers(M, cur, m, (int)blockIdx.x, toff, tbound, okeys, perm, sm);
+    else
+        place_movers(M, m, (int)((blockIdx.x - tiles) * blockDim.x + threadIdx.x),
+                     (int)((gridDim.x - tiles) * blockDim.x), tb, use_tables, okeys, perm);
+}
+
+// ---- few movers: the whole sort in one workgroup ----
+// The general path takes 3 launches per digit, each a few microseconds of
+// dependent launch latency for a few thousand keys; one workgroup of 16 waves
+// sorts up to kMsCap movers in registers and LDS instead.  Wave w owns items
+// [64 w per, 64 (w + 1) per), per = items per thread, so (wave, round, lane)
+// order is index order; it ranks its items with private digit counters (peers
+// by eight ballots, no barriers), the counters are scanned digit-major over
+// the waves, and the items change places through LDS.  Larger counts, which
+// the caller's last published count did not foresee, go through the same
+// ranking tile by tile with the passes' output in global memory: slow, and
+// the next sort takes the general path.  Finally each tile of slots gets the
+// sorted movers that precede its first slot (tbound), by search.
+constexpr int kMsThreads = 1024;
+constexpr int kMsItems = 16;
+constexpr int kMsCap = kMsThreads * kMsItems;
+struct MsLds {
+    uint32_t key[kMsCap], val[kMsCap];
+    uint32_t wcnt[kMsThreads / 64][256];
+    uint32_t base[256], run[256];
+    int lds4[4];
+};
+// ranks of the wave's items among its items of the same digit; wcnt[w]
+// receives the wave's digit counts
+__device__ __forceinline__ void ms_rank(const uint32_t (&k)[kMsItems], uint32_t (&rank)[kMsItems], int per, int first,
+                                        int cnt, int shift, uint32_t* wc) {
+    const int lane = threadIdx.x & 63;
+    const uint64_t lt = (lane == 0) ? 0ull : ((~0ull) >> (64 - lane));
+#pragma unroll
+    for (int q = 0; q < 4; ++q) wc[q * 64 + lane] = 0u;
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int r = 0; r < kMsItems; ++r) {
+        if (r < per) {   // uniform
+            const bool valid = first + r * 64 + lane < cnt;
+            const uint32_t d = (k[r] >> shift) & 255u;
+            uint64_t peers = __ballot(valid);
+#pragma unroll
+            for (int b = 0; b < 8; ++b) {
+                const int bit = (d >> b) & 1;
+                const uint64_t bal = __ballot(bit);
+                peers &= bit ? bal : ~bal;
+            }
+            const uint32_t prev = valid ? wc[d] : 0u;
+            rank[r] = prev + (uint32_t)__popcll(peers & lt);
+            __builtin_amdgcn_wave_barrier();
+            if (valid && (peers & lt) == 0ull) wc[d] = prev + (uint32_t)__popcll(peers);
+            __builtin_amdgcn_wave_barrier();
+        }
+    }
+}
+// digit-major exclusive offsets of the waves' counters; base[d] = start[d]
+// plus nothing for a single tile, run[d] = the tile's count of digit d
+__device__ __forceinline__ void ms_offsets(MsLds& L, int& mine) {
+    mine = 0;
+    if (threadIdx.x < 256) {
+        uint32_t s = 0;
+#pragma unroll
+        for (int w = 0; w < kMsThreads / 64; ++w) {
+            const uint32_t c = L.wcnt[w][threadIdx.x];
+            L.wcnt[w][threadIdx.x] = s;
+            s += c;
+        }
+        mine = (int)s;
+    }
+}
+// exclusive scan of one value of each of the first 256 threads into L.base
+// (every thread of the workgroup takes part in the barriers)
+__device__ __forceinline__ void ms_scan256(MsLds& L, int v) {
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int inc = wave_incl_scan(v);
+    if (w < 4 && lane == 63) L.lds4[w] = inc;
+    __syncthreads();
+    if (w < 4) {
+        int off = inc - v;
+        for (int q = 0; q < w; ++q) off += L.lds4[q];
+        L.base[threadIdx.x] = (uint32_t)off;
+    }
+    __syncthreads();
+}
+__global__ __launch_bounds__(kMsThreads) void k_mover_sort(const uint32_t* __restrict__ list, const int* m_dev, int n,
+                                                           int passes, uint32_t* kb0, uint32_t* vb0, uint32_t* kb1,
+                                                           uint32_t* vb1, const uint32_t* __restrict__ old,
+                                                           const int* __restrict__ toff, int tiles,
+                                                           int* __restrict__ tbound) {
+    __shared__ MsLds L;
+    int m = *m_dev;
+    m = m < n ? m : n;
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+    uint32_t k[kMsItems], v[kMsItems], rank[kMsItems];
+    const bool small = m <= kMsCap;
+    if (small) {
+        const int per = (m + kMsThreads - 1) / kMsThreads, first = w * 64 * per;
+#pragma unroll
+        for (int r = 0; r < kMsItems; ++r) {
+            const int i = first + r * 64 + lane;
+            const bool in = r < per && i < m;
+            k[r] = in ? list[i] : 0u;
+            v[r] = (uint32_t)i;
+        }
+        for (int p = 0; p < passes; ++p) {
+            ms_rank(k, rank, per, first, m, 8 * p, L.wcnt[w]);
+            __syncthreads();
+            int mine;
+            ms_offsets(L, mine);
+            ms_scan256(L, mine);
+#pragma unroll
+            for (int r = 0; r < kMsItems; ++r)
+                if (r < per && first + r * 64 + lane < m) {
+                    const uint32_t d = (k[r] >> (8 * p)) & 255u;
+                    const uint32_t pos = L.base[d] + L.wcnt[w][d] + rank[r];
+                    L.key[pos] = k[r];
+                    L.val[pos] = v[r];
+                }
+            __syncthreads();
+            if (p + 1 < passes) {
+#pragma unroll
+                for (int r = 0; r < kMsItems; ++r) {
+                    const int i = first + r * 64 + lane;
+                    if (r < per && i < m) {
+                        k[r] = L.key[i];
+                        v[r] = L.val[i];
+                    }
+                }
+                __syncthreads();
+            }
+        }
+        for (int i = tid; i < m; i += kMsThreads) {
+            kb1[i] = L.key[i];
+            vb1[i] = L.val[i];
+        }
+    } else {
+        for (int p = 0; p < passes; ++p) {
+            const int o = (passes - 1 - p) % 2 == 0 ? 1 : 0;   // the last pass writes kb1, vb1
+            const uint32_t* ki = p == 0 ? list : (o ? kb0 : kb1);
+            const uint32_t* vi = o ? vb0 : vb1;
+            uint32_t* ko = o ? kb1 : kb0;
+            uint32_t* vo = o ? vb1 : vb0;
+            // digit starts of the whole list
+            if (tid < 256) L.run[tid] = 0u;
+            __syncthreads();
+            for (int i = tid; i < m; i += kMsThreads) atomicAdd(&L.run[(ki[i] >> (8 * p)) & 255u], 1u);
+            __syncthreads();
+            ms_scan256(L, tid < 256 ? (int)L.run[tid] : 0);
+            for (int t0 = 0; t0 < m; t0 += kMsCap) {
+                const int cnt = m - t0 < kMsCap ? m - t0 : kMsCap;
+                const int per = (cnt + kMsThreads - 1) / kMsThreads, first = w * 64 * per;
+#pragma unroll
+                for (int r = 0; r < kMsItems; ++r) {
+                    const int i = first + r * 64 + lane;
+                    const bool in = r < per && i < cnt;
+                    k[r] = in ? ki[t0 + i] : 0u;
+                    v[r] = in ? (p == 0 ? (uint32_t)(t0 + i) : vi[t0 + i]) : 0u;
+                }
+                ms_rank(k, rank, per, first, cnt, 8 * p, L.wcnt[w]);
+                __syncthreads();
+                int mine;
+                ms_offsets(L, mine);
+                __syncthreads();
+#pragma unroll
+                for (int r = 0; r < kMsItems; ++r)
+                    if (r < per && first + r * 64 + lane < cnt) {
+                        const uint32_t d = (k[r] >> (8 * p)) & 255u;
+                        const uint32_t pos = L.base[d] + L.wcnt[w][d] + rank[r];
+                        ko[pos] = k[r];
+                        vo[pos] = v[r];
+                    }
+                __syncthreads();
+                if (tid < 256) L.base[tid] += (uint32_t)mine;
+                __syncthreads();
+            }
+        }
+    }
+    __syncthreads();
+    const uint32_t* sk = small ? L.key : kb1;
+    const uint32_t* sv = small ? L.val : vb1;
+    for (int t = tid; t <= tiles; t += kMsThreads) {
+        int a = 0, b = m;
+        if (t < tiles) {
+            const uint32_t K = old[t * kRsTile], r0 = (uint32_t)toff[t];
+            while (a < b) {
+                const int mid = (a + b) >> 1;
+                if (below<kPair>(sk, sv, mid, K, r0)) a = mid + 1;
+                else b = mid;
+            }
+        } else {
+            a = m;
+        }
+        tbound[t] = a;
     }
 }
 
@@ -736,16 +1006,25 @@ static hipError_t radix_passes(mpmx_ctx* c, const uint32_t* k_in, const uint32_t
                                uint32_t* const (&vb)[2], RsSize z, int grid, int* hist_n) {
     const int passes = (c->key_bits + 7) / 8;
     const int64_t hist_cap = (int64_t)256 * c->sort_tiles;
+    // a device count is scanned in one launch while the last published mover
+    // count keeps the histogram below a quarter of a million entries
+    const bool direct = z.n_dev && c->hc->movers >= 0 && c->hc->movers < (1 << 20);
+    uint32_t* const offs = direct ? c->hist2 : c->hist;
     const uint32_t* ki = k_in;
     const uint32_t* vi = vals_in;
     for (int p = 0; p < passes; ++p) {
         const int o = (passes - 1 - p) % 2 == 0 ? 1 : 0;
         k_radix_hist<<<grid, kRsThreads, 0, c->stream>>>(ki, z, 8 * p, c->hist, hist_n);
-        hipError_t e = z.n_dev ? scan_exclusive(c, (const int*)c->hist, (int*)c->hist, hist_cap, hist_n, hist_cap, nullptr)
+        hipError_t e = hipSuccess;
+        if (direct)
+            k_scan_direct<<<(int)((hist_cap + kScanTile - 1) / kScanTile), 256, 0, c->stream>>>(
+                (const int*)c->hist, (int*)c->hist2, hist_n, hist_cap);
+        else
+            e = z.n_dev ? scan_exclusive(c, (const int*)c->hist, (int*)c->hist, hist_cap, hist_n, hist_cap, nullptr)
                                : scan_exclusive(c, (const int*)c->hist, (int*)c->hist, (int64_t)256 * z.tiles,
                                                 nullptr, (int64_t)256 * z.tiles, nullptr);
         if (e != hipSuccess) return e;
-        k_radix_scatter<<<grid, kRsThreads, 0, c->stream>>>(ki, vi, kb[o], vb[o], z, 8 * p, c->hist);
+        k_radix_scatter<<<grid, kRsThreads, 0, c->stream>>>(ki, vi, kb[o], vb[o], z, 8 * p, offs);
         ki = kb[o];
         vi = vb[o];
     }
@@ -778,34 +1057,47 @@ static hipError_t sort_movers(mpmx_ctx* c) {
     const int n = (int)c->n;
     const int tiles = c->sort_tiles;
     k_mover_count<<<tiles, kRsThreads, 0, c->stream>>>(c->keys, c->keys_next, n, c->mv_tcount);
-    hipError_t e = scan_exclusive(c, c->mv_tcount, c->mv_toff, tiles, nullptr, tiles, &c->dc->movers);
-    if (e != hipSuccess) return e;
     // the movers' radix passes end in mv_key[1] / mv_val[1]; the list goes
     // to the buffer that the first pass does not write
     const int passes = (c->key_bits + 7) / 8;
     uint32_t* const list = c->mv_key[(passes - 1) % 2 == 0 ? 0 : 1];
-    k_mover_list<<<tiles, kRsThreads, 0, c->stream>>>(c->keys, c->keys_next, n, c->mv_toff, list, c->mv_old,
-                                                      c->mv_slot, c->mv_cpre, c->mv_cmask);
+    k_mover_list<<<tiles, kRsThreads, 0, c->stream>>>(c->keys, c->keys_next, n, c->mv_tcount, c->mv_toff,
+                                                      &c->dc->movers, list, c->mv_old, c->mv_slot, c->mv_cpre,
+                                                      c->mv_cmask);
+    const OldTables tb{c->pmask, c->wcount, c->page2particle, c->cell_start, &c->dc->num_page, c->cap_p};
+    const MoverSet M{c->keys, n, c->mv_key[1], c->mv_val[1], c->mv_old, c->mv_slot, c->mv_cpre, c->mv_cmask};
+    if (c->few_movers) {
+        k_mover_sort<<<1, kMsThreads, 0, c->stream>>>(list, &c->dc->movers, n, passes, c->mv_key[0], c->mv_val[0],
+                                                      c->mv_key[1], c->mv_val[1], c->keys, c->mv_toff, tiles,
+                                                      c->mv_tbound);
+        const int mwg = std::max(1, std::min(tiles, kMsCap / kRsThreads));
+        k_place<<<tiles + mwg, kRsThreads, 0, c->stream>>>(M, c->keys_next, &c->dc->movers, c->mv_toff, c->mv_tbound,
+                                                           tiles, tb, c->tables_match_keys, c->keys_alt, c->vals_alt);
+        c->gather_perm = c->vals_alt;
+        return hipGetLastError();
+    }
     const int grid = std::min(tiles, 4 * c->num_cu);
     uint32_t* const kb[2] = {c->mv_key[0], c->mv_key[1]};
     uint32_t* const vb[2] = {c->mv_val[0], c->mv_val[1]};
-    e = radix_passes(c, list, nullptr, kb, vb, RsSize{n, &c->dc->movers, tiles}, grid, &c->dc->mv_hist_n);
+    hipError_t e = radix_passes(c, list, nullptr, kb, vb, RsSize{n, &c->dc->movers, tiles}, grid, &c->dc->mv_hist_n);
     if (e != hipSuccess) return e;
     // one thread per mover up to n / 8 movers (the movers' searches are
     // chains of dependent loads: latency, hidden by many waves)
-    const OldTables tb{c->pmask, c->wcount, c->page2particle, c->cell_start, &c->dc->num_page, c->cap_p};
-    k_place_movers<<<tiles, kRsThreads, 0, c->stream>>>(c->keys, n, c->mv_key[1], c->mv_val[1], c->mv_old,
-                                                       c->mv_slot, &c->dc->movers, c->mv_cpre, c->mv_cmask,
-                                                       c->mv_toff, tiles, c->mv_tbound, tb, c->tables_match_keys,
-                                                       c->keys_alt, c->vals_alt);
-    k_place_stayers<<<tiles, kRsThreads, 0, c->stream>>>(c->keys, c->keys_next, n, c->mv_toff, c->mv_tbound,
-                                                         c->mv_key[1], c->mv_val[1], &c->dc->movers, c->keys_alt,
-                                                         c->vals_alt);
+    k_place_movers<<<tiles, kRsThreads, 0, c->stream>>>(M, &c->dc->movers, c->mv_toff, tiles, c->mv_tbound, tb,
+                                                       c->tables_match_keys, c->keys_alt, c->vals_alt);
+    k_place_stayers<<<tiles, kRsThreads, 0, c->stream>>>(M, c->keys_next, &c->dc->movers, c->mv_toff, c->mv_tbound,
+                                                         c->keys_alt, c->vals_alt);
     c->gather_perm = c->vals_alt;
     return hipGetLastError();
 }
 
+// Which path the next sort takes.  few_movers: the movers' own sort in one
+// workgroup, where the last published count (or n itself) leaves room for
+// growth by a third up to its capacity; a count not published yet (-1, the
+// first sorts after an upload) is taken as large unless n is small.
 void choose_sort_path(mpmx_ctx* c) {
+    const int64_t bound = c->hc->movers < 0 ? c->n : std::min<int64_t>(c->n, (int64_t)c->hc->movers * 4 / 3);
+    c->few_movers = bound <= kMsCap;
     if (c->cfg.sort_variant != 0) {
         c->sort_by_movers = c->cfg.sort_variant == 2;
         return;

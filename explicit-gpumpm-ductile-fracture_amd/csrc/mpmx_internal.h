@@ -212,6 +212,7 @@ struct mpmx_ctx {
     uint32_t* vals = nullptr;
     uint32_t* vals_alt = nullptr;
     uint32_t* hist = nullptr;
+    uint32_t* hist2 = nullptr;   // scanned histogram of the movers' radix passes
     int sort_tiles = 0;
     int key_bits = 0;
     bool sorted = false;     // particles gathered to the order of `keys`
@@ -226,6 +227,7 @@ struct mpmx_ctx {
     uint32_t* mv_slot = nullptr;
     bool sort_by_movers = true;   // the path the next sort takes (mpmx_config.sort_variant 0: from
                                   // the last published mover count)
+    bool few_movers = false;      // the movers are few enough for the one-workgroup sort
     bool old_keys_sorted = false; // keys holds a sort's output (the mover path's precondition)
     bool tables_match_keys = false;   // the page tables were built from keys (the mover path uses them)
     int* mv_tbound = nullptr;     // [sort_tiles + 1] sorted movers before each tile's first slot
@@ -281,6 +283,7 @@ struct mpmx_ctx {
         int iters = 0;
         int64_t blocks = 0;
         bool by_movers = false;   // the sort path captured
+        bool few_movers = false;
     } graphs[2];
     int cg_recent[8] = {0, 0, 0, 0, 0, 0, 0, 0};   // PCG iterations of the last substeps
     int* bcount = nullptr;           // [mask_words] per-word block counts, then their scan
