@@ -67,13 +67,10 @@ __device__ __forceinline__ uint32_t scene_page_key(const BlockTables& t, int px,
 // The same 27 source pages, grouped by class: bit 2 / 1 / 0 of the class set
 // when the page lies below the block along x / y / z.  Only the particles in
 // cells with index 2 or 3 along each such axis reach the block, and their
-// base node lies one or two nodes below it, so a class knows at compile time
-// which node offsets can fall outside the block.  Each source page is listed
+// base node lies one or two nodes below it.  Each source page is listed
 // as runs of its passing cells (cell = i<<4 | j<<2 | k, i, j, k in 0..3), with
 // the particle ranges from the page's cell starts, so every listed particle
-// reaches the block; a workgroup's threads are split among the classes, an
-// equal number of entries each, so that most waves hold particles of one
-// class and take the same branches.
+// reaches the block.
 // class:             0  1(z) 2(y) 3(yz) 4(x) 5(xz) 6(xy) 7(xyz)
 // pages:             8  4    4    2     4    2     2     1
 // runs per page:     1  16   4    8     1    8     2     4
@@ -92,8 +89,6 @@ struct BlockClasses {
     int pre[kMaxRuns + 1];   // particles listed before run r (all classes, in order)
     int page[27];            // particle page id of source slot s, or -1 (slot order)
     int out_page[8];
-    int thr0[9];             // threads [thr0[c], thr0[c + 1]) work on class c
-    int len[8];              // entries per thread of class c
 };
 
 // what the block G2P of a 2x2x2 block needs besides the grid: the grid pages
@@ -156,8 +151,8 @@ __device__ __forceinline__ void class_run(int cls, int r, int& c0, int& len) {
 // lane, all at once: the 27 source slots, the G2P region's 27 grid pages and
 // the block's own 8 grid pages), the 132 runs
 // of passing cells (three per lane) with their particle ranges read from the
-// cell starts, the exclusive prefix over the runs, and the threads of each
-// class of the 256-thread gathers.  Returns the block's entries.
+// cell starts, and the exclusive prefix over the runs.  Returns the block's
+// entries.
 __device__ __forceinline__ int block_lists_wave(const BlockTables& t, uint32_t bkey, int n, int np_raw, int np,
                                                  int nt, BlockClasses* __restrict__ dst, BlockG2P* __restrict__ g2p) {
     const int lane = threadIdx.x & 63;
@@ -255,52 +250,7 @@ __device__ __forceinline__ int block_lists_wave(const BlockTables& t, uint32_t b
     }
     const int all = carry;
     if (lane == 0) dst->pre[kMaxRuns] = all;
-    // every thread takes L = ceil(all / 248) entries of a single class (the
-    // last thread of a class fewer) and a class gets ceil(n_c / L) threads
-    // (at most 255 in all): waves stay within one class except where two
-    // classes meet, their lanes run L entries each, and the threads left
-    // over form idle trailing waves rather than short runs in busy ones
-    const int c = lane < 8 ? lane : 0;
-    int pre_c[2];
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-        const int b = class_first_run(c + h);
-        const int v0 = __shfl(excl[0], b & 63, 64), v1 = __shfl(excl[1], b & 63, 64),
-                  v2 = __shfl(excl[2], b & 63, 64);
-        pre_c[h] = b >= kMaxRuns ? all : ((b >> 6) == 0 ? v0 : ((b >> 6) == 1 ? v1 : v2));
-    }
-    const int n_c = pre_c[1] - pre_c[0];
-    const int L = all > 0 ? (all + 247) / 248 : 1;
-    int thr = 0;
-    if (lane < 8 && n_c > 0) thr = (n_c + L - 1) / L;
-    int tin = thr;
-#pragma unroll
-    for (int o = 1; o < 8; o <<= 1) {
-        const int up = __shfl_up(tin, o, 64);
-        if (lane >= o) tin += up;
-    }
-    if (lane < 8) {
-        dst->thr0[lane] = tin - thr;
-        dst->len[lane] = thr > 0 ? L : 0;
-    }
-    if (lane == 7) dst->thr0[8] = tin;
     return all;
-}
-
-// particles listed for class cls, and entry j of them
-__device__ __forceinline__ int class_count(const BlockClasses& S, int cls) {
-    return S.pre[cls == 7 ? kMaxRuns : class_first_run(cls + 1)] - S.pre[class_first_run(cls)];
-}
-__device__ __forceinline__ int class_entry(const BlockClasses& S, int cls, int j) {
-    const int lo0 = class_first_run(cls);
-    const int e = S.pre[lo0] + j;
-    int lo = lo0, hi = lo0 + (kClassFirstSlot[cls + 1] - kClassFirstSlot[cls]) * kClassRuns[cls] - 1;
-    while (lo < hi) {
-        const int mid = (lo + hi + 1) >> 1;
-        if (S.pre[mid] <= e) lo = mid;
-        else hi = mid - 1;
-    }
-    return S.start[lo] + (e - S.pre[lo]);
 }
 
 // The order in which the block kernels take the blocks: by work, longest
@@ -379,23 +329,6 @@ __device__ __forceinline__ void order_blocks(const uint8_t* __restrict__ wclass,
     }
 }
 
-// the class of the calling thread and its entries [jb, je) of that class;
-// false for threads without entries
-__device__ __forceinline__ bool thread_class(const BlockClasses& S, int& cls, int& jb, int& je) {
-    const int t = (int)threadIdx.x;
-    cls = -1;
-#pragma unroll
-    for (int c = 0; c < 8; ++c)
-        if (t >= S.thr0[c] && t < S.thr0[c + 1]) cls = c;
-    if (cls < 0) return false;
-    const int len = S.len[cls];
-    jb = (t - S.thr0[cls]) * len;
-    je = jb + len;
-    const int n = class_count(S, cls);
-    je = je < n ? je : n;
-    return jb < je;
-}
-
 // ---- fixed-point accumulation -----------------------------------------------
 // LDS float atomics cost ~190 CU cycles per wave instruction on gfx950 and
 // 64-bit integer atomics ~7, so the block gathers add in fixed point: a
@@ -440,6 +373,146 @@ constexpr int kAccZ = 9;
 constexpr int kAccX = 76;
 constexpr int kAccStride = 8 * kAccX;   // words per channel
 __host__ __device__ constexpr int acc_node(int lx, int ly, int lz) { return lx * kAccX + ly * kAccZ + lz; }
+
+// ---- tiles of the gathers ---------------------------------------------------------
+// A gather sums into a tile of E^3 nodes: a 2x2x2-page block (E = 8) or one of
+// its pages (E = 4).  Particles of the cells -2 .. E-1 along each axis reach it:
+// along an axis, those of cell -2 with one node (their third), of -1 with two,
+// of E-2 with two (their first two), of E-1 with one, the others with all three.
+// The tile's cells are taken in the order of these counts (x, then y, then
+// z, most nodes first, cells in order inside), so that the lanes of a wave,
+// which hold neighbours of that order, run the same node loops.  The first
+// nodes of the cell, those below the tile, are dropped by shifting the
+// weights, which makes the loops of cells at either side alike.
+template <int E> struct TileAcc {
+    // node strides: z padded by one and x by a few words, so that the 64-bit
+    // atomics of a wave, whose lanes hold neighbouring cells, spread over the
+    // LDS banks
+    static constexpr int kZ = E + 1;
+    static constexpr int kX = E == 8 ? kAccX : 21;
+    static constexpr int kStride = E * kX;   // words per channel
+};
+template <int E> struct TileOrder {
+    static constexpr int kCells = (E + 2) * (E + 2) * (E + 2);
+    uint16_t cell[kCells];   // (x + 2) << 8 | (y + 2) << 4 | (z + 2)
+};
+template <int E> constexpr TileOrder<E> tile_order() {
+    TileOrder<E> t{};
+    // cells along one axis by their nodes in the tile: 3, 2, 1
+    int line[E + 2] = {}, m = 0, first[4] = {};
+    for (int want = 3; want >= 1; --want) {
+        first[3 - want] = m;
+        for (int l = -2; l < E; ++l) {
+            const int cnt = (l + 3 < E ? l + 3 : E) - (l < 0 ? 0 : l);
+            if (cnt == want) line[m++] = l + 2;
+        }
+    }
+    first[3] = m;
+    int q = 0;
+    for (int gx = 0; gx < 3; ++gx)
+        for (int gy = 0; gy < 3; ++gy)
+            for (int gz = 0; gz < 3; ++gz)
+                for (int x = first[gx]; x < first[gx + 1]; ++x)
+                    for (int y = first[gy]; y < first[gy + 1]; ++y)
+                        for (int z = first[gz]; z < first[gz + 1]; ++z)
+                            t.cell[q++] = (uint16_t)((line[x] << 8) | (line[y] << 4) | line[z]);
+    return t;
+}
+template <int E> __device__ __constant__ const TileOrder<E> kTileOrder = tile_order<E>();
+
+constexpr int kTileThreads = 256;   // per workgroup
+
+// the tile's cells that hold particles, in that order, and the pairs of
+// particles they make (the last pair of an odd cell is a single)
+template <int E> struct TileCells {
+    static constexpr int kCells = TileOrder<E>::kCells;
+    static constexpr int kPer = (kCells + kTileThreads - 1) / kTileThreads;
+    int start[kCells];       // first particle
+    int pairs[kCells + 1];   // pairs before the cell
+    uint16_t place[kCells];  // TileOrder; bit 12: an odd number of particles
+    int page[27];            // particle pages 2b - 1 .. 2b + 1 of the block, by place
+    int wsum[2][kTileThreads / 64];
+    int cells;
+};
+
+// Builds S for the tile at o3 (nodes) of the block with lists L; called and
+// left by the whole workgroup (a barrier at its end)
+template <int E>
+__device__ __forceinline__ void tile_cells(const BlockClasses* __restrict__ L, const int* __restrict__ cell_start,
+                                           int n, const int (&o3)[3], TileCells<E>& S) {
+    constexpr int kPer = TileCells<E>::kPer, kCells = TileCells<E>::kCells;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    if (tid < 27) {
+        int cls, d[3];
+        source_slot(tid, cls, d);
+        S.page[(d[0] + 1) * 9 + (d[1] + 1) * 3 + d[2] + 1] = L->page[tid];
+    }
+    __syncthreads();
+    int st[kPer], cnt[kPer], pairs = 0, cells = 0;
+#pragma unroll
+    for (int k = 0; k < kPer; ++k) {
+        const int r = tid * kPer + k;
+        const int w = r < kCells ? (int)kTileOrder<E>.cell[r] : 0;
+        const int x = o3[0] + (w >> 8) + 2, y = o3[1] + ((w >> 4) & 15) + 2, z = o3[2] + (w & 15) + 2;   // cell + 4
+        const int pg = r < kCells ? S.page[(x >> 2) * 9 + (y >> 2) * 3 + (z >> 2)] : -1;
+        int a = 0, b = 0;
+        if (pg >= 0) {
+            const int* cs = cell_start + (int64_t)pg * 65 + (((x & 3) << 4) | ((y & 3) << 2) | (z & 3));
+            a = cs[0];
+            b = cs[1];
+            a = a < 0 ? 0 : (a > n ? n : a);
+            b = b < a ? a : (b > n ? n : b);
+        }
+        st[k] = a;
+        cnt[k] = b - a;
+        pairs += (cnt[k] + 1) >> 1;
+        cells += cnt[k] > 0 ? 1 : 0;
+    }
+    const int ip = wave_incl_scan_i(pairs), ic = wave_incl_scan_i(cells);
+    if (lane == 63) {
+        S.wsum[0][wave] = ip;
+        S.wsum[1][wave] = ic;
+    }
+    __syncthreads();
+    int p = ip - pairs, c = ic - cells, tp = 0, tc = 0;
+#pragma unroll
+    for (int q = 0; q < kTileThreads / 64; ++q) {
+        p += q < wave ? S.wsum[0][q] : 0;
+        c += q < wave ? S.wsum[1][q] : 0;
+        tp += S.wsum[0][q];
+        tc += S.wsum[1][q];
+    }
+#pragma unroll
+    for (int k = 0; k < kPer; ++k)
+        if (cnt[k] > 0) {
+            S.start[c] = st[k];
+            S.pairs[c] = p;
+            S.place[c] = (uint16_t)(kTileOrder<E>.cell[tid * kPer + k] | ((cnt[k] & 1) << 12));
+            p += (cnt[k] + 1) >> 1;
+            ++c;
+        }
+    if (tid == 0) {
+        S.pairs[tc] = tp;
+        S.cells = tc;
+    }
+    __syncthreads();
+}
+// cell of pair e (0 <= e < S.pairs[S.cells]): the last that starts at or before e
+template <int E>
+__device__ __forceinline__ int tile_find(const TileCells<E>& S, int e) {
+    int lo = 0, hi = S.cells - 1;
+    while (lo < hi) {
+        const int mid = (lo + hi + 1) >> 1;
+        if (S.pairs[mid] <= e) lo = mid;
+        else hi = mid - 1;
+    }
+    return lo;
+}
+// the nodes of one axis moved down by s places (0 .. 2)
+__device__ __forceinline__ void drop_nodes(float (&w)[3], int s) {
+    w[0] = s == 0 ? w[0] : (s == 1 ? w[1] : w[2]);
+    w[1] = s == 0 ? w[1] : w[2];
+}
 
 __device__ __forceinline__ float ld_x(const PState& s, int i, int a) { return s.x[3 * i + a]; }
 __device__ __forceinline__ float ld_x(const MState& s, int i, int a) { return s.x[3 * i + a]; }

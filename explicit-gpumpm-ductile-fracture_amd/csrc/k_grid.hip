@@ -8,19 +8,19 @@
 //   grid  undateGrid_kernal + collideWithGround / PullGrid (TimeIntegrator.cu:
 //         63-261) and the PCG initialisation of ExplicitTimeIntegrator.cu:914-935.
 //
-// Gather form: a workgroup owns one 2x2x2 block of grid pages (8^3 nodes, the
-// pages 8b .. 8b+7 in Morton order) at a time.  Particles of page P reach the
+// Gather form: a workgroup owns one tile of grid nodes at a time, a 2x2x2
+// block of grid pages (8^3 nodes, the pages 8b .. 8b+7 in Morton order) or,
+// where the blocks are few, one page (4^3).  Particles of page P reach the
 // nodes of P and its +1 neighbours, so block b receives from the 27 particle
-// pages 2b-1 .. 2b+1 (per axis); of a page below the block along an axis only
-// the particles whose cell has index & 3 >= 2 on that axis reach it.  The
-// workgroup loads the block's source lists (runs of passing cells, built with
-// the page tables by k_block_lists), takes the fixed-point scale of each
-// channel from the per-page bounds of its 27 source pages (written with the
-// payload), and adds every listed particle's contributions to the block's
-// nodes in LDS with 64-bit integer atomics.  It then updates its nodes in
-// place and writes them once: no global atomics, no zero fill of the grid,
-// and sums that do not depend on the order of the additions.  Each particle
-// is read by the one to eight blocks it reaches (about twice on average).
+// pages 2b-1 .. 2b+1 (per axis), from their cells -2 .. 7 of the block.  The
+// workgroup lists those cells in the order of the nodes they reach (TileCells),
+// takes the fixed-point scale of each channel from the per-page bounds of the
+// 27 source pages (written with the payload), and adds the particles'
+// contributions to the tile's nodes in LDS with 64-bit integer atomics, two
+// particles of a cell at a time.  It then updates its nodes in place and
+// writes them once: no global atomics, no zero fill of the grid, and sums that
+// do not depend on the order of the additions.  Each particle is read by the
+// one to eight blocks it reaches (about twice on average).
 #include "payload.h"
 
 namespace mpmx {
@@ -37,9 +37,11 @@ __device__ __forceinline__ float node_update(const DevParams& dp, int gi, int gj
     if (!(W > 0.f)) return 0.f;
     const float inv = 1.0f / ch[0];
     const float c = ch[4] / W;
-    float v0 = ch[1] * inv + dp.gravity[0] * dt;
-    float v1 = ch[2] * inv + dp.gravity[1] * dt;
-    float v2 = ch[3] * inv + dp.gravity[2] * dt;
+    // the fused multiply-adds spelled out here and below, so that every
+    // kernel that updates nodes rounds them alike
+    float v0 = fmaf(ch[1], inv, dp.gravity[0] * dt);
+    float v1 = fmaf(ch[2], inv, dp.gravity[1] * dt);
+    float v2 = fmaf(ch[3], inv, dp.gravity[2] * dt);
     if (dp.grip_lo >= 0) {
         if (gi <= dp.grip_lo) { v0 = -dp.grip_v; v1 = 0.f; v2 = 0.f; }
         if (gi >= dp.grip_hi) { v0 = dp.grip_v; v1 = 0.f; v2 = 0.f; }
@@ -57,7 +59,7 @@ __device__ __forceinline__ float node_update(const DevParams& dp, int gi, int gj
     ch[4] = c;
     const float VW = ch[6], VFW = ch[7];
     const float rhs = VW * (c / dt + dp.M);
-    const float D = dp.M * VFW + VW / dt;
+    const float D = fmaf(dp.M, VFW, VW / dt);
     ch[6] = rhs;
     ch[7] = D;
     r = rhs;
@@ -123,57 +125,111 @@ __device__ __forceinline__ void scale_terms(P2GTerms& T, const float (&sc)[kP2GC
     T.VF *= sc[7];
 }
 
-// add the particle's contributions (terms scaled by scale_terms, sc5 the
-// scale of the weight channel) to the block's 8^3 nodes in fixed point.
-// Nodes outside the block are skipped; a wave whose lanes all hold particles
-// of one source class (see BlockClasses) skips them together.
+// Two particles of one cell at once: their contributions to the cell's nodes
+// inside the tile.  The nodes are the first n[a] of each axis
+// after the weights have been moved down by s[a] (the nodes below the tile), so
+// lanes with the same counts take the same branches.  A term (scaled by
+// scale_terms, sc5 the scale of the weight channel) is truncated to a 32-bit
+// integer by itself, as if it were added alone; its weight is at most 0.75^3
+// (0.75^2 for APIC's gradients), so two of at most 2^30 times that add up in 32
+// bits, and one 64-bit LDS atomic takes both.
 // The affine term ar + Qd (ii, jj, kk) is accumulated axis by axis with one
-// fused multiply-add per nonzero offset, shared by the nodes of a row; a zero
-// offset adds nothing (for finite terms it could only change the sign of a
-// zero, which converts to the same integer).
-template <int TRANSFER>
-__device__ __forceinline__ void p2g_fix(const P2GTerms& T, float sc5, unsigned long long* acc) {
+// fused multiply-add per offset, shared by the nodes of a row; a zero offset
+// adds nothing (for finite terms it could only change the sign of a zero,
+// which converts to the same integer).
+template <int TRANSFER, int SX, int SY, int SC>
+__device__ __forceinline__ void p2g_fix(const P2GTerms (&T)[2], const int (&s)[3], const int (&n)[3], float sc5,
+                                        unsigned long long* acc) {
+    float of[3];
+#pragma unroll
+    for (int a = 0; a < 3; ++a) of[a] = (float)s[a];
 #pragma unroll
     for (int ii = 0; ii < 3; ++ii) {
-        const int la = T.l0[0] + ii;
-        if (la < 0 || la >= 8) continue;
-        float ax[3];
+        if (ii >= n[0]) break;
+        const float fi = of[0] + (float)ii;
+        float ax[2][3];
 #pragma unroll
-        for (int r = 0; r < 3; ++r) ax[r] = ii == 0 ? T.ar[r] : fmaf(T.Qd[r], (float)ii, T.ar[r]);
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+            for (int r = 0; r < 3; ++r) ax[h][r] = fmaf(T[h].Qd[r], fi, T[h].ar[r]);
 #pragma unroll
         for (int jj = 0; jj < 3; ++jj) {
-            const int lb = T.l0[1] + jj;
-            if (lb < 0 || lb >= 8) continue;
-            const float wxy = T.w[0][ii] * T.w[1][jj];
-            float axy[3];
+            if (jj >= n[1]) break;
+            const float fj = of[1] + (float)jj;
+            float wxy[2], axy[2][3];
 #pragma unroll
-            for (int r = 0; r < 3; ++r) axy[r] = jj == 0 ? ax[r] : fmaf(T.Qd[r + 3], (float)jj, ax[r]);
+            for (int h = 0; h < 2; ++h) {
+                wxy[h] = T[h].w[0][ii] * T[h].w[1][jj];
+#pragma unroll
+                for (int r = 0; r < 3; ++r) axy[h][r] = fmaf(T[h].Qd[r + 3], fj, ax[h][r]);
+            }
 #pragma unroll
             for (int kk = 0; kk < 3; ++kk) {
-                const int lc = T.l0[2] + kk;
-                if (lc < 0 || lc >= 8) continue;
-                const float wt = wxy * T.w[2][kk];
-                float pr[3];
+                if (kk >= n[2]) break;
+                const float fk = of[2] + (float)kk;
+                int add[kP2GCh];
 #pragma unroll
-                for (int r = 0; r < 3; ++r) pr[r] = wt * (kk == 0 ? axy[r] : fmaf(T.Qd[r + 6], (float)kk, axy[r]));
-                if (TRANSFER == 1) {
-                    const float g0 = T.gw[0][ii] * T.w[1][jj] * T.w[2][kk];
-                    const float g1 = T.w[0][ii] * T.gw[1][jj] * T.w[2][kk];
-                    const float g2 = T.w[0][ii] * T.w[1][jj] * T.gw[2][kk];
+                for (int h = 0; h < 2; ++h) {
+                    const P2GTerms& t = T[h];
+                    const float wt = wxy[h] * t.w[2][kk];
+                    float pr[3];
 #pragma unroll
-                    for (int r = 0; r < 3; ++r) pr[r] -= T.sg[r] * g0 + T.sg[r + 3] * g1 + T.sg[r + 6] * g2;
+                    for (int r = 0; r < 3; ++r) pr[r] = wt * fmaf(t.Qd[r + 6], fk, axy[h][r]);
+                    if (TRANSFER == 1) {
+                        const float g0 = t.gw[0][ii] * t.w[1][jj] * t.w[2][kk];
+                        const float g1 = t.w[0][ii] * t.gw[1][jj] * t.w[2][kk];
+                        const float g2 = t.w[0][ii] * t.w[1][jj] * t.gw[2][kk];
+#pragma unroll
+                        for (int r = 0; r < 3; ++r) pr[r] -= t.sg[r] * g0 + t.sg[r + 3] * g1 + t.sg[r + 6] * g2;
+                    }
+                    const float v[kP2GCh] = {wt * t.m, pr[0], pr[1], pr[2], wt * t.cphase, wt * sc5, wt * t.V, wt * t.VF};
+#pragma unroll
+                    for (int k = 0; k < kP2GCh; ++k) add[k] = h == 0 ? (int)v[k] : add[k] + (int)v[k];
                 }
-                unsigned long long* a = acc + acc_node(la, lb, lc);
-                const float add[kP2GCh] = {wt * T.m, pr[0], pr[1], pr[2], wt * T.cphase, wt * sc5, wt * T.V, wt * T.VF};
+                unsigned long long* a = acc + (ii * SX + jj * SY + kk);
                 // the weights are >= 0, so channel 5 needs no sign extension
 #pragma unroll
                 for (int k = 0; k < kP2GCh; ++k)
-                    atomicAdd(a + k * kAccStride, k == 5 ? to_fix_scaled_nonneg(add[k]) : to_fix_scaled(add[k]));
+                    atomicAdd(a + k * SC, k == 5 ? (unsigned long long)(unsigned)add[k]
+                                                 : (unsigned long long)(long long)add[k]);
             }
         }
     }
 }
 
+// particles i and (two set) i + 1, of the cell at `place` of the tile, into the tile's sums
+template <int E, int TRANSFER>
+__device__ __forceinline__ void p2g_pair(const float* __restrict__ pay, int i, bool two, int place,
+                                         const float (&sc)[kP2GCh], unsigned long long* acc) {
+    using A = TileAcc<E>;
+    P2GTerms T[2];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        payload_terms<TRANSFER>(pay, two ? i + h : i, T[h]);
+        scale_terms<TRANSFER>(T[h], sc);
+    }
+    // a missing second particle: zero weights
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        T[1].w[2][k] = two ? T[1].w[2][k] : 0.f;
+        if (TRANSFER == 1) T[1].gw[2][k] = two ? T[1].gw[2][k] : 0.f;
+    }
+    int s[3], cnt[3], node = 0;
+#pragma unroll
+    for (int ax = 0; ax < 3; ++ax) {
+        const int l = ((place >> (8 - 4 * ax)) & 15) - 2;   // cell in the tile, -2 .. E-1
+        const int f = l < 0 ? 0 : l;
+        s[ax] = f - l;
+        cnt[ax] = (l + 3 < E ? l + 3 : E) - f;
+        node += f * (ax == 0 ? A::kX : (ax == 1 ? A::kZ : 1));
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            drop_nodes(T[h].w[ax], s[ax]);
+            if (TRANSFER == 1) drop_nodes(T[h].gw[ax], s[ax]);
+        }
+    }
+    p2g_fix<TRANSFER, A::kX, A::kZ, A::kStride>(T, s, cnt, sc[5], acc + node);
+}
 
 // payload of every particle and its page's channel bounds (page_bounds)
 template <int TRANSFER, typename ST>
@@ -197,83 +253,94 @@ __global__ __launch_bounds__(256) void k_p2g_prep(DevParams dp, ST s, WaveMap wm
     page_bounds(valid, pk, b, t, pbound, dc);
 }
 
-// the calling thread's run [jb, je) of the entries of one class of the
-// block's sources: the particles of one cell (adjacent after the sort) go
-// through one lane in turn instead of hitting the same nodes in one
-// instruction
-template <int TRANSFER>
-__device__ __forceinline__ void p2g_class(const BlockClasses& S, const BlockTables& t, const float* __restrict__ pay,
-                                          const int (&org)[3], const float (&sc)[kP2GCh], unsigned long long* acc,
-                                          int cls, int jb, int je) {
-    for (int j = jb; j < je; ++j) {
-        const int i = class_entry(S, cls, j);
-        P2GTerms T;
-        payload_load<TRANSFER>(pay, i, t.keys[i], org, T);
-        scale_terms<TRANSFER>(T, sc);
-        p2g_fix<TRANSFER>(T, sc[5], acc);
-    }
-}
-
-template <int TRANSFER, typename ST>
-__global__ __launch_bounds__(256, 4) void k_p2g_block(DevParams dp, const float* __restrict__ pay,
-                                                   const unsigned* __restrict__ pbound, BlockTables t,
-                                                   const BlockClasses* __restrict__ lists, float* __restrict__ grid,
-                                                   float* __restrict__ grid_raw, CGVec cg, float dt, int n,
-                                                   const DevCounts* __restrict__ dc) {
-    __shared__ unsigned long long acc[kP2GCh * kAccStride];
-    __shared__ BlockClasses S;
+// The LDS atomics bound it (6.3 cycles of the CU per wave instruction, more
+// with bank conflicts, eight per node), then the latency of a sparse tile's
+// dependent loads.  Against one particle per lane with one atomic per term
+// and lanes idle where their nodes fall outside the block: 8M impact (8
+// particles a cell) 743 -> 396 us, 256-scene batch (4, random) 1,340 -> 1,020
+// us, 64,000 cube 175 -> 36 us (page tiles; 94 with block tiles), 1M bar
+// (0.6) 142 -> 149 us.  Measured and not taken: 512 threads (443, 1,221 us),
+// pairs and the odd cells' last particles in two passes (405, 1,105 us), tiles
+// taken in turn by resident workgroups with the next tile's cells loaded ahead
+// (467, 1,170 us).
+template <int E, int TRANSFER>
+__global__ __launch_bounds__(kTileThreads, TRANSFER == 0 ? 4 : 3) void k_p2g_tile(
+    DevParams dp, const float* __restrict__ pay, const unsigned* __restrict__ pbound, BlockTables t,
+    const BlockClasses* __restrict__ lists, float* __restrict__ grid, float* __restrict__ grid_raw, CGVec cg, float dt,
+    int n, const DevCounts* __restrict__ dc) {
+    using A = TileAcc<E>;
+    __shared__ unsigned long long acc[kP2GCh * A::kStride];
+    __shared__ TileCells<E> S;
     __shared__ int sexp[kP2GCh];
     dt = substep_dt(dt, dc);
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     int nb = dc->num_blocks;
     nb = nb < t.cap_blocks ? nb : (int)t.cap_blocks;
-    FOR_LOGICAL_ITEMS(item, nb) {
-        const int blk = t.order ? t.order[item] : item;
-        const uint32_t bkey = t.block_key[blk];
-        int bc[3];
-        unmorton(bkey, bc[0], bc[1], bc[2]);
-        const DevParams sp = dp.scenes[__builtin_amdgcn_readfirstlane(scene_of_page(dp, bkey << 3))];
-        // the block's source lists, built with the page tables
+    const int items = E == 8 ? nb : 8 * nb;
+    FOR_LOGICAL_ITEMS(item, items) {
+        const int at = E == 8 ? item : item >> 3, child = E == 8 ? 0 : item & 7;
+        const int blk = t.order ? t.order[at] : at;
+        // the block's source pages, listed with the page tables
         const BlockClasses* L = lists + blk;
-        classes_load(L, S);
-        for (int q = tid; q < kP2GCh * kAccStride; q += 256) acc[q] = 0ull;
-        const int org[3] = {8 * bc[0], 8 * bc[1], 8 * bc[2]};
-        // scales: the largest contribution per channel of the 27 source pages
+        if (E == 4 && L->out_page[child] < 0) continue;   // uniform over the workgroup
+        const int o3[3] = {4 * ((child >> 2) & 1), 4 * ((child >> 1) & 1), 4 * (child & 1)};
+        for (int q = tid; q < kP2GCh * A::kStride; q += kTileThreads) acc[q] = 0ull;
+        // scales: the largest contribution per channel of the block's 27 source pages
         if (wave == 1) {
             const int pg = lane < 27 ? L->page[lane] : -1;
-            float bmax[kP2GCh];
+            float4 lo = make_float4(0.f, 0.f, 0.f, 0.f), hi = lo;
+            if (pg >= 0) {   // the bits of non-negative floats
+                const float4* b = reinterpret_cast<const float4*>(pbound + (int64_t)pg * kP2GCh);
+                lo = b[0];
+                hi = b[1];
+            }
+            const float bnd[kP2GCh] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+            float v = 0.f;
 #pragma unroll
-            for (int k = 0; k < kP2GCh; ++k)
-                bmax[k] = wave_max(pg >= 0 ? __uint_as_float(pbound[(int64_t)pg * kP2GCh + k]) : 0.f);
-            if (lane < kP2GCh) {
-                float v = bmax[0];
+            for (int k = 0; k < kP2GCh; ++k) {
+                const float m = wave_max(bnd[k]);
+                v = lane == k ? m : v;
+            }
+            if (lane < kP2GCh) sexp[lane] = fix_exp(v);
+        }
+        tile_cells<E>(L, t.cell_start, n, o3, S);   // ends in a barrier
+        float sc[kP2GCh];
 #pragma unroll
-                for (int k = 1; k < kP2GCh; ++k) v = (lane == k) ? bmax[k] : v;
-                sexp[lane] = fix_exp(v);
+        for (int k = 0; k < kP2GCh; ++k) sc[k] = ldexpf(1.0f, sexp[k]);
+        // P consecutive pairs per lane, about a cell's, so that the lanes of a
+        // wave add to different nodes
+        const int cells = S.cells, pairs = S.pairs[cells];
+        if (pairs > 0) {
+            const int all = (pairs + kTileThreads - 1) / kTileThreads, one = (pairs + cells - 1) / cells;
+            const int P = all < one ? all : one;
+            for (int c0 = tid * P; c0 < pairs; c0 += kTileThreads * P) {
+                const int ce = c0 + P < pairs ? c0 + P : pairs;
+                int r = tile_find(S, c0);
+                for (int e = c0; e < ce; ++e) {
+                    while (e >= S.pairs[r + 1]) ++r;
+                    const int place = S.place[r];
+                    p2g_pair<E, TRANSFER>(pay, S.start[r] + 2 * (e - S.pairs[r]), !(place >> 12) || e + 1 < S.pairs[r + 1],
+                                          place, sc, acc);
+                }
             }
         }
         __syncthreads();
-        int e[kP2GCh];
-        float sc[kP2GCh];
-#pragma unroll
-        for (int k = 0; k < kP2GCh; ++k) {
-            e[k] = sexp[k];
-            sc[k] = ldexpf(1.0f, e[k]);
-        }
-        int cls, jb, je;
-        if (thread_class(S, cls, jb, je)) p2g_class<TRANSFER>(S, t, pay, org, sc, acc, cls, jb, je);
-        __syncthreads();
-        // grid update of the block's pages, written page-major (coalesced)
-        for (int q = tid; q < 512; q += 256) {
-            const int o = q >> 6, cell = q & 63;
-            const int G = S.out_page[o];
+        // grid update of the tile's pages, written page-major (coalesced)
+        const uint32_t bkey = t.block_key[blk];
+        int bc[3];
+        unmorton(bkey, bc[0], bc[1], bc[2]);
+        const int org[3] = {8 * bc[0], 8 * bc[1], 8 * bc[2]};
+        const DevParams sp = dp.scenes[__builtin_amdgcn_readfirstlane(scene_of_page(dp, bkey << 3))];
+        for (int q = tid; q < E * E * E; q += kTileThreads) {
+            const int o = E == 8 ? q >> 6 : child, cell = q & 63;
+            const int G = L->out_page[o];
             if (G < 0) continue;
             const int lx = ((o >> 2) & 1) * 4 + (cell >> 4), ly = ((o >> 1) & 1) * 4 + ((cell >> 2) & 3),
                       lz = (o & 1) * 4 + (cell & 3);
-            const int node = acc_node(lx, ly, lz);
+            const int node = (lx - o3[0]) * A::kX + (ly - o3[1]) * A::kZ + (lz - o3[2]);
             float ch[kP2GCh];
 #pragma unroll
-            for (int k = 0; k < kP2GCh; ++k) ch[k] = from_fix(acc[k * kAccStride + node], e[k]);
+            for (int k = 0; k < kP2GCh; ++k) ch[k] = from_fix(acc[k * A::kStride + node], sexp[k]);
             if (grid_raw) {
                 float* rp = grid_raw + (int64_t)G * kPageFloats + cell;
 #pragma unroll
@@ -299,7 +366,6 @@ __global__ __launch_bounds__(256, 4) void k_p2g_block(DevParams dp, const float*
         __syncthreads();
     }
 }
-
 
 // the grid update after the scatter P2G: one wave per 128-node PCG block, two
 // nodes per lane
@@ -710,7 +776,7 @@ __global__ __launch_bounds__(256) void k_p2g_shell(DevParams dp, BlockTables t, 
 }
 
 // block P2G (with grid update and PCG set-up) over the payload and page bounds
-template <int TRANSFER, typename ST>
+template <int TRANSFER>
 static hipError_t gather_blocks_t(mpmx_ctx* c, float dt) {
     const BlockTables t = block_tables_of(c);
     float* raw = (c->keep_p2g && c->grid_p2g) ? c->grid_p2g : nullptr;
@@ -730,9 +796,15 @@ static hipError_t gather_blocks_t(mpmx_ctx* c, float dt) {
         timer_push(c, "p2g_block", false);
         return hipGetLastError();
     }
-    MPMX_TIMED(c, "p2g_block", (k_p2g_block<TRANSFER, ST><<<g, 256, 0, c->stream>>>(
-                                    c->dp, c->payload, c->pbound, t, static_cast<BlockClasses*>(c->block_lists),
-                                    c->grid, raw, cg_vec(c), dt, (int)c->n, c->dc)));
+    const BlockClasses* lists = static_cast<BlockClasses*>(c->block_lists);
+    if (tiles_are_pages(c))
+        MPMX_TIMED(c, "p2g_block", (k_p2g_tile<4, TRANSFER><<<8 * g, kTileThreads, 0, c->stream>>>(
+                                        c->dp, c->payload, c->pbound, t, lists, c->grid, raw, cg_vec(c), dt, (int)c->n,
+                                        c->dc)));
+    else
+        MPMX_TIMED(c, "p2g_block", (k_p2g_tile<8, TRANSFER><<<g, kTileThreads, 0, c->stream>>>(
+                                        c->dp, c->payload, c->pbound, t, lists, c->grid, raw, cg_vec(c), dt, (int)c->n,
+                                        c->dc)));
     // the PCG's starting "dot"(r, z) comes with its first "dot"(s, q) (k_cg_dot)
     return hipGetLastError();
 }
@@ -746,7 +818,7 @@ static hipError_t gather_dispatch_t(mpmx_ctx* c, ST st, float dt) {
     MPMX_TIMED(c, "p2g_prep", (k_p2g_prep<TRANSFER, ST><<<particle_blocks(c), c->particle_wg, 0, c->stream>>>(
                                    c->dp, st, c->wmap, c->sigma, c->FP, c->vol, t, c->payload, c->pbound, dt,
                                    (int)c->n, c->dc)));
-    return gather_blocks_t<TRANSFER, ST>(c, dt);
+    return gather_blocks_t<TRANSFER>(c, dt);
 }
 
 template <typename ST>
@@ -777,9 +849,7 @@ hipError_t launch_stress_p2g(mpmx_ctx* c, float dt) {
     c->order_ok = true;   // the stress pass orders the blocks
     MPMX_TIMED(c, "stress_prep", e = launch_stress_prep(c, dt));
     if (e != hipSuccess) return e;
-    const bool mixed = c->cfg.precision != MPMX_FP32;
-    if (c->P.transfer == 0) e = mixed ? gather_blocks_t<0, MState>(c, dt) : gather_blocks_t<0, PState>(c, dt);
-    else e = mixed ? gather_blocks_t<1, MState>(c, dt) : gather_blocks_t<1, PState>(c, dt);
+    e = c->P.transfer == 0 ? gather_blocks_t<0>(c, dt) : gather_blocks_t<1>(c, dt);
     c->grid_fused = true;
     return e;
 }

@@ -370,6 +370,15 @@ int block_grid(mpmx_ctx* c, int pct) {
     return nb < 8 ? 8 : (int)nb;
 }
 
+// Page tiles while the blocks (by the last published count) are at most 1.5 per
+// CU: eight times the workgroups, each particle in 3.4 tiles instead of 1.95.
+// P2G by pages / by blocks: 64,000 cube (64 blocks) 36 / 94 us, 333,333 sphere
+// (~300) 72 / 84, 512,000 cube (~340) 85 / 100, 1M impact (~550) 134 / 108,
+// 16-scene batch (~700) 82 / 66.
+bool tiles_are_pages(const mpmx_ctx* c) {
+    return c->hc->num_blocks > 0 && 2 * (int64_t)c->hc->num_blocks <= 3 * (int64_t)c->num_cu;
+}
+
 int transfer_grid_blocks(mpmx_ctx* c) {
     // enough workgroups to fill every CU several times over; a multiple of 8 so
     // that the XCD-aware remap of block ids applies

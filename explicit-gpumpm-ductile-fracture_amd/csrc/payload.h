@@ -99,10 +99,9 @@ __device__ __forceinline__ void payload_store(float* __restrict__ pay, int64_t i
     }
 }
 
-// the terms of particle i (key k) relative to the block whose first node is org
+// the terms of record i, all but the base node
 template <int TRANSFER>
-__device__ __forceinline__ void payload_load(const float* __restrict__ pay, int64_t i, uint32_t key,
-                                             const int (&org)[3], P2GTerms& T) {
+__device__ __forceinline__ void payload_terms(const float* __restrict__ pay, int64_t i, P2GTerms& T) {
     const float4* q = reinterpret_cast<const float4*>(pay + i * Payload<TRANSFER>::kFloats);
     const float4 a = q[0], b = q[1], c0 = q[2], c1 = q[3], c2 = q[4];
     const float d0[3] = {a.x, a.y, a.z};
@@ -118,17 +117,24 @@ __device__ __forceinline__ void payload_load(const float* __restrict__ pay, int6
         T.sg[4] = s1.x; T.sg[5] = s1.y; T.sg[6] = s1.z; T.sg[7] = s1.w;
         T.sg[8] = c2.w;
     }
+#pragma unroll
+    for (int ax = 0; ax < 3; ++ax) {
+        if (TRANSFER == 0) bspline(d0[ax], T.w[ax]);
+        else bspline_grad(d0[ax], T.w[ax], T.gw[ax]);
+    }
+}
+
+// the terms of particle i (key k) relative to the block whose first node is org
+template <int TRANSFER>
+__device__ __forceinline__ void payload_load(const float* __restrict__ pay, int64_t i, uint32_t key,
+                                             const int (&org)[3], P2GTerms& T) {
+    payload_terms<TRANSFER>(pay, i, T);
     int px, py, pz;
     unmorton(key >> 6, px, py, pz);
     const int cell = (int)(key & 63u);
     T.l0[0] = 4 * px + (cell >> 4) - org[0];
     T.l0[1] = 4 * py + ((cell >> 2) & 3) - org[1];
     T.l0[2] = 4 * pz + (cell & 3) - org[2];
-#pragma unroll
-    for (int ax = 0; ax < 3; ++ax) {
-        if (TRANSFER == 0) bspline(d0[ax], T.w[ax]);
-        else bspline_grad(d0[ax], T.w[ax], T.gw[ax]);
-    }
 }
 
 // payload record i of the particle whose state sits at o of s, and its
