@@ -57,6 +57,19 @@ __device__ __forceinline__ uint32_t scene_page_key(const BlockTables& t, int px,
     return (int)(k >> t.slot_shift) == scene ? k : ~0u;
 }
 
+// particles [a, b) of grid page pg of np_raw particle pages (none for a
+// neighbour-only or absent page), clamped so that stale tables after a
+// capacity overflow still index inside the arrays
+__device__ __forceinline__ void page_particles(const BlockTables& t, int pg, int np_raw, int n, int& a, int& b) {
+    const int np = np_raw < t.cap_p ? np_raw : (int)t.cap_p;
+    a = b = 0;
+    if (pg < 0 || pg >= np) return;
+    a = t.page2particle[pg];
+    b = t.page2particle[pg + 1];
+    a = a < 0 ? 0 : (a > n ? n : a);
+    b = b < a ? a : (b > n ? n : b);
+}
+
 // ---- shared pieces of the block gathers ---------------------------------------
 // A block gathers from the particle pages 2b-1 .. 2b+1 (per axis) of block b:
 // its own 8 pages, whose particles all reach it, and the 19 pages just below

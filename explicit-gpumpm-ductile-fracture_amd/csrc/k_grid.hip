@@ -797,7 +797,7 @@ static hipError_t gather_blocks_t(mpmx_ctx* c, float dt) {
         return hipGetLastError();
     }
     const BlockClasses* lists = static_cast<BlockClasses*>(c->block_lists);
-    if (tiles_are_pages(c))
+    if (tiles_are_pages(c, 150))
         MPMX_TIMED(c, "p2g_block", (k_p2g_tile<4, TRANSFER><<<8 * g, kTileThreads, 0, c->stream>>>(
                                         c->dp, c->payload, c->pbound, t, lists, c->grid, raw, cg_vec(c), dt, (int)c->n,
                                         c->dc)));

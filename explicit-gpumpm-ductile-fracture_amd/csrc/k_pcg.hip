@@ -130,118 +130,96 @@ __global__ __launch_bounds__(BLOCK) void k_cg_apply(DevParams dp, ST s, const fl
 
 // ---- block form of (K s) (variant 2) ----------------------------------------
 // col_p = M V dx^2 sum_j grad w_jp s_j for every particle of a 2x2x2 page
-// block, from the block's 10^3-node s region staged in LDS; with it, the
-// largest |col_p|_1 of each of the block's pages (cbound, float bits), from
-// which k_cg_q takes its fixed-point scale
-template <typename ST>
+// block (E = 8) or of one of its pages (E = 4), from the tile's (E + 2)^3-node
+// s region staged in LDS; with it, the largest |col_p|_1 of each of the tile's
+// pages (cbound, float bits), from which the K s gathers take their
+// fixed-point scale
+template <int E, typename ST>
 __global__ __launch_bounds__(256) void k_cg_col(DevParams dp, ST s, const float* __restrict__ vol, BlockTables t,
-                                                const float* __restrict__ cgs, float* __restrict__ col,
-                                                unsigned* __restrict__ cbound, int n,
+                                                const BlockClasses* __restrict__ lists,
+                                                const BlockG2P* __restrict__ info, const float* __restrict__ cgs,
+                                                float* __restrict__ col, unsigned* __restrict__ cbound, int n,
                                                 const SceneCG* __restrict__ scg, DevCounts* dc) {
-    constexpr int R = 10, R3 = R * R * R;
+    constexpr int R = E + 2, R3 = R * R * R;
     __shared__ float ts[R3];
-    __shared__ int spg[27];
-    __shared__ int prange[2];
-    __shared__ int opg[8];          // page ids of the block's own pages (-1: none)
-    __shared__ unsigned omax[8];    // their largest |col|_1 (float bits)
+    __shared__ unsigned omax[8];    // largest |col|_1 of the block's own pages (float bits)
     if (cg_stopped(dc)) return;
     const int np_raw = dc->num_page;
     const int np = np_raw < t.cap_p ? np_raw : (int)t.cap_p;
-    int nt = dc->num_total;
-    nt = nt < t.cap_tp ? nt : (int)t.cap_tp;
     int nb = dc->num_blocks;
     nb = nb < t.cap_blocks ? nb : (int)t.cap_blocks;
     const int tid = threadIdx.x;
-    FOR_LOGICAL_ITEMS(item, nb) {
-        const int blk = t.order ? t.order[item] : item;
+    const int items = E == 8 ? nb : 8 * nb;
+    FOR_LOGICAL_ITEMS(item, items) {
+        const int at = E == 8 ? item : item >> 3, child = E == 8 ? 0 : item & 7;
+        const int blk = t.order ? t.order[at] : at;
         const uint32_t bkey = t.block_key[blk];
         const int scene = __builtin_amdgcn_readfirstlane(scene_of_page(dp, bkey << 3));
         if (scg[scene].done) continue;   // uniform over the workgroup
+        const BlockClasses* L = lists + blk;
+        const BlockG2P* B = info + blk;
+        int pa, pb;
+        if (E == 8) {
+            pa = __builtin_amdgcn_readfirstlane(B->pa);
+            pb = __builtin_amdgcn_readfirstlane(B->pb);
+        } else {
+            page_particles(t, L->out_page[child], np_raw, n, pa, pb);
+        }
+        if (pa >= pb) continue;   // uniform; a page without particles has no bound
         const DevParams sp = dp.scenes[scene];
         const float para_scale = 4.0f * sp.L0 * sp.L0 * sp.inv_dx * sp.inv_dx;
         int bc[3];
         unmorton(bkey, bc[0], bc[1], bc[2]);
-        if (tid < 27) {
-            const int px = 2 * bc[0] + tid / 9, py = 2 * bc[1] + (tid / 3) % 3, pz = 2 * bc[2] + tid % 3;
-            int id = -1;
-            const uint32_t key = scene_page_key(t, px, py, pz, scene);
-            if (key != ~0u) id = page_rank(key, t.pmask, t.nmask, t.wpre, t.spre, np_raw);
-            spg[tid] = (id >= 0 && id < nt) ? id : -1;
-        }
-        if (tid >= 64 && tid < 128) {
-            const int o = tid - 64;
-            int id = -1;
-            if (o < 8) id = page_rank((bkey << 3) | (uint32_t)o, t.pmask, t.nmask, t.wpre, t.spre, np_raw);
-            const bool own = id >= 0 && id < np;
-            // opg and omax are written and read by these 8 threads only
-            if (o < 8) {
-                opg[o] = own ? id : -1;
-                omax[o] = 0u;
-            }
-            int lo = own ? id : 0x7fffffff, hi = own ? id : -1;
-#pragma unroll
-            for (int w = 32; w > 0; w >>= 1) {
-                lo = min(lo, __shfl_xor(lo, w, 64));
-                hi = max(hi, __shfl_xor(hi, w, 64));
-            }
-            if (o == 0) {
-                int a = 0, b = 0;
-                if (hi >= 0) {
-                    a = t.page2particle[lo];
-                    b = t.page2particle[hi + 1];
-                    a = a < 0 ? 0 : (a > n ? n : a);
-                    b = b < a ? a : (b > n ? n : b);
-                }
-                prange[0] = a;
-                prange[1] = b;
-            }
+        // the tile's first page in its block
+        const int c0 = (child >> 2) & 1, c1 = (child >> 1) & 1, c2 = child & 1;
+        if (tid < 8) omax[tid] = 0u;
+        for (int q = tid; q < R3; q += 256) {
+            const int X = q / (R * R), Y = (q / R) % R, Z = q % R;
+            const int G = B->page[((X >> 2) + c0) * 9 + ((Y >> 2) + c1) * 3 + (Z >> 2) + c2];
+            ts[q] = G >= 0 ? cgs[(int64_t)G * 64 + (((X & 3) << 4) | ((Y & 3) << 2) | (Z & 3))] : 0.f;
         }
         __syncthreads();
-        const int pa = prange[0], pb = prange[1];
-        if (pa < pb) {
-            for (int q = tid; q < R3; q += 256) {
-                const int X = q / 100, Y = (q / 10) % 10, Z = q % 10;
-                const int G = spg[(X >> 2) * 9 + (Y >> 2) * 3 + (Z >> 2)];
-                ts[q] = G >= 0 ? cgs[(int64_t)G * 64 + (((X & 3) << 4) | ((Y & 3) << 2) | (Z & 3))] : 0.f;
+        // the region's first node in scene-local cells
+        const int org[3] = {8 * bc[0] + 4 * c0 - sp.origin[0], 8 * bc[1] + 4 * c1 - sp.origin[1],
+                            8 * bc[2] + 4 * c2 - sp.origin[2]};
+        for (int i = pa + tid; i < pb; i += 256) {
+            float d0[3], w[3][3], gw[3][3];
+            int l[3];
+#pragma unroll
+            for (int a = 0; a < 3; ++a) {
+                const float xa = ld_x(s, i, a);
+                const int b = base_node(xa, sp.N);
+                d0[a] = xa * sp.inv_dx - (float)b;
+                const int la = b - org[a];
+                l[a] = la < 0 ? 0 : (la > R - 3 ? R - 3 : la);
+                bspline_grad(d0[a], w[a], gw[a]);
             }
-            __syncthreads();
-            // the region's first node in scene-local cells
-            const int org[3] = {8 * bc[0] - sp.origin[0], 8 * bc[1] - sp.origin[1], 8 * bc[2] - sp.origin[2]};
-            for (int i = pa + tid; i < pb; i += 256) {
-                float d0[3], w[3][3], gw[3][3];
-                int l[3];
+            float gs[3] = {0.f, 0.f, 0.f};
 #pragma unroll
-                for (int a = 0; a < 3; ++a) {
-                    const float xa = ld_x(s, i, a);
-                    const int b = base_node(xa, sp.N);
-                    d0[a] = xa * sp.inv_dx - (float)b;
-                    const int la = b - org[a];
-                    l[a] = la < 0 ? 0 : (la > R - 3 ? R - 3 : la);
-                    bspline_grad(d0[a], w[a], gw[a]);
-                }
-                float gs[3] = {0.f, 0.f, 0.f};
+            for (int ii = 0; ii < 3; ++ii)
 #pragma unroll
-                for (int ii = 0; ii < 3; ++ii)
+                for (int jj = 0; jj < 3; ++jj)
 #pragma unroll
-                    for (int jj = 0; jj < 3; ++jj)
-#pragma unroll
-                        for (int kk = 0; kk < 3; ++kk) {
-                            const float sv = ts[((l[0] + ii) * R + (l[1] + jj)) * R + (l[2] + kk)];
-                            gs[0] += gw[0][ii] * w[1][jj] * w[2][kk] * sv;
-                            gs[1] += w[0][ii] * gw[1][jj] * w[2][kk] * sv;
-                            gs[2] += w[0][ii] * w[1][jj] * gw[2][kk] * sv;
-                        }
-                const float sc = vol[i] * para_scale * sp.M;
-                const float c0 = gs[0] * sc, c1 = gs[1] * sc, c2 = gs[2] * sc;
-                col[3 * (int64_t)i + 0] = c0;
-                col[3 * (int64_t)i + 1] = c1;
-                col[3 * (int64_t)i + 2] = c2;
-                // the particle's page is child (key >> 6) & 7 of the block
-                atomicMax(&omax[(t.keys[i] >> 6) & 7u], __float_as_uint(fabsf(c0) + fabsf(c1) + fabsf(c2)));
-            }
+                    for (int kk = 0; kk < 3; ++kk) {
+                        const float sv = ts[((l[0] + ii) * R + (l[1] + jj)) * R + (l[2] + kk)];
+                        gs[0] += gw[0][ii] * w[1][jj] * w[2][kk] * sv;
+                        gs[1] += w[0][ii] * gw[1][jj] * w[2][kk] * sv;
+                        gs[2] += w[0][ii] * w[1][jj] * gw[2][kk] * sv;
+                    }
+            const float sc = vol[i] * para_scale * sp.M;
+            const float c0 = gs[0] * sc, c1 = gs[1] * sc, c2 = gs[2] * sc;
+            col[3 * (int64_t)i + 0] = c0;
+            col[3 * (int64_t)i + 1] = c1;
+            col[3 * (int64_t)i + 2] = c2;
+            // the particle's page is child (key >> 6) & 7 of the block
+            atomicMax(&omax[(t.keys[i] >> 6) & 7u], __float_as_uint(fabsf(c0) + fabsf(c1) + fabsf(c2)));
         }
         __syncthreads();
-        if (tid >= 64 && tid < 72 && opg[tid - 64] >= 0) cbound[opg[tid - 64]] = omax[tid - 64];
+        if (tid < 8 && (E == 8 || tid == child)) {
+            const int pg = L->out_page[tid];
+            if (pg >= 0 && pg < np) cbound[pg] = omax[tid];
+        }
+        __syncthreads();   // omax and ts are reused by the next tile
     }
 }
 
@@ -292,6 +270,66 @@ __device__ __forceinline__ void cgq_entry(const DevParams& sp, const float (&xp)
             }
         }
     }
+}
+
+// two particles of one cell at `place` of a page tile (i and, with two set, i +
+// 1) into the tile's sums, with the arithmetic of cgq_entry
+template <typename ST>
+__device__ __forceinline__ void cgq_pair(const DevParams& sp, const ST& s, int i, bool two, int place,
+                                         const float* __restrict__ col, float sc, unsigned long long* acc) {
+    using A = TileAcc<4>;
+    float w[2][3][3], gw[2][3][3], cs[2][3];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        const int k = two ? i + h : i;
+#pragma unroll
+        for (int a = 0; a < 3; ++a) {
+            const float xa = ld_x(s, k, a);
+            const float d0 = xa * sp.inv_dx - (float)base_node(xa, sp.N);
+            bspline_grad(d0, w[h][a], gw[h][a]);
+            cs[h][a] = h == 0 || two ? col[3 * (int64_t)k + a] * sc : 0.f;
+        }
+    }
+    int cnt[3], node = 0;
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+        const int l = ((place >> (8 - 4 * a)) & 15) - 2;   // cell in the tile, -2 .. 3
+        const int f = l < 0 ? 0 : l;
+        cnt[a] = (l + 3 < 4 ? l + 3 : 4) - f;
+        node += f * (a == 0 ? A::kX : (a == 1 ? A::kZ : 1));
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            drop_nodes(w[h][a], f - l);
+            drop_nodes(gw[h][a], f - l);
+        }
+    }
+#pragma unroll
+    for (int ii = 0; ii < 3; ++ii) {
+        if (ii >= cnt[0]) break;
+#pragma unroll
+        for (int jj = 0; jj < 3; ++jj) {
+            if (jj >= cnt[1]) break;
+            float rA[2], rB[2];
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                rA[h] = fmaf(gw[h][0][ii] * w[h][1][jj], cs[h][0], w[h][0][ii] * gw[h][1][jj] * cs[h][1]);
+                rB[h] = w[h][0][ii] * w[h][1][jj] * cs[h][2];
+            }
+#pragma unroll
+            for (int kk = 0; kk < 3; ++kk) {
+                if (kk >= cnt[2]) break;
+                int add = 0;
+#pragma unroll
+                for (int h = 0; h < 2; ++h) add += (int)fmaf(w[h][2][kk], rA[h], gw[h][2][kk] * rB[h]);
+                atomicAdd(&acc[node + ii * A::kX + jj * A::kZ + kk], (unsigned long long)(long long)add);
+            }
+        }
+    }
+}
+
+// q of a node from its fixed-point sum, its s and its diagonal
+__device__ __forceinline__ float cgq_node(unsigned long long sum, int e, float s, float D) {
+    return fmaf(s, D, from_fix(sum, e));
 }
 
 // entries staged in LDS per round, and the staged words per component (one
@@ -377,7 +415,77 @@ __global__ __launch_bounds__(256) void k_cg_q(DevParams dp, ST s, BlockTables t,
                       lz = (o & 1) * 4 + (cell & 3);
             const int64_t nn = (int64_t)G * 64 + cell;
             const float D = grid[(int64_t)G * kPageFloats + 7 * 64 + cell];
-            cgq[nn] = from_fix(acc[acc_node(lx, ly, lz)], e) + cgs[nn] * D;
+            cgq[nn] = cgq_node(acc[acc_node(lx, ly, lz)], e, cgs[nn], D);
+        }
+        __syncthreads();
+    }
+}
+
+// the same for one page of a block per workgroup, for scenes of few blocks:
+// the page's cells and pairs as in the P2G (TileCells), the particles read
+// directly (such a scene's positions and columns stay in the L2), two particles
+// of a cell per atomic (|grad w . col| <= 0.75^2 |col|_1, so two terms of at
+// most 2^30 times that add up in 32 bits).  The scale is the block's, so the
+// sums are k_cg_q's bit for bit.  64,000 cube 74 -> 16 us, 333,333 sphere
+// 60 -> 30.
+template <typename ST>
+__global__ __launch_bounds__(kTileThreads) void k_cg_q_page(DevParams dp, ST s, BlockTables t,
+                                                            const BlockClasses* __restrict__ lists,
+                                                            const float* __restrict__ col,
+                                                            const unsigned* __restrict__ cbound,
+                                                            const float* __restrict__ grid,
+                                                            const float* __restrict__ cgs, float* __restrict__ cgq,
+                                                            int n, const SceneCG* __restrict__ scg, DevCounts* dc) {
+    using A = TileAcc<4>;
+    __shared__ unsigned long long acc[A::kStride];
+    __shared__ TileCells<4> S;
+    __shared__ int sexp;
+    if (cg_stopped(dc)) return;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    int nb = dc->num_blocks;
+    nb = nb < t.cap_blocks ? nb : (int)t.cap_blocks;
+    FOR_LOGICAL_ITEMS(item, 8 * nb) {
+        const int at = item >> 3, child = item & 7;
+        const int blk = t.order ? t.order[at] : at;
+        const BlockClasses* L = lists + blk;
+        const int G = L->out_page[child];
+        if (G < 0) continue;   // uniform over the workgroup
+        const uint32_t bkey = t.block_key[blk];
+        const int scene = __builtin_amdgcn_readfirstlane(scene_of_page(dp, bkey << 3));
+        if (scg[scene].done) continue;   // uniform over the workgroup
+        const int o3[3] = {4 * ((child >> 2) & 1), 4 * ((child >> 1) & 1), 4 * (child & 1)};
+        for (int q = tid; q < A::kStride; q += kTileThreads) acc[q] = 0ull;
+        if (wave == 1) {
+            const int pg = lane < 27 ? L->page[lane] : -1;
+            const float bm = wave_max(pg >= 0 ? __uint_as_float(cbound[pg]) : 0.f);
+            if (lane == 0) sexp = fix_exp(bm);
+        }
+        tile_cells<4>(L, t.cell_start, n, o3, S);   // ends in a barrier
+        const int e = sexp;
+        const float sc = ldexpf(1.0f, e);
+        const DevParams sp = dp.scenes[scene];
+        const int cells = S.cells, pairs = S.pairs[cells];
+        if (pairs > 0) {
+            // as in the P2G: about a cell's pairs per lane
+            const int all = (pairs + kTileThreads - 1) / kTileThreads, one = (pairs + cells - 1) / cells;
+            const int P = all < one ? all : one;
+            for (int c0 = tid * P; c0 < pairs; c0 += kTileThreads * P) {
+                const int ce = c0 + P < pairs ? c0 + P : pairs;
+                int r = tile_find(S, c0);
+                for (int q = c0; q < ce; ++q) {
+                    while (q >= S.pairs[r + 1]) ++r;
+                    const int place = S.place[r], i = S.start[r] + 2 * (q - S.pairs[r]);
+                    const bool two = !(place >> 12) || q + 1 < S.pairs[r + 1];
+                    cgq_pair(sp, s, i, two, place, col, sc, acc);
+                }
+            }
+        }
+        __syncthreads();
+        if (tid < 64) {
+            const int node = (tid >> 4) * A::kX + ((tid >> 2) & 3) * A::kZ + (tid & 3);
+            const int64_t nn = (int64_t)G * 64 + tid;
+            const float D = grid[(int64_t)G * kPageFloats + 7 * 64 + tid];
+            cgq[nn] = cgq_node(acc[node], e, cgs[nn], D);
         }
         __syncthreads();
     }
@@ -568,12 +676,21 @@ static void apply_block(mpmx_ctx* c, ST st) {
 template <typename ST>
 static void apply_blocks(mpmx_ctx* c, ST st) {
     const BlockTables t = block_tables_of(c);
-    const int g1 = block_grid(c, c->cg_pct), g2 = g1;
-    MPMX_TIMED(c, "cg_col", (k_cg_col<ST><<<(int)g1, 256, 0, c->stream>>>(
-                                c->dp, st, c->vol, t, c->cg_s, c->cg_col, c->cbound, (int)c->n, c->scg, c->dc)));
-    MPMX_TIMED(c, "cg_q", (k_cg_q<ST><<<(int)g2, 256, 0, c->stream>>>(
-                              c->dp, st, t, static_cast<const BlockClasses*>(c->block_lists), c->cg_col, c->cbound,
-                              c->grid, c->cg_s, c->cg_q, (int)c->n, c->scg, c->dc)));
+    const BlockClasses* lists = static_cast<const BlockClasses*>(c->block_lists);
+    const BlockG2P* info = static_cast<const BlockG2P*>(c->block_g2p);
+    const int g = block_grid(c, c->cg_pct), n = (int)c->n;
+    if (tiles_are_pages(c, 400)) {
+        MPMX_TIMED(c, "cg_col", (k_cg_col<4, ST><<<8 * g, 256, 0, c->stream>>>(c->dp, st, c->vol, t, lists, info, c->cg_s,
+                                                                            c->cg_col, c->cbound, n, c->scg, c->dc)));
+        MPMX_TIMED(c, "cg_q", (k_cg_q_page<ST><<<8 * g, kTileThreads, 0, c->stream>>>(
+                                  c->dp, st, t, lists, c->cg_col, c->cbound, c->grid, c->cg_s, c->cg_q, n, c->scg,
+                                  c->dc)));
+        return;
+    }
+    MPMX_TIMED(c, "cg_col", (k_cg_col<8, ST><<<g, 256, 0, c->stream>>>(c->dp, st, c->vol, t, lists, info, c->cg_s,
+                                                                    c->cg_col, c->cbound, n, c->scg, c->dc)));
+    MPMX_TIMED(c, "cg_q", (k_cg_q<ST><<<g, 256, 0, c->stream>>>(c->dp, st, t, lists, c->cg_col, c->cbound, c->grid,
+                                                              c->cg_s, c->cg_q, n, c->scg, c->dc)));
 }
 
 static hipError_t pcg_iteration(mpmx_ctx* c, int k) {

@@ -293,56 +293,67 @@ __global__ __launch_bounds__(BLOCK) void k_g2p(DevParams dp, ST s, Tables t, con
     }
 }
 
-// block G2P (variant 2): a workgroup stages the 10^3 nodes that the particles
-// of one 2x2x2 page block reach (the block's 8^3 nodes and two layers of the
-// +x/+y/+z neighbours) and runs every particle of the block; the block's
-// particles are one contiguous range because its 8 pages are consecutive
-// Morton codes.  The region's grid pages and the particle range come with the
-// page tables (BlockG2P).
-constexpr int kBR = 10;                       // staged region edge
-constexpr int kBR3 = kBR * kBR * kBR;
-
-template <int TRANSFER, typename ST>
+// block G2P (variant 2): a workgroup stages the (E + 2)^3 nodes that the
+// particles of one 2x2x2 page block (E = 8) or of one of its pages (E = 4)
+// reach (the tile's nodes and two layers of the +x/+y/+z neighbours) and runs
+// the tile's particles, one contiguous range (a block's 8 pages are
+// consecutive Morton codes).  The block's grid pages and particle range come
+// with the page tables (BlockG2P).  Pages where the blocks are few
+// (tiles_are_pages): 64,000 cube 48 -> 13 us, 333,333 sphere 74 -> 31.
+template <int E, int TRANSFER, typename ST>
 __global__ __launch_bounds__(256) void k_g2p_block(DevParams dp, ST s, BlockTables t,
+                                                   const BlockClasses* __restrict__ lists,
                                                    const BlockG2P* __restrict__ info, const float* __restrict__ grid,
                                                    const float* __restrict__ cgx, uint32_t* __restrict__ keys,
                                                    float dt, int n, const SceneCG* __restrict__ scg, DevCounts* dc) {
-    __shared__ float tv[4 * kBR3];
+    constexpr int R = E + 2, R3 = R * R * R;
+    __shared__ float tv[4 * R3];
     dt = substep_dt(dt, dc);
     int nb = dc->num_blocks;
     nb = nb < t.cap_blocks ? nb : (int)t.cap_blocks;
-    FOR_LOGICAL_ITEMS(item, nb) {
-        const int blk = t.order ? t.order[item] : item;
+    const int items = E == 8 ? nb : 8 * nb;
+    FOR_LOGICAL_ITEMS(item, items) {
+        const int at = E == 8 ? item : item >> 3, child = E == 8 ? 0 : item & 7;
+        const int blk = t.order ? t.order[at] : at;
         const uint32_t bkey = t.block_key[blk];
         const int scene = __builtin_amdgcn_readfirstlane(scene_of_page(dp, bkey << 3));
-        const DevParams sp = dp.scenes[scene];   // loaded once per block, before the particle loop
+        const DevParams sp = dp.scenes[scene];   // loaded once per tile, before the particle loop
         const bool breakdown = scg[scene].breakdown != 0;
         int bc[3];
         unmorton(bkey, bc[0], bc[1], bc[2]);
         const int tid = threadIdx.x;
         const BlockG2P* B = info + blk;
-        const int pa = __builtin_amdgcn_readfirstlane(B->pa), pb = __builtin_amdgcn_readfirstlane(B->pb);
+        int pa, pb;
+        if (E == 8) {
+            pa = __builtin_amdgcn_readfirstlane(B->pa);
+            pb = __builtin_amdgcn_readfirstlane(B->pb);
+        } else {
+            page_particles(t, lists[blk].out_page[child], dc->num_page, n, pa, pb);
+        }
         if (pa < pb) {
+            // the tile's first page in its block
+            const int c0 = (child >> 2) & 1, c1 = (child >> 1) & 1, c2 = child & 1;
             // the thread's first particle, loaded while the region is staged
             G2PIn P;
             if (pa + tid < pb) g2p_load(s, pa + tid, P);
-            for (int q = tid; q < kBR3; q += 256) {
-                const int X = q / 100, Y = (q / 10) % 10, Z = q % 10;
-                const int G = B->page[(X >> 2) * 9 + (Y >> 2) * 3 + (Z >> 2)];
+            for (int q = tid; q < R3; q += 256) {
+                const int X = q / (R * R), Y = (q / R) % R, Z = q % R;
+                const int G = B->page[((X >> 2) + c0) * 9 + ((Y >> 2) + c1) * 3 + (Z >> 2) + c2];
                 float v0 = 0.f, v1 = 0.f, v2 = 0.f, dcn = 0.f;
                 if (G >= 0)
                     g2p_node(sp, grid, cgx, breakdown, (int64_t)G * 64 + (((X & 3) << 4) | ((Y & 3) << 2) | (Z & 3)),
                              v0, v1, v2, dcn);
                 tv[q] = v0;
-                tv[kBR3 + q] = v1;
-                tv[2 * kBR3 + q] = v2;
-                tv[3 * kBR3 + q] = dcn;
+                tv[R3 + q] = v1;
+                tv[2 * R3 + q] = v2;
+                tv[3 * R3 + q] = dcn;
             }
             __syncthreads();
-            const int org[3] = {8 * bc[0] - sp.origin[0], 8 * bc[1] - sp.origin[1], 8 * bc[2] - sp.origin[2]};
+            const int org[3] = {8 * bc[0] + 4 * c0 - sp.origin[0], 8 * bc[1] + 4 * c1 - sp.origin[1],
+                                8 * bc[2] + 4 * c2 - sp.origin[2]};
             for (int i = pa + tid; i < pb; i += 256) {
                 if (i != pa + tid) g2p_load(s, i, P);
-                g2p_particle<TRANSFER, kBR>(sp, s, i, n, dt, org, tv, P, keys, dc);
+                g2p_particle<TRANSFER, R>(sp, s, i, n, dt, org, tv, P, keys, dc);
             }
             __syncthreads();
         }
@@ -370,13 +381,17 @@ int block_grid(mpmx_ctx* c, int pct) {
     return nb < 8 ? 8 : (int)nb;
 }
 
-// Page tiles while the blocks (by the last published count) are at most 1.5 per
-// CU: eight times the workgroups, each particle in 3.4 tiles instead of 1.95.
-// P2G by pages / by blocks: 64,000 cube (64 blocks) 36 / 94 us, 333,333 sphere
-// (~300) 72 / 84, 512,000 cube (~340) 85 / 100, 1M impact (~550) 134 / 108,
-// 16-scene batch (~700) 82 / 66.
-bool tiles_are_pages(const mpmx_ctx* c) {
-    return c->hc->num_blocks > 0 && 2 * (int64_t)c->hc->num_blocks <= 3 * (int64_t)c->num_cu;
+// Page tiles while the blocks (by the last published count) are at most
+// percent % of the CUs: eight times the workgroups, but each particle in 3.4
+// gather tiles instead of 1.95, and 3.4 nodes staged per node instead of 1.95.
+// P2G (150): by pages / by blocks, 64,000 cube (64 blocks) 36 / 94 us, 333,333
+// sphere (~300) 72 / 84, 512,000 cube (~340) 85 / 100, 1M impact (~450) 134 /
+// 108, 16-scene batch (~600) 82 / 66.
+// K s gather, K s column and G2P (400), which leave more of the GPU idle by
+// blocks: 1M impact 62 / 78, 17 / 26 and 52 / 73 us, 16-scene batch 32 / 42, 11
+// / 14 and 26 / 34, 64-scene batch (~2,400) 103 / 48, 33 / 19 and 104 / 68.
+bool tiles_are_pages(const mpmx_ctx* c, int percent) {
+    return c->hc->num_blocks > 0 && 100 * (int64_t)c->hc->num_blocks <= percent * (int64_t)c->num_cu;
 }
 
 int transfer_grid_blocks(mpmx_ctx* c) {
@@ -439,20 +454,26 @@ static void g2p_block(mpmx_ctx* c, ST st, float dt) {
     }
 }
 
-template <typename ST>
-static void g2p_block_kernel(mpmx_ctx* c, ST st, float dt) {
+template <int E, int TRANSFER, typename ST>
+static void g2p_block_launch(mpmx_ctx* c, ST st, float dt) {
     // the blocks in the gathers' order (by gather entries; a block's own
     // particles, the G2P's work, go with them): 0.34 -> 0.29 ms on the 8M
     // impact against block order
-    const BlockTables t = block_tables_of(c);
-    const int g = block_grid(c, c->g2p_pct);
+    const int g = block_grid(c, c->g2p_pct) * (E == 8 ? 1 : 8);
+    k_g2p_block<E, TRANSFER, ST><<<g, 256, 0, c->stream>>>(
+        c->dp, st, block_tables_of(c), static_cast<const BlockClasses*>(c->block_lists),
+        static_cast<const BlockG2P*>(c->block_g2p), c->grid, c->cg_x, c->keys_next, dt, (int)c->n, c->scg, c->dc);
+}
+template <typename ST>
+static void g2p_block_kernel(mpmx_ctx* c, ST st, float dt) {
     MPMX_TIMED(c, "g2p_block", ({
-                   if (c->P.transfer == 0)
-                       k_g2p_block<0, ST><<<(int)g, 256, 0, c->stream>>>(c->dp, st, t, static_cast<const BlockG2P*>(c->block_g2p), c->grid, c->cg_x, c->keys_next, dt,
-                                                                         (int)c->n, c->scg, c->dc);
-                   else
-                       k_g2p_block<1, ST><<<(int)g, 256, 0, c->stream>>>(c->dp, st, t, static_cast<const BlockG2P*>(c->block_g2p), c->grid, c->cg_x, c->keys_next, dt,
-                                                                         (int)c->n, c->scg, c->dc);
+                   if (tiles_are_pages(c, 400)) {
+                       if (c->P.transfer == 0) g2p_block_launch<4, 0>(c, st, dt);
+                       else g2p_block_launch<4, 1>(c, st, dt);
+                   } else {
+                       if (c->P.transfer == 0) g2p_block_launch<8, 0>(c, st, dt);
+                       else g2p_block_launch<8, 1>(c, st, dt);
+                   }
                }));
 }
 
