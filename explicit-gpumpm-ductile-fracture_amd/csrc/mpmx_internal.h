@@ -432,6 +432,22 @@ __device__ __forceinline__ float wave_max(float v) {
     return v;
 }
 
+// the same for v >= 0, in VALU lane moves (DPP: shifts by 1, 2, 4 and 8 inside
+// rows of 16 lanes, then the last lane of a row to the next row or rows)
+// instead of LDS permutes; every lane active
+__device__ __forceinline__ float wave_max_nonneg(float v) {
+    int b = __float_as_int(v);   // non-negative floats order like their bits
+#define MPMX_DPP_MAX(ctrl, rows) b = max(b, __builtin_amdgcn_update_dpp(0, b, ctrl, rows, 0xf, false))
+    MPMX_DPP_MAX(0x111, 0xf);
+    MPMX_DPP_MAX(0x112, 0xf);
+    MPMX_DPP_MAX(0x114, 0xf);
+    MPMX_DPP_MAX(0x118, 0xf);
+    MPMX_DPP_MAX(0x142, 0xa);
+    MPMX_DPP_MAX(0x143, 0xc);
+#undef MPMX_DPP_MAX
+    return __int_as_float(__builtin_amdgcn_readlane(b, 63));
+}
+
 // max (MAX) or sum of parts[0..cnt) for every thread of the workgroup, in a
 // fixed order (thread-strided, wave butterfly, waves in order); lds holds one
 // float per wave
