@@ -127,10 +127,10 @@ __device__ __forceinline__ void scene_counts_of(const DevParams& dp, int s, cons
 // each scene's page ranges, one thread per bitmap word
 __global__ void k_page_keys(DevParams dp, const uint64_t* __restrict__ pmask, const uint64_t* __restrict__ nmask,
                             const int* __restrict__ wpre, const int* __restrict__ spre,
-                            const int* __restrict__ bpre, int64_t words, uint32_t* page_key, int64_t cap_p,
+                            const int* __restrict__ bpre, int64_t words, int per, uint32_t* page_key, int64_t cap_p,
                             int64_t cap_tp, uint32_t* __restrict__ block_key, int64_t cap_blocks,
                             SceneCG* __restrict__ scg, DevCounts* dc) {
-    // a wave per 64 consecutive words: one lane per word finds the words that
+    // a wave per `per` (<= 64) consecutive words: one lane per word finds the words that
     // hold a page (a batch's page space is mostly empty), then the wave takes
     // those words one at a time with one lane per bit: a set bit's id is the
     // word's prefix plus the set bits below it.  The 2x2x2-page blocks of the
@@ -147,10 +147,10 @@ __global__ void k_page_keys(DevParams dp, const uint64_t* __restrict__ pmask, co
         if (num_page > cap_p || total > cap_tp) atomicOr(&dc->err, kErrCapacity);
     }
     if (t < dp.num_scenes) scene_counts_of(dp, (int)t, wpre, spre, scg, dc);
-    const int64_t w0 = (t >> 6) * 64;   // the wave's first word
+    const int64_t w0 = (t >> 6) * per;   // the wave's first word
     uint64_t Pl = 0ull, Nl = 0ull;
     int wl = 0, sl = 0, bl = 0;         // the word's prefixes, loaded with it (the loop below only shuffles)
-    if (w0 + b < words) {
+    if (b < per && w0 + b < words) {
         Pl = pmask[w0 + b];
         Nl = nmask[w0 + b];
         wl = wpre[w0 + b];
@@ -353,10 +353,13 @@ hipError_t build_tables(mpmx_ctx* c) {
     ScanSet3 sc{{c->wcount, c->scount, c->bcount}, {c->wcount, c->scount, c->bcount},
                 {&c->dc->num_page, &c->dc->num_supp, &c->dc->num_blocks}};
     if ((e = scan_exclusive3(c, sc, 3, words)) != hipSuccess) return e;
-    // one thread per word (at least one workgroup: its first threads also
-    // write the per-scene page ranges)
-    k_page_keys<<<(int)std::max<int64_t>(1, (words + 255) / 256), 256, 0, c->stream>>>(
-        c->dp, c->pmask, c->nmask, c->wcount, c->scount, c->bcount, words, c->page_key, c->cap_p, c->cap_tp,
+    // words per wave: a wave takes its occupied words one after another, so
+    // the words are spread out (8 a wave, 1M bar's 4,096 words 38 -> 7 us) until
+    // there are waves enough without (64 a wave: a batch's mostly empty ones).
+    // At least a thread per word: the first also write the per-scene ranges.
+    const int per = words <= (1 << 17) ? 8 : 64;
+    k_page_keys<<<(int)((words + 4 * per - 1) / (4 * per)), 256, 0, c->stream>>>(
+        c->dp, c->pmask, c->nmask, c->wcount, c->scount, c->bcount, words, per, c->page_key, c->cap_p, c->cap_tp,
         c->block_key, c->tp_bound, c->scg, c->dc);
     k_page_heads<<<(n + 256 * kHeadItems - 1) / (256 * kHeadItems), 256, 0, c->stream>>>(c->keys, n, c->pmask, c->nmask, c->wcount, c->scount,
                                                           c->page2particle, c->cell_start, c->cap_p, c->dc);
