@@ -13,6 +13,7 @@
 // One lane per particle; F, sigma component-major (coalesced across lanes).
 #include "payload.h"
 #include "svd3.h"
+#include <type_traits>
 
 namespace mpmx {
 
@@ -35,18 +36,15 @@ __device__ __forceinline__ void usv(const T (&U)[3][3], const T (&d)[3], const T
             P[r][cc] = d[0] * U[r][0] * V[cc][0] + d[1] * U[r][1] * V[cc][1] + d[2] * U[r][2] * V[cc][2];
 }
 
-// the return mapping in precision T (float, or double for the near-degenerate fallback)
+// the return mapping in the principal axes: S becomes the final singular values
+// (returns whether they changed), P_hat the principal first Piola stress;
+// alpha, psi, FP and g are set
 template <typename T>
-__device__ __forceinline__ void von_mises(const DevParams& dp, const StressIn& in, StressOut& out,
-                                          const T (&U)[3][3], T (&S)[3], const T (&V)[3][3]) {
+__device__ __forceinline__ bool von_mises(const DevParams& dp, const StressIn& in, StressOut& out, T (&S)[3],
+                                          T (&P_hat)[3]) {
     const T lambda = dp.lambda, mu = dp.mu, kappa = dp.kappa;
     T g = in.g;
     T alpha = in.alpha;
-    T Fm[3][3];
-#pragma unroll
-    for (int r = 0; r < 3; ++r)
-#pragma unroll
-        for (int cc = 0; cc < 3; ++cc) Fm[r][cc] = in.F[r][cc];
 
     const T c0 = T(2) * mu + lambda;
     T eps[3];
@@ -69,7 +67,8 @@ __device__ __forceinline__ void von_mises(const DevParams& dp, const StressIn& i
     const T sq23 = sqrt(p23);
     const T Rh = T(dp.sq23f) * T(dp.yield) - (T(dp.sq23f) * T(dp.yield) - T(dp.yield)) * exp(-T(dp.hard) * alpha);
     const T y = tau_tr_F - g * Rh * sq23;
-    if (y >= T(1e-12)) {
+    const bool flow = y >= T(1e-12);
+    if (flow) {
         T dlambda = T(0);
         const T bss = p23 * g * tau_tr_sum;
         if (bss > T(0)) dlambda = y / bss;
@@ -102,24 +101,19 @@ __device__ __forceinline__ void von_mises(const DevParams& dp, const StressIn& i
             S[a] = exp(eps_nn[a]);
             lnS[a] = eps_nn[a];
         }
-        usv(U, S, V, Fm);
     }
-#pragma unroll
-    for (int r = 0; r < 3; ++r)
-#pragma unroll
-        for (int cc = 0; cc < 3; ++cc) out.F[r][cc] = (float)Fm[r][cc];
 
     const T J = S[0] * S[1] * S[2];
-    // J^(-2/3) and ln J from the logarithms already at hand where every
-    // singular value is positive (one exp instead of pow and log)
+    // J^(-2/3) and ln J from the logarithms already at hand; a singular value
+    // that is not positive makes J <= 0
     const bool pos = S[0] > T(0) && S[1] > T(0) && S[2] > T(0);
     const T lnJ = lnS[0] + lnS[1] + lnS[2];
-    const T J_bar = pos ? exp(-p23 * lnJ) : pow(J, -p23);
+    const T J_bar = pos ? exp(-p23 * lnJ) : (J == T(0) ? T(INFINITY) : T(NAN));
     T be[3];
 #pragma unroll
     for (int a = 0; a < 3; ++a) be[a] = J_bar * S[a] * S[a];
     const T be_sum = be[0] + be[1] + be[2];
-    const T ln_J = pos ? lnJ : ((J > T(0)) ? log(J) : T(0));
+    const T ln_J = pos ? lnJ : T(0);
     const T Psi_vol = (kappa * T(0.5)) * (((J * J - T(1)) * T(0.5)) - ln_J);
     const T Psi_dev = (mu * T(0.5)) * (be_sum - T(3));
     const T Psi_pos = (J < T(1)) ? Psi_dev : Psi_dev + Psi_vol;
@@ -138,45 +132,12 @@ __device__ __forceinline__ void von_mises(const DevParams& dp, const StressIn& i
     const T bthird = (T(1) / T(3)) * be_sum;
     g = T(in.c) * T(in.c) * (T(1) - theta) + theta;
     out.g = (float)g;
-    T P_hat[3];
 #pragma unroll
     for (int a = 0; a < 3; ++a) {
         const T td = mu * (be[a] - bthird);
         P_hat[a] = (J < T(1)) ? g * td + tau_vol : g * (td + tau_vol);
     }
-    T P[3][3];
-    usv(U, P_hat, V, P);
-    // sigma = V0 P F^T
-#pragma unroll
-    for (int r = 0; r < 3; ++r)
-#pragma unroll
-        for (int cc = 0; cc < 3; ++cc)
-            out.sigma[r][cc] = (float)((P[r][0] * Fm[cc][0] + P[r][1] * Fm[cc][1] + P[r][2] * Fm[cc][2]) * T(dp.V0));
-    const T det = Fm[0][0] * (Fm[1][1] * Fm[2][2] - Fm[1][2] * Fm[2][1]) -
-                  Fm[0][1] * (Fm[1][0] * Fm[2][2] - Fm[1][2] * Fm[2][0]) +
-                  Fm[0][2] * (Fm[1][0] * Fm[2][1] - Fm[1][1] * Fm[2][0]);
-    out.vol = (float)(T(dp.V0) * det);
-}
-
-// sigma = V0 U diag(P_hat) V^T F^T, F = in.F
-template <typename T>
-__device__ __forceinline__ void contribution(const DevParams& dp, const StressIn& in, const T (&U)[3][3],
-                                             const T (&P_hat)[3], const T (&V)[3][3], StressOut& out) {
-    T P[3][3];
-    usv(U, P_hat, V, P);
-#pragma unroll
-    for (int r = 0; r < 3; ++r)
-#pragma unroll
-        for (int cc = 0; cc < 3; ++cc)
-            out.sigma[r][cc] = (float)((P[r][0] * T(in.F[cc][0]) + P[r][1] * T(in.F[cc][1]) + P[r][2] * T(in.F[cc][2])) *
-                                       T(dp.V0));
-}
-
-template <typename T>
-__device__ __forceinline__ T det3(const float (&F)[3][3]) {
-    return T(F[0][0]) * (T(F[1][1]) * T(F[2][2]) - T(F[1][2]) * T(F[2][1])) -
-           T(F[0][1]) * (T(F[1][0]) * T(F[2][2]) - T(F[1][2]) * T(F[2][0])) +
-           T(F[0][2]) * (T(F[1][0]) * T(F[2][1]) - T(F[1][1]) * T(F[2][0]));
+    return flow;
 }
 
 // computeContributionNeoHookean (ExplicitTimeIntegrator.cu:372-446): phase-
@@ -186,21 +147,17 @@ __device__ __forceinline__ T det3(const float (&F)[3][3]) {
 // and ln J is unguarded.
 template <typename T>
 __device__ __forceinline__ void neo_hookean(const DevParams& dp, const StressIn& in, StressOut& out,
-                                            const T (&U)[3][3], const T (&S)[3], const T (&V)[3][3]) {
+                                            const T (&S)[3], T (&P_hat)[3]) {
     const T mu = dp.mu, kappa = dp.kappa;
-#pragma unroll
-    for (int r = 0; r < 3; ++r)
-#pragma unroll
-        for (int cc = 0; cc < 3; ++cc) out.F[r][cc] = in.F[r][cc];
     out.g = in.g;
     out.alpha = in.alpha;
     const T J = S[0] * S[1] * S[2];
-    const T J_bar = pow(J, -T(2.0f / 3.0f));
+    const T ln_J = log(J);
+    const T J_bar = exp(-T(2.0f / 3.0f) * ln_J);
     T be[3];
 #pragma unroll
     for (int a = 0; a < 3; ++a) be[a] = J_bar * S[a] * S[a];
     const T be_sum = be[0] + be[1] + be[2];
-    const T ln_J = log(J);
     const T Psi_vol = kappa / T(2) * ((J - T(1)) / T(2) - ln_J);
     const T Psi_dev = mu / T(2) * (be_sum - T(3));
     const T Psi_pos = (J < T(1)) ? Psi_dev : Psi_dev + Psi_vol;
@@ -213,14 +170,11 @@ __device__ __forceinline__ void neo_hookean(const DevParams& dp, const StressIn&
     const T third = (T(1) / T(3)) * be_sum;
     const T theta = dp.theta;
     const T g = T(in.c) * T(in.c) * (T(1) - theta) + theta;
-    T P_hat[3];
 #pragma unroll
     for (int a = 0; a < 3; ++a) {
         const T td = mu * (be[a] - third);
         P_hat[a] = (J < T(1)) ? g * td + tau_vol : g * (td + tau_vol);
     }
-    contribution<T>(dp, in, U, P_hat, V, out);
-    out.vol = (float)(T(dp.V0) * det3<T>(in.F));
 }
 
 // computeContributionFixedCorotated (ExplicitTimeIntegrator.cu:22-47): no
@@ -228,35 +182,106 @@ __device__ __forceinline__ void neo_hookean(const DevParams& dp, const StressIn&
 // for the record; the solve does not run)
 template <typename T>
 __device__ __forceinline__ void fixed_corotated(const DevParams& dp, const StressIn& in, StressOut& out,
-                                                const T (&U)[3][3], const T (&S)[3], const T (&V)[3][3]) {
-#pragma unroll
-    for (int r = 0; r < 3; ++r)
-#pragma unroll
-        for (int cc = 0; cc < 3; ++cc) out.F[r][cc] = in.F[r][cc];
+                                                const T (&S)[3], T (&P_hat)[3]) {
     out.g = in.g;
     out.alpha = in.alpha;
     out.psi = in.psi;
     const T mu = dp.mu, lambda = dp.lambda;
     const T J = S[0] * S[1] * S[2];
     const T scaled_mu = T(2) * mu, scaled_lambda = lambda * (J - T(1));
-    const T P_hat[3] = {scaled_mu * (S[0] - T(1)) + scaled_lambda * (S[1] * S[2]),
-                        scaled_mu * (S[1] - T(1)) + scaled_lambda * (S[0] * S[2]),
-                        scaled_mu * (S[2] - T(1)) + scaled_lambda * (S[0] * S[1])};
-    contribution<T>(dp, in, U, P_hat, V, out);
+    P_hat[0] = scaled_mu * (S[0] - T(1)) + scaled_lambda * (S[1] * S[2]);
+    P_hat[1] = scaled_mu * (S[1] - T(1)) + scaled_lambda * (S[0] * S[2]);
+    P_hat[2] = scaled_mu * (S[2] - T(1)) + scaled_lambda * (S[0] * S[1]);
     out.FP = 1.0f;
-    out.vol = (float)(T(dp.V0) * det3<T>(in.F));
 }
 
-// the energy of the scene: von Mises (2), Neo-Hookean (1), fixed corotated (0)
+// the energy of the scene: von Mises (2), Neo-Hookean (1), fixed corotated (0);
+// whether the singular values changed
+template <typename T>
+__device__ __forceinline__ bool principal(const DevParams& dp, const StressIn& in, StressOut& out, T (&S)[3],
+                                          T (&P_hat)[3]) {
+    if (dp.model == 2) return von_mises<T>(dp, in, out, S, P_hat);
+    if (dp.model == 1) neo_hookean<T>(dp, in, out, S, P_hat);
+    else fixed_corotated<T>(dp, in, out, S, P_hat);
+    return false;
+}
+
+// the energy from a full decomposition F = U diag(S) V^T:
+// sigma = V0 P F^T with P = U diag(P_hat) V^T and the final F
 template <typename T>
 __device__ __forceinline__ void energy(const DevParams& dp, const StressIn& in, StressOut& out,
                                        const T (&U)[3][3], T (&S)[3], const T (&V)[3][3]) {
-    if (dp.model == 2) von_mises<T>(dp, in, out, U, S, V);
-    else if (dp.model == 1) neo_hookean<T>(dp, in, out, U, S, V);
-    else fixed_corotated<T>(dp, in, out, U, S, V);
+    T P_hat[3], P[3][3], Fm[3][3];
+    const bool changed = principal<T>(dp, in, out, S, P_hat);
+#pragma unroll
+    for (int r = 0; r < 3; ++r)
+#pragma unroll
+        for (int cc = 0; cc < 3; ++cc) Fm[r][cc] = in.F[r][cc];
+    if (changed) usv(U, S, V, Fm);
+    usv(U, P_hat, V, P);
+#pragma unroll
+    for (int r = 0; r < 3; ++r)
+#pragma unroll
+        for (int cc = 0; cc < 3; ++cc) {
+            out.F[r][cc] = (float)Fm[r][cc];
+            out.sigma[r][cc] = (float)((P[r][0] * Fm[cc][0] + P[r][1] * Fm[cc][1] + P[r][2] * Fm[cc][2]) * T(dp.V0));
+        }
+    const T det = Fm[0][0] * (Fm[1][1] * Fm[2][2] - Fm[1][2] * Fm[2][1]) -
+                  Fm[0][1] * (Fm[1][0] * Fm[2][2] - Fm[1][2] * Fm[2][0]) +
+                  Fm[0][2] * (Fm[1][0] * Fm[2][1] - Fm[1][1] * Fm[2][0]);
+    out.vol = (float)(T(dp.V0) * det);
 }
 
-// ALL64: SVD and return mapping in FP64 for every particle.  Otherwise FP32,
+// the energy in FP64 from the principal axes alone:
+// sigma = V0 sum_a P_hat_a S_a u_a u_a^T, final F = sum_a (S_a / S_a before) u_a u_a^T F,
+// V = V0 S_0 S_1 S_2
+__device__ __forceinline__ void energy64(const DevParams& dp, const StressIn& in, StressOut& out) {
+    double U[3][3], S[3], R[3], P_hat[3];
+    const bool regular = principal_axes(in.F, U, S, R);
+    const bool changed = principal<double>(dp, in, out, S, P_hat);
+    const double V0 = dp.V0;
+    out.vol = (float)(V0 * (S[0] * S[1] * S[2]));
+#pragma unroll
+    for (int r = 0; r < 3; ++r)
+#pragma unroll
+        for (int cc = 0; cc < 3; ++cc) out.F[r][cc] = in.F[r][cc];
+    if (!regular) {
+        double V[3][3], Fm[3][3];
+        principal_axes_singular(in.F, R, U, V);
+        usv(U, S, V, Fm);
+#pragma unroll
+        for (int r = 0; r < 3; ++r)
+#pragma unroll
+            for (int cc = 0; cc < 3; ++cc) out.F[r][cc] = changed ? (float)Fm[r][cc] : out.F[r][cc];
+    } else if (changed) {
+        double M[3][3];
+#pragma unroll
+        for (int a = 0; a < 3; ++a) R[a] *= S[a];
+#pragma unroll
+        for (int r = 0; r < 3; ++r)
+#pragma unroll
+            for (int cc = 0; cc <= r; ++cc)
+                M[r][cc] = M[cc][r] = fma(R[2] * U[r][2], U[cc][2],
+                                          fma(R[1] * U[r][1], U[cc][1], R[0] * U[r][0] * U[cc][0]));
+#pragma unroll
+        for (int r = 0; r < 3; ++r)
+#pragma unroll
+            for (int cc = 0; cc < 3; ++cc)
+                out.F[r][cc] = (float)fma(M[r][2], (double)in.F[2][cc],
+                                          fma(M[r][1], (double)in.F[1][cc], M[r][0] * in.F[0][cc]));
+    }
+#pragma unroll
+    for (int a = 0; a < 3; ++a) P_hat[a] *= S[a] * V0;
+#pragma unroll
+    for (int r = 0; r < 3; ++r)
+#pragma unroll
+        for (int cc = 0; cc <= r; ++cc)
+            out.sigma[r][cc] = out.sigma[cc][r] =
+                (float)fma(P_hat[2] * U[r][2], U[cc][2],
+                           fma(P_hat[1] * U[r][1], U[cc][1], P_hat[0] * U[r][0] * U[cc][0]));
+}
+
+// ALL64: principal axes and return mapping in FP64 for every particle.  Otherwise FP32,
 // redone in FP64 where the smallest singular-value gap is below svd_gap (the
 // directions of near-equal singular values are ill-conditioned in FP32).
 // Returns whether the FP64 redo ran.
@@ -264,13 +289,7 @@ template <bool ALL64>
 __device__ __forceinline__ bool stress_one(const DevParams& dp, const StressIn& in, StressOut& out) {
     out.alpha = in.alpha;
     if (ALL64) {
-        double Ad[3][3], Ud[3][3], Sd[3], Vd[3][3];
-#pragma unroll
-        for (int r = 0; r < 3; ++r)
-#pragma unroll
-            for (int cc = 0; cc < 3; ++cc) Ad[r][cc] = in.F[r][cc];
-        svd3<double>(Ad, Ud, Sd, Vd);
-        energy<double>(dp, in, out, Ud, Sd, Vd);
+        energy64(dp, in, out);
         return false;
     }
     float A[3][3], U[3][3], S[3], V[3][3];
@@ -389,38 +408,86 @@ __global__ __launch_bounds__(256) void k_stress(DevParams dp, ST s, WaveMap wm, 
     stress_write(s, i, n, sigma, FP, vol, dc, out);
 }
 
-// the state fields the stress leaves unchanged, moved from o of s to i of d
-// (every load before any store); v and B only with vb set: the G2P of the
-// substep writes both afresh without reading them, so a substep that runs it
-// leaves them out
+__device__ __forceinline__ uint32_t to_word(float f) { return __float_as_uint(f); }
+__device__ __forceinline__ uint32_t to_word(uint16_t h) { return h; }
+__device__ __forceinline__ void from_word(uint32_t w, float& f) { f = __uint_as_float(w); }
+__device__ __forceinline__ void from_word(uint32_t w, uint16_t& h) { h = (uint16_t)w; }
+// the state fields the stress leaves unchanged, in the storage form
 template <typename ST>
-__device__ __forceinline__ void carry_state(const ST& s, int o, const ST& d, int i, int n, bool vb) {
-    decltype(+s.x[0]) x[3];
-    decltype(+s.v[0]) v[3];
-    decltype(+s.B[0]) B[9];
+struct Carried {
+    std::remove_reference_t<decltype(*ST::x)> x[3];
+    std::remove_reference_t<decltype(*ST::v)> v[3];
+    std::remove_reference_t<decltype(*ST::B)> B[9];
+    std::remove_reference_t<decltype(*ST::c)> c;
+    float mass;
+    int id;
+};
+template <typename ST>
+__device__ __forceinline__ void carried_load(const ST& s, int o, int n, Carried<ST>& r) {
 #pragma unroll
-    for (int a = 0; a < 3; ++a) x[a] = s.x[3 * o + a];
-    if (vb) {
+    for (int a = 0; a < 3; ++a) r.x[a] = s.x[3 * o + a];
 #pragma unroll
-        for (int a = 0; a < 3; ++a) v[a] = s.v[3 * o + a];
+    for (int a = 0; a < 3; ++a) r.v[a] = s.v[3 * o + a];
 #pragma unroll
-        for (int a = 0; a < 9; ++a) B[a] = s.B[(int64_t)a * n + o];
-    }
-    const auto c = s.c[o];
-    const auto mass = s.mass[o];
-    const int id = s.id[o];
-#pragma unroll
-    for (int a = 0; a < 3; ++a) d.x[3 * i + a] = x[a];
-    if (vb) {
-#pragma unroll
-        for (int a = 0; a < 3; ++a) d.v[3 * i + a] = v[a];
-#pragma unroll
-        for (int a = 0; a < 9; ++a) d.B[(int64_t)a * n + i] = B[a];
-    }
-    d.c[i] = c;
-    d.mass[i] = mass;
-    d.id[i] = id;
+    for (int a = 0; a < 9; ++a) r.B[a] = s.B[(int64_t)a * n + o];
+    r.c = s.c[o];
+    r.mass = s.mass[o];
+    r.id = s.id[o];
 }
+// v and B only with vb set: the G2P of the substep writes both afresh without
+// reading them, so a substep that runs it leaves them out
+template <typename ST>
+__device__ __forceinline__ void carried_store(const Carried<ST>& r, const ST& d, int i, int n, bool vb) {
+#pragma unroll
+    for (int a = 0; a < 3; ++a) d.x[3 * i + a] = r.x[a];
+    if (vb) {
+#pragma unroll
+        for (int a = 0; a < 3; ++a) d.v[3 * i + a] = r.v[a];
+#pragma unroll
+        for (int a = 0; a < 9; ++a) d.B[(int64_t)a * n + i] = r.B[a];
+    }
+    d.c[i] = r.c;
+    d.mass[i] = r.mass;
+    d.id[i] = r.id;
+}
+// a wave's fields parked in LDS, a row of 64 words per field
+constexpr int kCarriedWords = 18;   // at most a payload record's
+template <typename ST>
+__device__ __forceinline__ void carried_park(const Carried<ST>& r, uint32_t* lds) {
+    const int lane = threadIdx.x & 63;
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+        lds[a * 64 + lane] = to_word(r.x[a]);
+        lds[(3 + a) * 64 + lane] = to_word(r.v[a]);
+    }
+#pragma unroll
+    for (int a = 0; a < 9; ++a) lds[(6 + a) * 64 + lane] = to_word(r.B[a]);
+    lds[15 * 64 + lane] = to_word(r.c);
+    lds[16 * 64 + lane] = to_word(r.mass);
+    lds[17 * 64 + lane] = (uint32_t)r.id;
+}
+template <typename ST>
+__device__ __forceinline__ void carried_fetch(const uint32_t* lds, Carried<ST>& r) {
+    const int lane = threadIdx.x & 63;
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+        from_word(lds[a * 64 + lane], r.x[a]);
+        from_word(lds[(3 + a) * 64 + lane], r.v[a]);
+    }
+#pragma unroll
+    for (int a = 0; a < 9; ++a) from_word(lds[(6 + a) * 64 + lane], r.B[a]);
+    from_word(lds[15 * 64 + lane], r.c);
+    from_word(lds[16 * 64 + lane], r.mass);
+    r.id = (int)lds[17 * 64 + lane];
+}
+// what the P2G terms read (ld_x and its like of access.h)
+__device__ __forceinline__ float as_float(float f) { return f; }
+__device__ __forceinline__ float as_float(uint16_t h) { return bf2f(h); }
+template <typename ST> __device__ __forceinline__ float ld_x(const Carried<ST>& r, int, int a) { return r.x[a]; }
+template <typename ST> __device__ __forceinline__ float ld_v(const Carried<ST>& r, int, int a) { return as_float(r.v[a]); }
+template <typename ST> __device__ __forceinline__ float ld_B(const Carried<ST>& r, int, int k, int) { return as_float(r.B[k]); }
+template <typename ST> __device__ __forceinline__ float ld_c(const Carried<ST>& r, int) { return as_float(r.c); }
+template <typename ST> __device__ __forceinline__ float ld_m(const Carried<ST>& r, int) { return r.mass; }
 
 // v and B in the new order, for a substep that stopped between its stress
 // pass (which left them out) and its G2P
@@ -461,22 +528,34 @@ hipError_t finish_carry_vb(mpmx_ctx* c) {
 // particle i reads its state at perm[i] of s and writes all of it to i of d
 // (the stand-alone gather's reads are the ones the stress makes anyway);
 // without, s and d are the same sorted state.
-// Three waves per SIMD (158 VGPRs): 138 us against 161 us at the two waves an
-// unconstrained allocation allows, 175 us at four (1M particles).
+// The FP64 update takes about 0.4 ms of VALU time on the 8M impact and the state
+// and payload (2.3 GB) 0.5 ms at the rate of a large copy, so it needs waves
+// and loads in flight: four waves per SIMD (128 VGPRs); every field is loaded
+// ahead of the update, and those it does not change wait in LDS; the payload
+// records leave through the same LDS, so that the wave writes whole lines
+// instead of 16 bytes of 64 lines per store.  8M impact (mixed) 825 -> 791 us with
+// the principal axes in place of the full SVD, 730 at four waves, 670 with whole
+// lines, 627 with the loads ahead; 256-scene batch 1,352 -> 1,295, 1,186, 1,108,
+// 1,007; 1M bar (FP32) 127 -> 119, 118, 107, 96.  Loads ahead kept in registers
+// spill at four waves (756 us on the impact) and take 664 at three.
 template <bool ALL64, int TRANSFER, typename ST>
-__global__ __launch_bounds__(256, 3) void k_stress_prep(DevParams dp, ST s, ST d, const uint32_t* __restrict__ perm,
+__global__ __launch_bounds__(256, 4) void k_stress_prep(DevParams dp, ST s, ST d, const uint32_t* __restrict__ perm,
                                                      int carry_vb, WaveMap wm, float* __restrict__ sigma,
                                                      float* __restrict__ FP, float* __restrict__ vol, BlockTables t,
                                                      float* __restrict__ pay, unsigned* __restrict__ pbound, float dt,
                                                      int n, const uint8_t* __restrict__ wclass,
                                                      int* __restrict__ order, DevCounts* dc) {
+    constexpr int kRec = Payload<TRANSFER>::kFloats / 4;
+    __shared__ float4 lds[kOrderClasses * 256 / 4];   // the order's counts, or the waves' payload records
+    __shared__ int olds[4];
+    static_assert(kCarriedWords <= 4 * kRec, "the fields wait where the record goes");
+    static_assert(kRec * 256 <= kOrderClasses * 256 / 4, "the records of 256 particles");
     dt = substep_dt(dt, dc);
     // the first workgroup orders the blocks for the block kernels that follow
     // (k_block_lists has just listed them); dispatched first, it runs beside
     // the stress waves instead of after them
     if ((int)blockIdx.x < kOrderGroups) {
-        __shared__ int ocnt[kOrderClasses * 256];
-        __shared__ int olds[4];
+        int* ocnt = reinterpret_cast<int*>(lds);
         int nb = dc->num_blocks;
         nb = nb < t.cap_blocks ? nb : (int)t.cap_blocks;
         order_blocks(wclass, order, nb, ocnt, olds);
@@ -488,24 +567,38 @@ __global__ __launch_bounds__(256, 3) void k_stress_prep(DevParams dp, ST s, ST d
 #pragma unroll
     for (int k = 0; k < kP2GCh; ++k) b[k] = 0.f;
     uint32_t pk = 0xffffffffu;
+    const int lane = threadIdx.x & 63;
+    float4* rec = lds + (threadIdx.x >> 6) * (64 * kRec);
     if (valid) {
         const DevParams& sp = dp.scenes[scene];
         const int o = perm ? (int)perm[i] : i;
+        Carried<ST> rest;
+        carried_load(s, o, n, rest);
+        carried_park(rest, reinterpret_cast<uint32_t*>(rec));
+        pk = t.keys[i] >> 6;
         StressOut out;
         stress_compute<ALL64>(sp, s, o, n, dc, out);
-        pk = t.keys[i] >> 6;
         float sig[9];
 #pragma unroll
         for (int r = 0; r < 3; ++r)
 #pragma unroll
             for (int cc = 0; cc < 3; ++cc) sig[r + 3 * cc] = out.sigma[r][cc];
-        // the payload reads x, m, c, v and B, none of which the stress
-        // changes: it goes first, so that its loads need not wait behind the
-        // stores of the updated state
-        prep_particle<TRANSFER>(sp, s, sig, out.FP, out.vol, o, i, n, dt, pay, b);
-        if (perm) carry_state(s, o, d, i, n, carry_vb != 0);
+        carried_fetch(reinterpret_cast<const uint32_t*>(rec), rest);
+        // every lane has its fields before any writes its record over them
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        prep_particle<TRANSFER>(sp, rest, sig, out.FP, out.vol, o, n, dt, rec + lane * kRec, b);
+        if (perm) carried_store(rest, d, i, n, carry_vb != 0);
         stress_write(d, i, n, sigma, FP, vol, dc, out);
     }
+    // the wave's records in whole lines
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    const int m = __popcll(__ballot(valid)) * kRec;
+    float4* out = reinterpret_cast<float4*>(pay) + (int64_t)(i - lane) * kRec;
+#pragma unroll
+    for (int k = 0; k < kRec; ++k)
+        if (lane + 64 * k < m) out[lane + 64 * k] = rec[lane + 64 * k];
     page_bounds(valid, pk, b, t, pbound, dc);
 }
 

@@ -85,9 +85,7 @@ __device__ __forceinline__ void p2g_bounds(const P2GTerms& T, float (&b)[kP2GCh]
 template <int TRANSFER> struct Payload { static constexpr int kFloats = TRANSFER ? 28 : 20; };
 
 template <int TRANSFER>
-__device__ __forceinline__ void payload_store(float* __restrict__ pay, int64_t i, const float (&d0)[3],
-                                              const P2GTerms& T) {
-    float4* q = reinterpret_cast<float4*>(pay + i * Payload<TRANSFER>::kFloats);
+__device__ __forceinline__ void payload_store(float4* q, const float (&d0)[3], const P2GTerms& T) {
     q[0] = make_float4(d0[0], d0[1], d0[2], T.m);
     q[1] = make_float4(T.ar[0], T.ar[1], T.ar[2], T.cphase);
     q[2] = make_float4(T.Qd[0], T.Qd[1], T.Qd[2], T.Qd[3]);
@@ -137,17 +135,16 @@ __device__ __forceinline__ void payload_load(const float* __restrict__ pay, int6
     T.l0[2] = 4 * pz + (cell & 3) - org[2];
 }
 
-// payload record i of the particle whose state sits at o of s, and its
+// payload record rec of the particle whose state sits at o of s, and its
 // per-channel bounds b
 template <int TRANSFER, typename ST>
 __device__ __forceinline__ void prep_particle(const DevParams& dp, const ST& s, const float (&sig)[9], float FPv,
-                                              float V, int o, int i, int n, float dt, float* __restrict__ pay,
-                                              float (&b)[kP2GCh]) {
+                                              float V, int o, int n, float dt, float4* rec, float (&b)[kP2GCh]) {
     const int org[3] = {0, 0, 0};
     P2GTerms T;
     float d0[3];
     p2g_terms<TRANSFER>(dp, s, sig, FPv, V, o, n, dt, org, d0, T);
-    payload_store<TRANSFER>(pay, i, d0, T);
+    payload_store<TRANSFER>(rec, d0, T);
     p2g_bounds<TRANSFER>(T, b);
 }
 

@@ -10,9 +10,9 @@
 // Written for registers: matrices are plain T[3][3] arrays fully unrolled by
 // the compiler; a Givens rotation is (i, k, c, s).  The sweep loop is bounded
 // (kMaxSweeps) so that a non-converging input can never stall a wavefront; the
-// reference loop is unbounded.  Templated on float and double (the stress
-// update runs it in FP64 by default: FP64 is half the FP32 rate on CDNA4 and
-// the update is bound by particle-state traffic).
+// reference loop is unbounded.  Templated on float and double.  It serves the FP32
+// stress arithmetic and its FP64 redo; the default FP64 update takes the principal
+// axes below.
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -266,6 +266,156 @@ __device__ __forceinline__ int svd3(const T (&A)[3][3], T (&U)[3][3], T (&S)[3],
         order1(U, S, V);
     }
     return sweeps;
+}
+
+// ---- principal axes in FP64 ----------------------------------------------------
+// The isotropic updates need the left singular vectors and the singular values
+// only: functions of them act on F as sum_a f_a u_a u_a^T F, so V is never formed.
+// One-sided Jacobi: rotations from the right make the columns of G = F V
+// orthogonal; then |g_a| = |S_a| and u_a = g_a / |S_a|.  It works on F itself (a
+// product F F^T would square the condition number), needs two reciprocal square
+// roots and 27 multiply-adds per rotation, no division, and keeps nine doubles,
+// where the QR iteration above keeps B, U and V.  A pair of columns counts as
+// orthogonal below 2^-50 of their lengths' product.
+constexpr int kMaxJacobi = 32;
+
+__device__ __forceinline__ void jacobi_columns(double (&G)[3][3]) {
+    constexpr double tol2 = 0x1p-100;
+    for (int sweep = 0; sweep < kMaxJacobi; ++sweep) {
+        bool turned = false;
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            const int p = k == 2 ? 1 : 0, q = k == 0 ? 1 : 2;
+            const double a = fma(G[2][p], G[2][p], fma(G[1][p], G[1][p], G[0][p] * G[0][p]));
+            const double b = fma(G[2][q], G[2][q], fma(G[1][q], G[1][q], G[0][q] * G[0][q]));
+            const double c = fma(G[2][p], G[2][q], fma(G[1][p], G[1][q], G[0][p] * G[0][q]));
+            if (c * c > tol2 * (a * b)) {
+                // tan 2t = 2c / (b - a); cos t >= sqrt(1/2)
+                const double d = b - a, r = rsqrt_acc(fma(d, d, 4.0 * (c * c)));
+                const double h = fma(0.5 * fabs(d), r, 0.5), rh = rsqrt_acc(h);
+                const double cs = h * rh, sn = copysign(1.0, d) * (c * r) * rh;
+#pragma unroll
+                for (int i = 0; i < 3; ++i) {
+                    const double x = G[i][p], y = G[i][q];
+                    G[i][p] = fma(cs, x, -sn * y);
+                    G[i][q] = fma(sn, x, cs * y);
+                }
+                turned = true;
+            }
+        }
+        if (!turned) break;
+    }
+}
+
+// F = sum_a S_a u_a v_a^T, u_a the columns of U, R_a = 1 / S_a; no order, at most
+// one S_a < 0 (the smallest, where det F < 0).  False where the smallest is below
+// 1e-5 of the largest: there u_a is not to be had from g_a, nor v_a from u_a^T F.
+__device__ __forceinline__ bool principal_axes(const float (&F)[3][3], double (&U)[3][3], double (&S)[3],
+                                               double (&R)[3]) {
+#pragma unroll
+    for (int r = 0; r < 3; ++r)
+#pragma unroll
+        for (int c = 0; c < 3; ++c) U[r][c] = F[r][c];
+    jacobi_columns(U);
+    const double det = U[0][0] * (U[1][1] * U[2][2] - U[1][2] * U[2][1]) -
+                       U[0][1] * (U[1][0] * U[2][2] - U[1][2] * U[2][0]) +
+                       U[0][2] * (U[1][0] * U[2][1] - U[1][1] * U[2][0]);
+    double n2[3];
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+        n2[a] = fma(U[2][a], U[2][a], fma(U[1][a], U[1][a], U[0][a] * U[0][a]));
+        R[a] = n2[a] > 0.0 ? rsqrt_acc(n2[a]) : 0.0;
+        S[a] = n2[a] * R[a];
+#pragma unroll
+        for (int r = 0; r < 3; ++r) U[r][a] *= R[a];
+    }
+    const double lo = fmin(n2[0], fmin(n2[1], n2[2])), hi = fmax(n2[0], fmax(n2[1], n2[2]));
+    if (det < 0.0) {
+        const int m = n2[0] == lo ? 0 : (n2[1] == lo ? 1 : 2);
+#pragma unroll
+        for (int a = 0; a < 3; ++a)
+            if (a == m) {
+                S[a] = -S[a];
+                R[a] = -R[a];
+            }
+    }
+    return lo > 1e-10 * hi;
+}
+
+// a unit vector across u
+__device__ __forceinline__ void across(const double (&u)[3], double (&v)[3]) {
+    const bool x = fabs(u[0]) < 0.6;
+    const double d = x ? u[0] : u[1];
+    double n = 0.0;
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+        v[i] = (i == (x ? 0 : 1) ? 1.0 : 0.0) - d * u[i];
+        n = fma(v[i], v[i], n);
+    }
+    n = rsqrt_acc(n);
+#pragma unroll
+    for (int i = 0; i < 3; ++i) v[i] *= n;
+}
+
+__device__ __forceinline__ double pick(const double (&x)[3], int i) { return i == 0 ? x[0] : (i == 1 ? x[1] : x[2]); }
+
+// where principal_axes returned false: the smallest singular value's directions,
+// u and v alike, completed to right-handed bases from the other two (of a lower
+// rank: any vectors across).  R as principal_axes left it (0 for S = 0); i is the
+// smallest, (i, j, k) cyclic.
+__device__ __forceinline__ void principal_axes_singular(const float (&F)[3][3], const double (&R)[3],
+                                                        double (&U)[3][3], double (&V)[3][3]) {
+    double S[3];
+#pragma unroll
+    for (int a = 0; a < 3; ++a) S[a] = R[a] != 0.0 ? 1.0 / fabs(R[a]) : 0.0;
+    const int i = S[0] <= S[1] && S[0] <= S[2] ? 0 : (S[1] <= S[2] ? 1 : 2), j = i == 2 ? 0 : i + 1,
+              k = j == 2 ? 0 : j + 1;
+    const double sj = pick(S, j), sk = pick(S, k);
+    double uj[3], uk[3], vj[3], vk[3], ui[3], vi[3];
+    double nj = 0.0, nk = 0.0;
+#pragma unroll
+    for (int r = 0; r < 3; ++r) {
+        uj[r] = pick(U[r], j);
+        uk[r] = pick(U[r], k);
+    }
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+        vj[c] = F[0][c] * uj[0] + F[1][c] * uj[1] + F[2][c] * uj[2];
+        vk[c] = F[0][c] * uk[0] + F[1][c] * uk[1] + F[2][c] * uk[2];
+        nj += vj[c] * vj[c];
+        nk += vk[c] * vk[c];
+    }
+    nj = rsqrt_acc(nj);
+    nk = rsqrt_acc(nk);
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+        vj[c] *= nj;
+        vk[c] *= nk;
+    }
+    if (!(sj > 0.0 || sk > 0.0)) {
+        uj[0] = vj[0] = 1.0;
+        uj[1] = uj[2] = vj[1] = vj[2] = 0.0;
+    }
+    if (!(sk > 0.0)) {
+        across(uj, uk);
+        across(vj, vk);
+    } else if (!(sj > 0.0)) {
+        across(uk, uj);
+        across(vk, vj);
+    }
+    ui[0] = uj[1] * uk[2] - uj[2] * uk[1];
+    ui[1] = uj[2] * uk[0] - uj[0] * uk[2];
+    ui[2] = uj[0] * uk[1] - uj[1] * uk[0];
+    vi[0] = vj[1] * vk[2] - vj[2] * vk[1];
+    vi[1] = vj[2] * vk[0] - vj[0] * vk[2];
+    vi[2] = vj[0] * vk[1] - vj[1] * vk[0];
+#pragma unroll
+    for (int a = 0; a < 3; ++a)
+#pragma unroll
+        for (int r = 0; r < 3; ++r) {
+            U[r][a] = a == i ? ui[r] : (a == j ? uj[r] : uk[r]);
+            V[r][a] = a == i ? vi[r] : (a == j ? vj[r] : vk[r]);
+        }
 }
 
 }  // namespace mpmx
