@@ -513,7 +513,7 @@ __global__ __launch_bounds__(256) void k_cg_dot(DevParams dp, const float* __res
                                                 const DevCounts* __restrict__ dc) {
     __shared__ float lds[4];
     const SceneBlocks sb = scene_blocks(scg, wg_scene);
-    if (scene_stopped(scg, sb.scene)) return;
+    if ((int)blockIdx.x - sb.wg0 >= sb.nwg || scene_stopped(scg, sb.scene)) return;
     const int num_page = dc->num_page;
     const bool maxdot = dp.dot_mode == 0;
     float wacc = maxdot ? -INFINITY : 0.f, racc = wacc;
@@ -564,7 +564,7 @@ __global__ __launch_bounds__(256) void k_cg_update(DevParams dp, const float* __
                                                    const DevCounts* __restrict__ dc) {
     __shared__ float lds[4];
     const SceneBlocks sb = scene_blocks(scg, wg_scene);
-    if (scene_stopped(scg, sb.scene)) return;
+    if ((int)blockIdx.x - sb.wg0 >= sb.nwg || scene_stopped(scg, sb.scene)) return;
     const float sq = reduce_dot(dp, part + sb.wg0, sb.nwg, lds);
     const float rho_old = reduce_dot(dp, part + (1 + (k & 1)) * nb + sb.wg0, sb.nwg, lds);
     const float alpha = rho_old / sq;
@@ -622,7 +622,7 @@ __global__ __launch_bounds__(256) void k_cg_direction(DevParams dp, const float*
                                                       const uint64_t* __restrict__ amask, DevCounts* dc) {
     __shared__ float lds[4];
     const SceneBlocks sb = scene_blocks(scg, wg_scene);
-    if (scene_stopped(scg, sb.scene)) return;
+    if ((int)blockIdx.x - sb.wg0 >= sb.nwg || scene_stopped(scg, sb.scene)) return;
     const float norm = reduce_parts<true>(part + 3 * nb + sb.wg0, sb.nwg, lds);
     const float rho_old = reduce_dot(dp, part + (1 + (k & 1)) * nb + sb.wg0, sb.nwg, lds);
     const float rho = reduce_dot(dp, part + (1 + ((k + 1) & 1)) * nb + sb.wg0, sb.nwg, lds);
@@ -774,11 +774,13 @@ __global__ void k_publish_counts(const DevCounts* __restrict__ dc, DevCounts* pu
     if (lane == 0) __hip_atomic_store(&pub->seq, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
-hipError_t counts_to_host(mpmx_ctx* c) {
-    const unsigned want = ++c->pub_seq;
-    k_publish_counts<<<1, 64, 0, c->stream>>>(c->dc, c->pub, want);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
+hipError_t publish_counts(mpmx_ctx* c) {
+    k_publish_counts<<<1, 64, 0, c->stream>>>(c->dc, c->pub, ++c->pub_seq);
+    return hipGetLastError();
+}
+hipError_t await_counts(mpmx_ctx* c) {
+    const unsigned want = c->pub_seq;
+    hipError_t e;
     // the copy lands when every earlier kernel of the stream has finished;
     // past two seconds (a stalled stream, or a launch that failed late) the
     // stream synchronisation below reports what happened
@@ -797,6 +799,10 @@ hipError_t counts_to_host(mpmx_ctx* c) {
     }
     std::memcpy(c->hc, c->pub, sizeof(DevCounts));
     return hipSuccess;
+}
+hipError_t counts_to_host(mpmx_ctx* c) {
+    const hipError_t e = publish_counts(c);
+    return e == hipSuccess ? await_counts(c) : e;
 }
 
 }  // namespace mpmx

@@ -300,14 +300,19 @@ __global__ __launch_bounds__(BLOCK) void k_g2p(DevParams dp, ST s, Tables t, con
 // consecutive Morton codes).  The block's grid pages and particle range come
 // with the page tables (BlockG2P).  Pages where the blocks are few
 // (tiles_are_pages): 64,000 cube 48 -> 13 us, 333,333 sphere 74 -> 31.
+// With if_solved set the kernel does nothing while the solve goes on: it is
+// queued behind the iterations the last substep needed, before the host knows
+// whether they were enough.
 template <int E, int TRANSFER, typename ST>
 __global__ __launch_bounds__(256) void k_g2p_block(DevParams dp, ST s, BlockTables t,
                                                    const BlockClasses* __restrict__ lists,
                                                    const BlockG2P* __restrict__ info, const float* __restrict__ grid,
                                                    const float* __restrict__ cgx, uint32_t* __restrict__ keys,
-                                                   float dt, int n, const SceneCG* __restrict__ scg, DevCounts* dc) {
+                                                   float dt, int n, int if_solved,
+                                                   const SceneCG* __restrict__ scg, DevCounts* dc) {
     constexpr int R = E + 2, R3 = R * R * R;
     __shared__ float tv[4 * R3];
+    if (if_solved && !dc->cg_done) return;   // uniform over the grid
     dt = substep_dt(dt, dc);
     int nb = dc->num_blocks;
     nb = nb < t.cap_blocks ? nb : (int)t.cap_blocks;
@@ -455,36 +460,37 @@ static void g2p_block(mpmx_ctx* c, ST st, float dt) {
 }
 
 template <int E, int TRANSFER, typename ST>
-static void g2p_block_launch(mpmx_ctx* c, ST st, float dt) {
+static void g2p_block_launch(mpmx_ctx* c, ST st, float dt, bool if_solved) {
     // the blocks in the gathers' order (by gather entries; a block's own
     // particles, the G2P's work, go with them): 0.34 -> 0.29 ms on the 8M
     // impact against block order
     const int g = block_grid(c, c->g2p_pct) * (E == 8 ? 1 : 8);
     k_g2p_block<E, TRANSFER, ST><<<g, 256, 0, c->stream>>>(
         c->dp, st, block_tables_of(c), static_cast<const BlockClasses*>(c->block_lists),
-        static_cast<const BlockG2P*>(c->block_g2p), c->grid, c->cg_x, c->keys_next, dt, (int)c->n, c->scg, c->dc);
+        static_cast<const BlockG2P*>(c->block_g2p), c->grid, c->cg_x, c->keys_next, dt, (int)c->n,
+        if_solved ? 1 : 0, c->scg, c->dc);
 }
 template <typename ST>
-static void g2p_block_kernel(mpmx_ctx* c, ST st, float dt) {
+static void g2p_block_kernel(mpmx_ctx* c, ST st, float dt, bool if_solved) {
     MPMX_TIMED(c, "g2p_block", ({
                    if (tiles_are_pages(c, 400)) {
-                       if (c->P.transfer == 0) g2p_block_launch<4, 0>(c, st, dt);
-                       else g2p_block_launch<4, 1>(c, st, dt);
+                       if (c->P.transfer == 0) g2p_block_launch<4, 0>(c, st, dt, if_solved);
+                       else g2p_block_launch<4, 1>(c, st, dt, if_solved);
                    } else {
-                       if (c->P.transfer == 0) g2p_block_launch<8, 0>(c, st, dt);
-                       else g2p_block_launch<8, 1>(c, st, dt);
+                       if (c->P.transfer == 0) g2p_block_launch<8, 0>(c, st, dt, if_solved);
+                       else g2p_block_launch<8, 1>(c, st, dt, if_solved);
                    }
                }));
 }
 
-hipError_t launch_g2p(mpmx_ctx* c, float dt) {
+hipError_t launch_g2p(mpmx_ctx* c, float dt, bool if_solved) {
     c->vb_perm = nullptr;   // the G2P writes v and B of every particle
     if (c->cfg.p2g_variant == 1) {
         if (c->cfg.precision != MPMX_FP32) g2p_block(c, c->ms[c->cur], dt);
         else g2p_block(c, c->ps[c->cur], dt);
     } else {
-        if (c->cfg.precision != MPMX_FP32) g2p_block_kernel(c, c->ms[c->cur], dt);
-        else g2p_block_kernel(c, c->ps[c->cur], dt);
+        if (c->cfg.precision != MPMX_FP32) g2p_block_kernel(c, c->ms[c->cur], dt, if_solved);
+        else g2p_block_kernel(c, c->ps[c->cur], dt, if_solved);
     }
     return hipGetLastError();
 }

@@ -571,6 +571,9 @@ __device__ __forceinline__ SceneBlocks scene_blocks(const SceneCG* __restrict__ 
     b.nn = g.nn;
     b.nblk = (g.np + g.nn + 1) / 2;
     const int wpb = (int)(blockDim.x >> 6);
+    // workgroups past the scene's blocks have no part: their partials are not read
+    const int need = (b.nblk + wpb - 1) / wpb;
+    b.nwg = b.nwg < need ? b.nwg : (need > 0 ? need : 1);
     b.wave = (int)(blockIdx.x - b.wg0) * wpb + (int)(threadIdx.x >> 6);
     b.nwaves = b.nwg * wpb;
     return b;
@@ -616,13 +619,16 @@ hipError_t launch_stress_p2g(mpmx_ctx* c, float dt);
 hipError_t launch_block_lists(mpmx_ctx* c);
 // the device counters into c->hc once the work queued so far has finished:
 // a one-wave kernel copies them into coherent host memory, the host waits
-// for its sequence number (no stream synchronisation)
+// for its sequence number (no stream synchronisation); in two halves, so that
+// work can be queued before the wait
 hipError_t counts_to_host(mpmx_ctx* c);
+hipError_t publish_counts(mpmx_ctx* c);
+hipError_t await_counts(mpmx_ctx* c);
 hipError_t launch_grid_update(mpmx_ctx* c, float dt);
 hipError_t launch_pcg(mpmx_ctx* c, float dt);
 hipError_t launch_pcg_from(mpmx_ctx* c, int it0, int first_chunk);
 hipError_t queue_pcg_iterations(mpmx_ctx* c, int k0, int k1);
-hipError_t launch_g2p(mpmx_ctx* c, float dt);
+hipError_t launch_g2p(mpmx_ctx* c, float dt, bool if_solved = false);
 hipError_t launch_cg_reset(mpmx_ctx* c);
 hipError_t fill_zero(mpmx_ctx* c, void* p, int64_t bytes);
 hipError_t fill_zero_dev_count(mpmx_ctx* c, float* p, const int* count_dev, int64_t per_unit,
