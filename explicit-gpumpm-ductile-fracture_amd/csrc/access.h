@@ -433,27 +433,27 @@ template <int E> constexpr TileOrder<E> tile_order() {
 }
 template <int E> __device__ __constant__ const TileOrder<E> kTileOrder = tile_order<E>();
 
-constexpr int kTileThreads = 256;   // per workgroup
+constexpr int kTileThreads = 256;   // per workgroup of a block tile
 
 // the tile's cells that hold particles, in that order, and the pairs of
 // particles they make (the last pair of an odd cell is a single)
-template <int E> struct TileCells {
+template <int E, int NT> struct TileCells {   // NT threads
     static constexpr int kCells = TileOrder<E>::kCells;
-    static constexpr int kPer = (kCells + kTileThreads - 1) / kTileThreads;
+    static constexpr int kPer = (kCells + NT - 1) / NT;
     int start[kCells];       // first particle
     int pairs[kCells + 1];   // pairs before the cell
     uint16_t place[kCells];  // TileOrder; bit 12: an odd number of particles
     int page[27];            // particle pages 2b - 1 .. 2b + 1 of the block, by place
-    int wsum[2][kTileThreads / 64];
+    int wsum[2][NT / 64];
     int cells;
 };
 
 // Builds S for the tile at o3 (nodes) of the block with lists L; called and
 // left by the whole workgroup (a barrier at its end)
-template <int E>
+template <int E, int NT>
 __device__ __forceinline__ void tile_cells(const BlockClasses* __restrict__ L, const int* __restrict__ cell_start,
-                                           int n, const int (&o3)[3], TileCells<E>& S) {
-    constexpr int kPer = TileCells<E>::kPer, kCells = TileCells<E>::kCells;
+                                           int n, const int (&o3)[3], TileCells<E, NT>& S) {
+    constexpr int kPer = TileCells<E, NT>::kPer, kCells = TileCells<E, NT>::kCells;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     if (tid < 27) {
         int cls, d[3];
@@ -489,7 +489,7 @@ __device__ __forceinline__ void tile_cells(const BlockClasses* __restrict__ L, c
     __syncthreads();
     int p = ip - pairs, c = ic - cells, tp = 0, tc = 0;
 #pragma unroll
-    for (int q = 0; q < kTileThreads / 64; ++q) {
+    for (int q = 0; q < NT / 64; ++q) {
         p += q < wave ? S.wsum[0][q] : 0;
         c += q < wave ? S.wsum[1][q] : 0;
         tp += S.wsum[0][q];
@@ -511,8 +511,8 @@ __device__ __forceinline__ void tile_cells(const BlockClasses* __restrict__ L, c
     __syncthreads();
 }
 // cell of pair e (0 <= e < S.pairs[S.cells]): the last that starts at or before e
-template <int E>
-__device__ __forceinline__ int tile_find(const TileCells<E>& S, int e) {
+template <typename Cells>
+__device__ __forceinline__ int tile_find(const Cells& S, int e) {
     int lo = 0, hi = S.cells - 1;
     while (lo < hi) {
         const int mid = (lo + hi + 1) >> 1;
@@ -520,6 +520,44 @@ __device__ __forceinline__ int tile_find(const TileCells<E>& S, int e) {
         else hi = mid - 1;
     }
     return lo;
+}
+// the same for a whole wave, pair b + lane per lane (b < S.pairs[S.cells]), r0
+// the cell of pair b: the cells that start inside the wave's 64 pairs mark the
+// lanes of their first pairs (a lane of a pair past the last gets the last cell)
+template <typename Cells>
+__device__ __forceinline__ int tile_find_wave(const Cells& S, int cells, int r0, int b) {
+    const int lane = threadIdx.x & 63, c = r0 + lane;
+    const int at = c < cells ? S.pairs[c] - b : 64;
+    const int mark = __builtin_amdgcn_ds_permute(4 * (at > 0 && at < 64 ? at : 0), 1);   // lane 0 is marked anyway
+    const uint64_t m = __ballot(mark != 0) & ~1ull;
+    return r0 + __popcll(m & (~0ull >> (63 - lane)));
+}
+// A tile's pairs in groups of 64, a pair per lane, the wave's next group from a
+// counter in LDS (zero before): the cells come with the most nodes first, so the
+// waves, which would take from 27 nodes a pair to one in fixed shares, end
+// together.  f(pair's first particle, whether it has a second, place, number of
+// the pair in its cell).
+template <typename Cells, typename F>
+__device__ __forceinline__ void tile_pairs(const Cells& S, int* next, F f) {
+    const int lane = threadIdx.x & 63, cells = S.cells, pairs = S.pairs[cells];
+    for (;;) {
+        int g = 0;
+        if (lane == 0) g = atomicAdd(next, 1);
+        const int b = 64 * __builtin_amdgcn_readfirstlane(g), q = b + lane;
+        if (b >= pairs) break;
+        const int r = tile_find_wave(S, cells, tile_find(S, b), b);
+        if (q < pairs) {
+            const int j = q - S.pairs[r], place = S.place[r];
+            f(S.start[r] + 2 * j, !(place >> 12) || q + 1 < S.pairs[r + 1], place, j);
+        }
+    }
+}
+// the nodes of one axis turned by s places (0 .. 2)
+__device__ __forceinline__ void turn_nodes(float (&w)[3], int s) {
+    const float a = w[0], b = w[1], c = w[2];
+    w[0] = s == 0 ? a : (s == 1 ? b : c);
+    w[1] = s == 0 ? b : (s == 1 ? c : a);
+    w[2] = s == 0 ? c : (s == 1 ? a : b);
 }
 // the nodes of one axis moved down by s places (0 .. 2)
 __device__ __forceinline__ void drop_nodes(float (&w)[3], int s) {

@@ -264,14 +264,14 @@ __global__ __launch_bounds__(256) void k_p2g_prep(DevParams dp, ST s, WaveMap wm
 // pairs and the odd cells' last particles in two passes (405, 1,105 us), tiles
 // taken in turn by resident workgroups with the next tile's cells loaded ahead
 // (467, 1,170 us).
-template <int E, int TRANSFER>
-__global__ __launch_bounds__(kTileThreads, TRANSFER == 0 ? 4 : 3) void k_p2g_tile(
+template <int E, int TRANSFER, int NT>
+__global__ __launch_bounds__(NT, TRANSFER == 0 ? 4 : 3) void k_p2g_tile(
     DevParams dp, const float* __restrict__ pay, const unsigned* __restrict__ pbound, BlockTables t,
     const BlockClasses* __restrict__ lists, float* __restrict__ grid, float* __restrict__ grid_raw, CGVec cg, float dt,
     int n, const DevCounts* __restrict__ dc) {
     using A = TileAcc<E>;
     __shared__ unsigned long long acc[kP2GCh * A::kStride];
-    __shared__ TileCells<E> S;
+    __shared__ TileCells<E, NT> S;
     __shared__ int sexp[kP2GCh];
     dt = substep_dt(dt, dc);
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -285,7 +285,7 @@ __global__ __launch_bounds__(kTileThreads, TRANSFER == 0 ? 4 : 3) void k_p2g_til
         const BlockClasses* L = lists + blk;
         if (E == 4 && L->out_page[child] < 0) continue;   // uniform over the workgroup
         const int o3[3] = {4 * ((child >> 2) & 1), 4 * ((child >> 1) & 1), 4 * (child & 1)};
-        for (int q = tid; q < kP2GCh * A::kStride; q += kTileThreads) acc[q] = 0ull;
+        for (int q = tid; q < kP2GCh * A::kStride; q += NT) acc[q] = 0ull;
         // scales: the largest contribution per channel of the block's 27 source pages
         if (wave == 1) {
             const int pg = lane < 27 ? L->page[lane] : -1;
@@ -304,7 +304,7 @@ __global__ __launch_bounds__(kTileThreads, TRANSFER == 0 ? 4 : 3) void k_p2g_til
             }
             if (lane < kP2GCh) sexp[lane] = fix_exp(v);
         }
-        tile_cells<E>(L, t.cell_start, n, o3, S);   // ends in a barrier
+        tile_cells(L, t.cell_start, n, o3, S);   // ends in a barrier
         float sc[kP2GCh];
 #pragma unroll
         for (int k = 0; k < kP2GCh; ++k) sc[k] = ldexpf(1.0f, sexp[k]);
@@ -312,9 +312,9 @@ __global__ __launch_bounds__(kTileThreads, TRANSFER == 0 ? 4 : 3) void k_p2g_til
         // wave add to different nodes
         const int cells = S.cells, pairs = S.pairs[cells];
         if (pairs > 0) {
-            const int all = (pairs + kTileThreads - 1) / kTileThreads, one = (pairs + cells - 1) / cells;
+            const int all = (pairs + NT - 1) / NT, one = (pairs + cells - 1) / cells;
             const int P = all < one ? all : one;
-            for (int c0 = tid * P; c0 < pairs; c0 += kTileThreads * P) {
+            for (int c0 = tid * P; c0 < pairs; c0 += NT * P) {
                 const int ce = c0 + P < pairs ? c0 + P : pairs;
                 int r = tile_find(S, c0);
                 for (int e = c0; e < ce; ++e) {
@@ -332,7 +332,7 @@ __global__ __launch_bounds__(kTileThreads, TRANSFER == 0 ? 4 : 3) void k_p2g_til
         unmorton(bkey, bc[0], bc[1], bc[2]);
         const int org[3] = {8 * bc[0], 8 * bc[1], 8 * bc[2]};
         const DevParams sp = dp.scenes[__builtin_amdgcn_readfirstlane(scene_of_page(dp, bkey << 3))];
-        for (int q = tid; q < E * E * E; q += kTileThreads) {
+        for (int q = tid; q < E * E * E; q += NT) {
             const int o = E == 8 ? q >> 6 : child, cell = q & 63;
             const int G = L->out_page[o];
             if (G < 0) continue;
@@ -798,12 +798,16 @@ static hipError_t gather_blocks_t(mpmx_ctx* c, float dt) {
         return hipGetLastError();
     }
     const BlockClasses* lists = static_cast<BlockClasses*>(c->block_lists);
-    if (tiles_are_pages(c, 150))
-        MPMX_TIMED(c, "p2g_block", (k_p2g_tile<4, TRANSFER><<<8 * g, kTileThreads, 0, c->stream>>>(
+    if (tiles_are_pages(c, 150) && pages_are_few(c))
+        MPMX_TIMED(c, "p2g_block", (k_p2g_tile<4, TRANSFER, 512><<<8 * g, 512, 0, c->stream>>>(
+                                        c->dp, c->payload, c->pbound, t, lists, c->grid, raw, cg_vec(c), dt, (int)c->n,
+                                        c->dc)));
+    else if (tiles_are_pages(c, 150))
+        MPMX_TIMED(c, "p2g_block", (k_p2g_tile<4, TRANSFER, kTileThreads><<<8 * g, kTileThreads, 0, c->stream>>>(
                                         c->dp, c->payload, c->pbound, t, lists, c->grid, raw, cg_vec(c), dt, (int)c->n,
                                         c->dc)));
     else
-        MPMX_TIMED(c, "p2g_block", (k_p2g_tile<8, TRANSFER><<<g, kTileThreads, 0, c->stream>>>(
+        MPMX_TIMED(c, "p2g_block", (k_p2g_tile<8, TRANSFER, kTileThreads><<<g, kTileThreads, 0, c->stream>>>(
                                         c->dp, c->payload, c->pbound, t, lists, c->grid, raw, cg_vec(c), dt, (int)c->n,
                                         c->dc)));
     // the PCG's starting "dot"(r, z) comes with its first "dot"(s, q) (k_cg_dot)

@@ -273,19 +273,26 @@ __device__ __forceinline__ void cgq_entry(const DevParams& sp, const float (&xp)
 }
 
 // two particles of one cell at `place` of a page tile (i and, with two set, i +
-// 1) into the tile's sums, with the arithmetic of cgq_entry
+// 1) into the tile's sums, with the arithmetic of cgq_entry; org: the tile's first
+// node in scene-local cells.  The pairs of a cell, in neighbouring lanes, start at
+// different nodes of a row (turn by the pair's number j), so that they do not add
+// to one address at once.
 template <typename ST>
-__device__ __forceinline__ void cgq_pair(const DevParams& sp, const ST& s, int i, bool two, int place,
-                                         const float* __restrict__ col, float sc, unsigned long long* acc) {
+__device__ __forceinline__ void cgq_pair(const DevParams& sp, const ST& s, int i, bool two, int place, int j,
+                                         const int (&org)[3], const float* __restrict__ col, float sc,
+                                         unsigned long long* acc) {
     using A = TileAcc<4>;
     float w[2][3][3], gw[2][3][3], cs[2][3];
+    int l[3];   // cell in the tile, -2 .. 3
+#pragma unroll
+    for (int a = 0; a < 3; ++a) l[a] = ((place >> (8 - 4 * a)) & 15) - 2;
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
         const int k = two ? i + h : i;
 #pragma unroll
         for (int a = 0; a < 3; ++a) {
-            const float xa = ld_x(s, k, a);
-            const float d0 = xa * sp.inv_dx - (float)base_node(xa, sp.N);
+            // the particle is listed by its cell, so this is its base node
+            const float d0 = ld_x(s, k, a) * sp.inv_dx - (float)(org[a] + l[a]);
             bspline_grad(d0, w[h][a], gw[h][a]);
             cs[h][a] = h == 0 || two ? col[3 * (int64_t)k + a] * sc : 0.f;
         }
@@ -293,16 +300,24 @@ __device__ __forceinline__ void cgq_pair(const DevParams& sp, const ST& s, int i
     int cnt[3], node = 0;
 #pragma unroll
     for (int a = 0; a < 3; ++a) {
-        const int l = ((place >> (8 - 4 * a)) & 15) - 2;   // cell in the tile, -2 .. 3
-        const int f = l < 0 ? 0 : l;
-        cnt[a] = (l + 3 < 4 ? l + 3 : 4) - f;
+        const int f = l[a] < 0 ? 0 : l[a];
+        cnt[a] = (l[a] + 3 < 4 ? l[a] + 3 : 4) - f;
         node += f * (a == 0 ? A::kX : (a == 1 ? A::kZ : 1));
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
-            drop_nodes(w[h][a], f - l);
-            drop_nodes(gw[h][a], f - l);
+            drop_nodes(w[h][a], f - l[a]);
+            drop_nodes(gw[h][a], f - l[a]);
         }
     }
+    const int turn = cnt[2] == 3 ? (int)((unsigned)j % 3u) : 0;
+    unsigned long long* az[3];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        turn_nodes(w[h][2], turn);
+        turn_nodes(gw[h][2], turn);
+    }
+#pragma unroll
+    for (int k = 0; k < 3; ++k) az[k] = acc + node + (k + turn < 3 ? k + turn : k + turn - 3);
 #pragma unroll
     for (int ii = 0; ii < 3; ++ii) {
         if (ii >= cnt[0]) break;
@@ -321,7 +336,7 @@ __device__ __forceinline__ void cgq_pair(const DevParams& sp, const ST& s, int i
                 int add = 0;
 #pragma unroll
                 for (int h = 0; h < 2; ++h) add += (int)fmaf(w[h][2][kk], rA[h], gw[h][2][kk] * rB[h]);
-                atomicAdd(&acc[node + ii * A::kX + jj * A::kZ + kk], (unsigned long long)(long long)add);
+                atomicAdd(az[kk] + (ii * A::kX + jj * A::kZ), (unsigned long long)(long long)add);
             }
         }
     }
@@ -427,19 +442,23 @@ __global__ __launch_bounds__(256) void k_cg_q(DevParams dp, ST s, BlockTables t,
 // of a cell per atomic (|grad w . col| <= 0.75^2 |col|_1, so two terms of at
 // most 2^30 times that add up in 32 bits).  The scale is the block's, so the
 // sums are k_cg_q's bit for bit.  64,000 cube 74 -> 16 us, 333,333 sphere
-// 60 -> 30.
-template <typename ST>
-__global__ __launch_bounds__(kTileThreads) void k_cg_q_page(DevParams dp, ST s, BlockTables t,
-                                                            const BlockClasses* __restrict__ lists,
-                                                            const float* __restrict__ col,
-                                                            const unsigned* __restrict__ cbound,
-                                                            const float* __restrict__ grid,
-                                                            const float* __restrict__ cgs, float* __restrict__ cgq,
-                                                            int n, const SceneCG* __restrict__ scg, DevCounts* dc) {
+// 60 -> 30; with the pairs dealt to the waves as they end (tile_pairs) instead of a
+// cell's pairs per lane in fixed shares 29 -> 25, 16-scene batch 36 -> 32.
+// Measured and not taken: by 2x2x2 blocks too (1M bar 45 -> 66 us, 256-scene batch
+// 354 -> 437, 8M impact 210 -> 183: listing a block's 1,000 cells takes longer than
+// the runs of k_cg_q), and the P2G's pairs dealt like this (8M impact 391 -> 780 us:
+// its eight atomics per node suffer from neighbouring lanes in one cell).
+template <int NT, typename ST>
+__global__ __launch_bounds__(NT) void k_cg_q_page(DevParams dp, ST s, BlockTables t,
+                                                  const BlockClasses* __restrict__ lists,
+                                                  const float* __restrict__ col, const unsigned* __restrict__ cbound,
+                                                  const float* __restrict__ grid, const float* __restrict__ cgs,
+                                                  float* __restrict__ cgq, int n, const SceneCG* __restrict__ scg,
+                                                  DevCounts* dc) {
     using A = TileAcc<4>;
     __shared__ unsigned long long acc[A::kStride];
-    __shared__ TileCells<4> S;
-    __shared__ int sexp;
+    __shared__ TileCells<4, NT> S;
+    __shared__ int sexp, next;
     if (cg_stopped(dc)) return;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     int nb = dc->num_blocks;
@@ -454,32 +473,24 @@ __global__ __launch_bounds__(kTileThreads) void k_cg_q_page(DevParams dp, ST s, 
         const int scene = __builtin_amdgcn_readfirstlane(scene_of_page(dp, bkey << 3));
         if (scg[scene].done) continue;   // uniform over the workgroup
         const int o3[3] = {4 * ((child >> 2) & 1), 4 * ((child >> 1) & 1), 4 * (child & 1)};
-        for (int q = tid; q < A::kStride; q += kTileThreads) acc[q] = 0ull;
+        for (int q = tid; q < A::kStride; q += NT) acc[q] = 0ull;
+        if (tid == 0) next = 0;
         if (wave == 1) {
             const int pg = lane < 27 ? L->page[lane] : -1;
             const float bm = wave_max(pg >= 0 ? __uint_as_float(cbound[pg]) : 0.f);
             if (lane == 0) sexp = fix_exp(bm);
         }
-        tile_cells<4>(L, t.cell_start, n, o3, S);   // ends in a barrier
+        tile_cells(L, t.cell_start, n, o3, S);   // ends in a barrier
         const int e = sexp;
         const float sc = ldexpf(1.0f, e);
         const DevParams sp = dp.scenes[scene];
-        const int cells = S.cells, pairs = S.pairs[cells];
-        if (pairs > 0) {
-            // as in the P2G: about a cell's pairs per lane
-            const int all = (pairs + kTileThreads - 1) / kTileThreads, one = (pairs + cells - 1) / cells;
-            const int P = all < one ? all : one;
-            for (int c0 = tid * P; c0 < pairs; c0 += kTileThreads * P) {
-                const int ce = c0 + P < pairs ? c0 + P : pairs;
-                int r = tile_find(S, c0);
-                for (int q = c0; q < ce; ++q) {
-                    while (q >= S.pairs[r + 1]) ++r;
-                    const int place = S.place[r], i = S.start[r] + 2 * (q - S.pairs[r]);
-                    const bool two = !(place >> 12) || q + 1 < S.pairs[r + 1];
-                    cgq_pair(sp, s, i, two, place, col, sc, acc);
-                }
-            }
-        }
+        int bc[3], org[3];   // the tile's first node in scene-local cells
+        unmorton(bkey, bc[0], bc[1], bc[2]);
+#pragma unroll
+        for (int a = 0; a < 3; ++a) org[a] = 8 * bc[a] + o3[a] - sp.origin[a];
+        tile_pairs(S, &next, [&](int i, bool two, int place, int j) {
+            cgq_pair(sp, s, i, two, place, j, org, col, sc, acc);
+        });
         __syncthreads();
         if (tid < 64) {
             const int node = (tid >> 4) * A::kX + ((tid >> 2) & 3) * A::kZ + (tid & 3);
@@ -682,9 +693,14 @@ static void apply_blocks(mpmx_ctx* c, ST st) {
     if (tiles_are_pages(c, 400)) {
         MPMX_TIMED(c, "cg_col", (k_cg_col<4, ST><<<8 * g, 256, 0, c->stream>>>(c->dp, st, c->vol, t, lists, info, c->cg_s,
                                                                             c->cg_col, c->cbound, n, c->scg, c->dc)));
-        MPMX_TIMED(c, "cg_q", (k_cg_q_page<ST><<<8 * g, kTileThreads, 0, c->stream>>>(
-                                  c->dp, st, t, lists, c->cg_col, c->cbound, c->grid, c->cg_s, c->cg_q, n, c->scg,
-                                  c->dc)));
+        if (pages_are_few(c))
+            MPMX_TIMED(c, "cg_q", (k_cg_q_page<512, ST><<<8 * g, 512, 0, c->stream>>>(
+                                      c->dp, st, t, lists, c->cg_col, c->cbound, c->grid, c->cg_s, c->cg_q, n, c->scg,
+                                      c->dc)));
+        else
+            MPMX_TIMED(c, "cg_q", (k_cg_q_page<kTileThreads, ST><<<8 * g, kTileThreads, 0, c->stream>>>(
+                                      c->dp, st, t, lists, c->cg_col, c->cbound, c->grid, c->cg_s, c->cg_q, n, c->scg,
+                                      c->dc)));
         return;
     }
     MPMX_TIMED(c, "cg_col", (k_cg_col<8, ST><<<g, 256, 0, c->stream>>>(c->dp, st, c->vol, t, lists, info, c->cg_s,

@@ -399,6 +399,13 @@ bool tiles_are_pages(const mpmx_ctx* c, int percent) {
     return c->hc->num_blocks > 0 && 100 * (int64_t)c->hc->num_blocks <= percent * (int64_t)c->num_cu;
 }
 
+// The P2G and the K s gather take a page by 512 threads while there are about two
+// pages per CU, where a page's chain of pairs is what takes the time; with more
+// pages the extra threads only wait.  P2G by 512 / 256 threads, 1,000 cube 17 / 20
+// us, 64,000 cube (64 blocks) 30 / 37, 137,000 APIC sphere (~150) 73 / 61; K s 7.6 /
+// 8.9, 11.6 / 15.0, 20 / 18.
+bool pages_are_few(const mpmx_ctx* c) { return tiles_are_pages(c, 30); }
+
 int transfer_grid_blocks(mpmx_ctx* c) {
     // enough workgroups to fill every CU several times over; a multiple of 8 so
     // that the XCD-aware remap of block ids applies

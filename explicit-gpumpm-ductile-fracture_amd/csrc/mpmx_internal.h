@@ -636,6 +636,7 @@ hipError_t fill_zero_dev_count(mpmx_ctx* c, float* p, const int* count_dev, int6
 void timer_push(mpmx_ctx* c, const char* name, bool begin);
 void destroy_graphs(mpmx_ctx* c);
 int transfer_grid_blocks(mpmx_ctx* c);
+bool pages_are_few(const mpmx_ctx* c);                   // page tiles by 512 threads
 bool tiles_are_pages(const mpmx_ctx* c, int percent);   // gathers and G2P by page, not by 2x2x2 block
 int block_grid(mpmx_ctx* c, int pct);
 }  // namespace mpmx
