@@ -22,6 +22,7 @@
 // do not depend on the order of the additions.  Each particle is read by the
 // one to eight blocks it reaches (about twice on average).
 #include "payload.h"
+#include <type_traits>
 
 namespace mpmx {
 
@@ -260,7 +261,8 @@ __global__ __launch_bounds__(256) void k_p2g_prep(DevParams dp, ST s, WaveMap wm
 // and lanes idle where their nodes fall outside the block: 8M impact (8
 // particles a cell) 743 -> 396 us, 256-scene batch (4, random) 1,340 -> 1,020
 // us, 64,000 cube 175 -> 36 us (page tiles; 94 with block tiles), 1M bar
-// (0.6) 142 -> 149 us.  Measured and not taken: 512 threads (443, 1,221 us),
+// (0.6) 142 -> 149 us.  Measured and not taken: 512 threads (443, 1,221 us; taken for
+// few blocks, see the dispatch),
 // pairs and the odd cells' last particles in two passes (405, 1,105 us), tiles
 // taken in turn by resident workgroups with the next tile's cells loaded ahead
 // (467, 1,170 us).
@@ -798,18 +800,28 @@ static hipError_t gather_blocks_t(mpmx_ctx* c, float dt) {
         return hipGetLastError();
     }
     const BlockClasses* lists = static_cast<BlockClasses*>(c->block_lists);
-    if (tiles_are_pages(c, 150) && pages_are_few(c))
-        MPMX_TIMED(c, "p2g_block", (k_p2g_tile<4, TRANSFER, 512><<<8 * g, 512, 0, c->stream>>>(
+    auto tiles = [&](auto e, auto threads) {
+        constexpr int E = decltype(e)::value, NT = decltype(threads)::value;
+        MPMX_TIMED(c, "p2g_block", (k_p2g_tile<E, TRANSFER, NT><<<E == 8 ? g : 8 * g, NT, 0, c->stream>>>(
                                         c->dp, c->payload, c->pbound, t, lists, c->grid, raw, cg_vec(c), dt, (int)c->n,
                                         c->dc)));
-    else if (tiles_are_pages(c, 150))
-        MPMX_TIMED(c, "p2g_block", (k_p2g_tile<4, TRANSFER, kTileThreads><<<8 * g, kTileThreads, 0, c->stream>>>(
-                                        c->dp, c->payload, c->pbound, t, lists, c->grid, raw, cg_vec(c), dt, (int)c->n,
-                                        c->dc)));
-    else
-        MPMX_TIMED(c, "p2g_block", (k_p2g_tile<8, TRANSFER, kTileThreads><<<g, kTileThreads, 0, c->stream>>>(
-                                        c->dp, c->payload, c->pbound, t, lists, c->grid, raw, cg_vec(c), dt, (int)c->n,
-                                        c->dc)));
+    };
+    using std::integral_constant;
+    // Page tiles while the blocks are fewer than the CUs, 512 threads per tile
+    // while that fills idle SIMDs: a page's or a block's chain of pairs is then
+    // what takes the time.  With more blocks per CU a 256-thread tile ends
+    // sooner beside others.  P2G in us by pages of 256 and 512 threads, blocks of
+    // 256 and 512 (cubes of 8 and spheres of 3 particles per cell):
+    //   MLS   64 blocks 38 / 29 / 90 / 62, 125: 45 / 48 / 89 / 63, 216: 48 / 49 / 89 / 64
+    //         and 70 / 81 / 101 / 72, 317: 57 / 69 / 55 / 44, 512: 141 / 175 / 116 / 92,
+    //         828: 131 / 173 / 84 / 78, 1,000: 319 / 395 / 182 / 176, ~2,400: - / - / 124 / 147
+    //   APIC  64: 43 / 36 / 112 / 71, 125: 58 / 68 / 111 / 71, 216: 51 / 83 / 111 / 72 and
+    //         87 / 125 / 126 / 81, 317: 70 / 110 / 64 / 46, 512: 181 / 293 / 149 / 124,
+    //         595: 121 / 206 / 76 / 83, 1,000: 414 / 680 / 224 / 275
+    if (pages_are_few(c)) tiles(integral_constant<int, 4>{}, integral_constant<int, 512>{});
+    else if (tiles_are_pages(c, 85)) tiles(integral_constant<int, 4>{}, integral_constant<int, kTileThreads>{});
+    else if (tiles_are_pages(c, TRANSFER == 0 ? 400 : 200)) tiles(integral_constant<int, 8>{}, integral_constant<int, 512>{});
+    else tiles(integral_constant<int, 8>{}, integral_constant<int, kTileThreads>{});
     // the PCG's starting "dot"(r, z) comes with its first "dot"(s, q) (k_cg_dot)
     return hipGetLastError();
 }

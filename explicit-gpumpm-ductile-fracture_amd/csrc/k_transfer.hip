@@ -389,21 +389,18 @@ int block_grid(mpmx_ctx* c, int pct) {
 // Page tiles while the blocks (by the last published count) are at most
 // percent % of the CUs: eight times the workgroups, but each particle in 3.4
 // gather tiles instead of 1.95, and 3.4 nodes staged per node instead of 1.95.
-// P2G (150): by pages / by blocks, 64,000 cube (64 blocks) 36 / 94 us, 333,333
-// sphere (~300) 72 / 84, 512,000 cube (~340) 85 / 100, 1M impact (~450) 134 /
-// 108, 16-scene batch (~600) 82 / 66.
 // K s gather, K s column and G2P (400), which leave more of the GPU idle by
-// blocks: 1M impact 62 / 78, 17 / 26 and 52 / 73 us, 16-scene batch 32 / 42, 11
-// / 14 and 26 / 34, 64-scene batch (~2,400) 103 / 48, 33 / 19 and 104 / 68.
+// blocks (pages / blocks, us): 1M impact (~450 blocks) 62 / 78, 17 / 26 and 52 / 73,
+// 16-scene batch (~600) 32 / 42, 11 / 14 and 26 / 34, 64-scene batch (~2,400) 103 /
+// 48, 33 / 19 and 104 / 68.  The P2G's lines are at its dispatch.
 bool tiles_are_pages(const mpmx_ctx* c, int percent) {
     return c->hc->num_blocks > 0 && 100 * (int64_t)c->hc->num_blocks <= percent * (int64_t)c->num_cu;
 }
 
 // The P2G and the K s gather take a page by 512 threads while there are about two
 // pages per CU, where a page's chain of pairs is what takes the time; with more
-// pages the extra threads only wait.  P2G by 512 / 256 threads, 1,000 cube 17 / 20
-// us, 64,000 cube (64 blocks) 30 / 37, 137,000 APIC sphere (~150) 73 / 61; K s 7.6 /
-// 8.9, 11.6 / 15.0, 20 / 18.
+// pages the extra threads only wait.  K s by 512 / 256 threads, 1,000 cube 7.6 / 8.9
+// us, 64,000 cube (64 blocks) 11.6 / 15.0, 137,000 sphere (~150) 20 / 18.
 bool pages_are_few(const mpmx_ctx* c) { return tiles_are_pages(c, 30); }
 
 int transfer_grid_blocks(mpmx_ctx* c) {

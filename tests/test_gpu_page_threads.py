@@ -1,5 +1,6 @@
-"""Page tiles by 512 threads (about two pages per CU) and by 256 (more): alone,
-scenes on either side of the line; inside a batch of many blocks by 2x2x2 blocks.
+"""The P2G's tiles, pages by 512 or 256 threads and 2x2x2 blocks by 512 or 256, by
+the number of blocks (the K s gather's pages alike): scenes alone on either side of
+each line, and inside a batch of many blocks, by blocks of 256 threads.
 The fixed-point sums do not depend on the tiling, so all must agree bit for bit."""
 import numpy as np
 import pytest
@@ -11,12 +12,14 @@ FIELDS = ("x", "v", "F", "B", "c", "alpha", "psi", "g")
 
 @pytest.mark.parametrize("precision", ["fp32", "mixed"])
 @pytest.mark.parametrize("transfer", [0, 1])
-@pytest.mark.parametrize("cells,n", [(20, 20001), (28, 30000), (46, 30000)])   # 27, 64 and 216 blocks
+@pytest.mark.parametrize("cells,n", [(20, 20001), (28, 30000), (46, 30000), (54, 40000), (75, 60000)])
+# about 27, 64, 216, 340 and 1,000 blocks
 def test_page_tiles_equal_blocks(mpmx, cells, n, transfer, precision):
     cfg = mpmx.default_config(precision=mpmx.FP32 if precision == "fp32" else mpmx.MIXED)
-    p = mpmx.default_params(N=64, transfer=transfer, E=1e4, nu=0.3, V0=1e-7, yield_stress=100.0)
+    N = 96 if cells > 50 else 64
+    p = mpmx.default_params(N=N, transfer=transfer, E=1e4, nu=0.3, V0=1e-7, yield_stress=100.0)
     rng = np.random.default_rng(3)
-    x = ((8 + rng.uniform(0.0, cells, (n, 3))) / 64).astype(np.float32).astype(np.float64)
+    x = ((8 + rng.uniform(0.0, cells, (n, 3))) / N).astype(np.float32).astype(np.float64)
     v = rng.normal(0.0, 0.3, (n, 3)).astype(np.float32).astype(np.float64)
     pf = mpmx.default_params(N=128, transfer=transfer, E=1e4, nu=0.3, V0=1e-7, yield_stress=100.0)
     xf = rng.uniform(0.1, 0.9, (20000, 3)).astype(np.float32).astype(np.float64)
