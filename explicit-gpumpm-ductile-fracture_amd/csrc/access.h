@@ -583,15 +583,32 @@ __device__ __forceinline__ void st_B(const MState& s, int i, int k, int n, float
     s.B[(int64_t)k * n + i] = f2bf(f);
 }
 
-__device__ __forceinline__ float ld_F(const PState& s, int i, int k, int n) { return s.F[(int64_t)k * n + i]; }
-__device__ __forceinline__ float ld_F(const MState& s, int i, int k, int n) {
-    if (s.F32) return s.F32[(int64_t)k * n + i];
-    return h2f(s.F[(int64_t)k * n + i]) + ((k == 0 || k == 4 || k == 8) ? 1.0f : 0.0f);
+// all of F (k = r + 3c): one branch on the storage form for the nine of them
+__device__ __forceinline__ void ld_F(const PState& s, int i, int n, float (&F)[9]) {
+#pragma unroll
+    for (int k = 0; k < 9; ++k) F[k] = s.F[(int64_t)k * n + i];
 }
-__device__ __forceinline__ void st_F(const PState& s, int i, int k, int n, float f) { s.F[(int64_t)k * n + i] = f; }
-__device__ __forceinline__ void st_F(const MState& s, int i, int k, int n, float f) {
-    if (s.F32) s.F32[(int64_t)k * n + i] = f;
-    else s.F[(int64_t)k * n + i] = f2h(f - ((k == 0 || k == 4 || k == 8) ? 1.0f : 0.0f));
+__device__ __forceinline__ void ld_F(const MState& s, int i, int n, float (&F)[9]) {
+    if (s.F32) {
+#pragma unroll
+        for (int k = 0; k < 9; ++k) F[k] = s.F32[(int64_t)k * n + i];
+    } else {
+#pragma unroll
+        for (int k = 0; k < 9; ++k) F[k] = h2f(s.F[(int64_t)k * n + i]) + (k % 4 == 0 ? 1.0f : 0.0f);
+    }
+}
+__device__ __forceinline__ void st_F(const PState& s, int i, int n, const float (&F)[9]) {
+#pragma unroll
+    for (int k = 0; k < 9; ++k) s.F[(int64_t)k * n + i] = F[k];
+}
+__device__ __forceinline__ void st_F(const MState& s, int i, int n, const float (&F)[9]) {
+    if (s.F32) {
+#pragma unroll
+        for (int k = 0; k < 9; ++k) s.F32[(int64_t)k * n + i] = F[k];
+    } else {
+#pragma unroll
+        for (int k = 0; k < 9; ++k) s.F[(int64_t)k * n + i] = f2h(F[k] - (k % 4 == 0 ? 1.0f : 0.0f));
+    }
 }
 
 __device__ __forceinline__ float ld_c(const PState& s, int i) { return s.c[i]; }

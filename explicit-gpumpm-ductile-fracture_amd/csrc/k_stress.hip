@@ -322,44 +322,39 @@ __device__ __forceinline__ void count_fallbacks(bool fb, int* counter) {
 
 // state access of the two storage forms
 __device__ __forceinline__ void stress_load(const PState& s, int i, int n, StressIn& in) {
+    float F[9];
+    ld_F(s, i, n, F);
 #pragma unroll
-    for (int r = 0; r < 3; ++r)
-#pragma unroll
-        for (int cc = 0; cc < 3; ++cc) in.F[r][cc] = s.F[(int64_t)(r + 3 * cc) * n + i];
+    for (int k = 0; k < 9; ++k) in.F[k % 3][k / 3] = F[k];
     in.c = s.c[i];
     in.g = s.g[i];
     in.alpha = s.alpha[i];
     in.psi = s.psi[i];
 }
 __device__ __forceinline__ void stress_load(const MState& s, int i, int n, StressIn& in) {
+    float F[9];
+    ld_F(s, i, n, F);
 #pragma unroll
-    for (int r = 0; r < 3; ++r)
-#pragma unroll
-        for (int cc = 0; cc < 3; ++cc)
-            in.F[r][cc] = s.F32 ? s.F32[(int64_t)(r + 3 * cc) * n + i]
-                                : h2f(s.F[(int64_t)(r + 3 * cc) * n + i]) + (r == cc ? 1.0f : 0.0f);
+    for (int k = 0; k < 9; ++k) in.F[k % 3][k / 3] = F[k];
     in.c = bf2f(s.c[i]);
     in.g = bf2f(s.g[i]);
     in.alpha = bf2f(s.alpha[i]);
     in.psi = bf2f(s.psi[i]);
 }
 __device__ __forceinline__ void stress_store(const PState& s, int i, int n, const StressOut& out) {
+    float F[9];
 #pragma unroll
-    for (int r = 0; r < 3; ++r)
-#pragma unroll
-        for (int cc = 0; cc < 3; ++cc) s.F[(int64_t)(r + 3 * cc) * n + i] = out.F[r][cc];
+    for (int k = 0; k < 9; ++k) F[k] = out.F[k % 3][k / 3];
+    st_F(s, i, n, F);
     s.g[i] = out.g;
     s.alpha[i] = out.alpha;
     s.psi[i] = out.psi;
 }
 __device__ __forceinline__ void stress_store(const MState& s, int i, int n, const StressOut& out) {
+    float F[9];
 #pragma unroll
-    for (int r = 0; r < 3; ++r)
-#pragma unroll
-        for (int cc = 0; cc < 3; ++cc) {
-            if (s.F32) s.F32[(int64_t)(r + 3 * cc) * n + i] = out.F[r][cc];
-            else s.F[(int64_t)(r + 3 * cc) * n + i] = f2h(out.F[r][cc] - (r == cc ? 1.0f : 0.0f));
-        }
+    for (int k = 0; k < 9; ++k) F[k] = out.F[k % 3][k / 3];
+    st_F(s, i, n, F);
     s.g[i] = f2bf(out.g);
     s.alpha[i] = f2bf(out.alpha);
     s.psi[i] = f2bf(out.psi);

@@ -191,6 +191,12 @@ __device__ __forceinline__ void g2p_particle(const DevParams& dp, const ST& s, i
         // hoist all 108 staged-node reads and hold them in registers
         __builtin_amdgcn_sched_barrier(0);
     }
+    // G in registers here: its sums would be sunk to their use past the branch on
+    // F's storage form, with their terms (171 VGPRs)
+    if (TRANSFER == 1) {
+#pragma unroll
+        for (int k = 0; k < 9; ++k) asm volatile("" : "+v"(G[k]));
+    }
     // B and the damage update first: stored before the velocity clamp's
     // branch, their sums over the 27 nodes are not sunk past it (where their
     // terms would hold over a hundred registers)
@@ -219,9 +225,8 @@ __device__ __forceinline__ void g2p_particle(const DevParams& dp, const ST& s, i
     A[0] += 1.f;
     A[4] += 1.f;
     A[8] += 1.f;
-    float F[9];
-#pragma unroll
-    for (int k = 0; k < 9; ++k) F[k] = ld_F(s, i, k, n);
+    float F[9], Fn[9];
+    ld_F(s, i, n, F);
     bool finite = true;
 #pragma unroll
     for (int r = 0; r < 3; ++r)
@@ -231,8 +236,9 @@ __device__ __forceinline__ void g2p_particle(const DevParams& dp, const ST& s, i
             // the rounding does not depend on how the compiler pairs them
             const float f = fmaf(A[r + 6], F[3 * cc + 2], fmaf(A[r], F[3 * cc], A[r + 3] * F[3 * cc + 1]));
             finite = finite && isfinite(f);
-            st_F(s, i, r + 3 * cc, n, f);
+            Fn[r + 3 * cc] = f;
         }
+    st_F(s, i, n, Fn);
     const float lo = 2.0f * dp.dx, hi = 1.0f - 2.0f * dp.dx;
     if (!(xn[0] >= lo && xn[0] <= hi && xn[1] >= lo && xn[1] <= hi && xn[2] >= lo && xn[2] <= hi))
         atomicOr(&dc->err, isfinite(xn[0] + xn[1] + xn[2]) ? kErrDomain : kErrNonFinite);
