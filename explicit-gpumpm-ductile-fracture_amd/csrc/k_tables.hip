@@ -355,9 +355,11 @@ hipError_t build_tables(mpmx_ctx* c) {
     if ((e = scan_exclusive3(c, sc, 3, words)) != hipSuccess) return e;
     // words per wave: a wave takes its occupied words one after another, so
     // the words are spread out (8 a wave, 1M bar's 4,096 words 38 -> 7 us) until
-    // there are waves enough without (64 a wave: a batch's mostly empty ones).
+    // there are waves enough without (a batch's mostly empty words: 256 scenes of
+    // up to 200,000 particles 37, 25, 19 and 19 us by 64, 32, 16 and 8 a wave, of
+    // half that size 10.7, 10.6, 12.6 and 17.4).
     // At least a thread per word: the first also write the per-scene ranges.
-    const int per = words <= (1 << 17) ? 8 : 64;
+    const int per = words <= (1 << 17) ? 8 : 32;
     k_page_keys<<<(int)((words + 4 * per - 1) / (4 * per)), 256, 0, c->stream>>>(
         c->dp, c->pmask, c->nmask, c->wcount, c->scount, c->bcount, words, per, c->page_key, c->cap_p, c->cap_tp,
         c->block_key, c->tp_bound, c->scg, c->dc);
