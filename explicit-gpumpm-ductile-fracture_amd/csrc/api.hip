@@ -821,6 +821,8 @@ static mpmx_status upload_particles(mpmx_ctx* c, const int64_t* counts, const st
         HIPCHK(c, dalloc(&c->mv_val[b], n));
     }
     c->sort_by_movers = c->cfg.sort_variant != 1;
+    c->few_movers = false;
+    c->few_after = 0;
     // keys: cell bits, the slot's page bits and (batch) the slot index
     c->key_bits = c->num_scenes == 1 ? 6 + 3 * std::max(1, ceil_log2(c->P.N / 4))
                                      : 6 + 3 * c->slot_log2 + ceil_log2(c->num_scenes);

@@ -1100,10 +1100,15 @@ static hipError_t sort_movers(mpmx_ctx* c) {
 // Which path the next sort takes.  few_movers: the movers' own sort in one
 // workgroup, where the last published count (or n itself) leaves room for
 // growth by a third up to its capacity; a count not published yet (-1, the
-// first sorts after an upload) is taken as large unless n is small.
+// first sorts after an upload) is taken as large unless n is small.  A count
+// that jumps past the capacity (a lattice crossing its cells at once) takes that
+// workgroup about 10 ns a mover, 6 ms on the 8M impact: so not above 2,097,152
+// particles, and after such a jump not for as many sorts as make up for it.
 void choose_sort_path(mpmx_ctx* c) {
+    const int64_t now = c->sorts + c->substeps;
+    if (c->few_movers && c->hc->movers > kMsCap) c->few_after = now + 64 * std::max<int64_t>(1, c->n >> 18);
     const int64_t bound = c->hc->movers < 0 ? c->n : std::min<int64_t>(c->n, (int64_t)c->hc->movers * 4 / 3);
-    c->few_movers = bound <= kMsCap;
+    c->few_movers = bound <= kMsCap && (c->n <= kMsCap || (c->n <= (1 << 21) && now >= c->few_after));
     if (c->cfg.sort_variant != 0) {
         c->sort_by_movers = c->cfg.sort_variant == 2;
         return;
@@ -1119,6 +1124,7 @@ void choose_sort_path(mpmx_ctx* c) {
 // sort's keys, so the first sort after an upload takes the radix path.
 hipError_t sort_keys(mpmx_ctx* c) {
     choose_sort_path(c);
+    ++c->sorts;
     const bool movers = c->sort_by_movers && c->old_keys_sorted;
     hipError_t e = movers ? sort_movers(c) : sort_radix(c);
     if (e != hipSuccess) return e;

@@ -228,6 +228,7 @@ struct mpmx_ctx {
     bool sort_by_movers = true;   // the path the next sort takes (mpmx_config.sort_variant 0: from
                                   // the last published mover count)
     bool few_movers = false;      // the movers are few enough for the one-workgroup sort
+    int64_t sorts = 0, few_after = 0;   // sorts made; sorts + substeps from which few_movers may be set again
     bool old_keys_sorted = false; // keys holds a sort's output (the mover path's precondition)
     bool tables_match_keys = false;   // the page tables were built from keys (the mover path uses them)
     int* mv_tbound = nullptr;     // [sort_tiles + 1] sorted movers before each tile's first slot
