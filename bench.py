@@ -16,7 +16,7 @@ both sides).  `value` = particles x substeps / seconds of that window;
 `config.timed_substeps` names the window and `cg_iters_last` the PCG
 iterations of its last substep.
 
-`roofline`: the block P2G kernel (`k_p2g_block`, the largest kernel) timed
+`roofline`: the block P2G kernel (`k_p2g_tile`, the largest kernel) timed
 with HIP events around each launch in an instrumented pass of the same
 workload.  achieved = algorithmic bytes / average launch time, with the
 algorithmic bytes of an FP32 P2G, 104 B per particle (x, v, C, sigma, c and
@@ -152,7 +152,7 @@ TRAFFIC_SUMMARY = os.path.join(ROOT, "profiles", "traffic_p2g_block_%s.md")
 
 
 def measured_traffic(workload):
-    """HBM bytes per launch of k_p2g_block from the committed counter summary
+    """HBM bytes per launch of k_p2g_tile from the committed counter summary
     of this workload (line `traffic_bytes_per_launch: B`), or None."""
     path = TRAFFIC_SUMMARY % workload
     if not os.path.exists(path):
