@@ -743,8 +743,10 @@ __global__ __launch_bounds__(kRsThreads) void k_place(MoverSet M, const uint32_t
 // the waves, and the items change places through LDS.  Larger counts, which
 // the caller's last published count did not foresee, go through the same
 // ranking tile by tile with the passes' output in global memory: slow, and
-// the next sort takes the general path.  Finally each tile of slots gets the
-// sorted movers that precede its first slot (tbound), by search.
+// the next sort takes the general path.  list is one of the output buffers
+// (kb0 or kb1): the first pass reads it before anything overwrites it.
+// Finally each tile of slots gets the sorted movers that precede its first
+// slot (tbound), by search.
 constexpr int kMsThreads = 1024;
 constexpr int kMsItems = 16;
 constexpr int kMsCap = kMsThreads * kMsItems;
@@ -783,8 +785,8 @@ __device__ __forceinline__ void ms_rank(const uint32_t (&k)[kMsItems], uint32_t 
         }
     }
 }
-// digit-major exclusive offsets of the waves' counters; base[d] = start[d]
-// plus nothing for a single tile, run[d] = the tile's count of digit d
+// wcnt[w][d] becomes the items of digit d in the waves before w; mine, for
+// thread d < 256, the tile's count of digit d
 __device__ __forceinline__ void ms_offsets(MsLds& L, int& mine) {
     mine = 0;
     if (threadIdx.x < 256) {
@@ -812,7 +814,7 @@ __device__ __forceinline__ void ms_scan256(MsLds& L, int v) {
     }
     __syncthreads();
 }
-__global__ __launch_bounds__(kMsThreads) void k_mover_sort(const uint32_t* __restrict__ list, const int* m_dev, int n,
+__global__ __launch_bounds__(kMsThreads) void k_mover_sort(const uint32_t* list, const int* m_dev, int n,
                                                            int passes, uint32_t* kb0, uint32_t* vb0, uint32_t* kb1,
                                                            uint32_t* vb1, const uint32_t* __restrict__ old,
                                                            const int* __restrict__ toff, int tiles,
