@@ -756,6 +756,13 @@ struct MsLds {
     uint32_t base[256], run[256];
     int lds4[4];
 };
+// the wave's LDS writes before it are seen by all its lanes after it (the
+// barrier alone orders no memory)
+__device__ __forceinline__ void wave_lds_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+}
 // ranks of the wave's items among its items of the same digit; wcnt[w]
 // receives the wave's digit counts
 __device__ __forceinline__ void ms_rank(const uint32_t (&k)[kMsItems], uint32_t (&rank)[kMsItems], int per, int first,
@@ -764,7 +771,7 @@ __device__ __forceinline__ void ms_rank(const uint32_t (&k)[kMsItems], uint32_t 
     const uint64_t lt = (lane == 0) ? 0ull : ((~0ull) >> (64 - lane));
 #pragma unroll
     for (int q = 0; q < 4; ++q) wc[q * 64 + lane] = 0u;
-    __builtin_amdgcn_wave_barrier();
+    wave_lds_sync();
 #pragma unroll
     for (int r = 0; r < kMsItems; ++r) {
         if (r < per) {   // uniform
@@ -779,9 +786,9 @@ __device__ __forceinline__ void ms_rank(const uint32_t (&k)[kMsItems], uint32_t 
             }
             const uint32_t prev = valid ? wc[d] : 0u;
             rank[r] = prev + (uint32_t)__popcll(peers & lt);
-            __builtin_amdgcn_wave_barrier();
+            wave_lds_sync();
             if (valid && (peers & lt) == 0ull) wc[d] = prev + (uint32_t)__popcll(peers);
-            __builtin_amdgcn_wave_barrier();
+            wave_lds_sync();
         }
     }
 }
