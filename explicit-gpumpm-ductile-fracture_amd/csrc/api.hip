@@ -813,7 +813,7 @@ static mpmx_status upload_particles(mpmx_ctx* c, const int64_t* counts, const st
     HIPCHK(c, dalloc(&c->mv_toff, c->sort_tiles));
     HIPCHK(c, dalloc(&c->mv_old, n));
     HIPCHK(c, dalloc(&c->mv_slot, n));
-    HIPCHK(c, dalloc(&c->mv_tbound, c->sort_tiles + 1));
+    HIPCHK(c, dalloc(&c->mv_tbound, (int64_t)most_runs(n) * (c->sort_tiles + 1)));
     HIPCHK(c, dalloc(&c->mv_cpre, n / 64 + 1));
     HIPCHK(c, dalloc(&c->mv_cmask, n / 64 + 1));
     for (int b = 0; b < 2; ++b) {
@@ -821,8 +821,6 @@ static mpmx_status upload_particles(mpmx_ctx* c, const int64_t* counts, const st
         HIPCHK(c, dalloc(&c->mv_val[b], n));
     }
     c->sort_by_movers = c->cfg.sort_variant != 1;
-    c->few_movers = false;
-    c->few_after = 0;
     // keys: cell bits, the slot's page bits and (batch) the slot index
     c->key_bits = c->num_scenes == 1 ? 6 + 3 * std::max(1, ceil_log2(c->P.N / 4))
                                      : 6 + 3 * c->slot_log2 + ceil_log2(c->num_scenes);
@@ -1050,7 +1048,6 @@ static mpmx_status capture_substep(mpmx_ctx* c, double dt, int iters) {
     const int p = c->cur;
     choose_sort_path(c);
     const bool by_movers = c->sort_by_movers && c->old_keys_sorted;   // the path sort_keys takes
-    const bool few_movers = c->few_movers;
     uint32_t* const keys0 = c->keys;
     uint32_t* const keys1 = c->keys_alt;
     auto& G = c->graphs[p];
@@ -1100,7 +1097,6 @@ static mpmx_status capture_substep(mpmx_ctx* c, double dt, int iters) {
     G.dt = (float)dt;
     G.iters = iters;
     G.by_movers = by_movers;
-    G.few_movers = few_movers;
     G.blocks = c->hc->num_blocks;
     return MPMX_OK;
 }
@@ -1115,7 +1111,7 @@ static mpmx_status substep_graph(mpmx_ctx* c, double dt) {
     choose_sort_path(c);
     const bool by_movers = c->sort_by_movers && c->old_keys_sorted;
     if (!G.valid || G.dt != (float)dt || G.iters != want || c->hc->num_blocks > G.blocks + G.blocks / 4 + 64 ||
-        G.by_movers != by_movers || (by_movers && G.few_movers != c->few_movers)) {
+        G.by_movers != by_movers) {
         mpmx_status s = capture_substep(c, dt, want);
         if (s != MPMX_OK) return s;
     }

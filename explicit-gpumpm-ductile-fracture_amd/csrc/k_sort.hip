@@ -593,9 +593,47 @@ struct MoverSet {
     const int* cpre;
     const uint64_t* cmask;
 };
+// the movers before entry r (key K) of the sorted runs of kRunCap (see
+// k_mover_sort), which comes after `all` of the previous slots: those of its own
+// run, and of every other run those with (key, list index) below its own, by
+// search.  They lie between the run's bounds of the tile of slot all - 1 and of
+// the next: a tile that starts before slot `all` has a previous key <= K there
+// (the same only if the mover comes from a later slot), the next one >= K (the
+// same only if it comes from an earlier slot), so its bound lies on the same
+// side of the mover.  Four runs at a time, so that four loads are in flight.
+__device__ __forceinline__ int rank_in_runs(const uint32_t* __restrict__ skey, int m, int r, uint32_t K, int all,
+                                            const int* __restrict__ tbound, int tiles) {
+    const int own = r / kRunCap, t = all > 0 ? (all - 1) / kRsTile : 0;
+    int rank = r - own * kRunCap;
+    for (int u = 0; u * kRunCap < m; u += 4) {
+        int pos[4], hi[4], most = 0;
+#pragma unroll
+        for (int h = 0; h < 4; ++h) {
+            const int b = (u + h) * kRunCap, len = m - b < kRunCap ? m - b : kRunCap;
+            pos[h] = hi[h] = 0;
+            if (len > 0 && u + h != own) {
+                const int* tb = tbound + (int64_t)(u + h) * (tiles + 1) + t;
+                pos[h] = all > 0 ? tb[0] : 0;
+                hi[h] = tb[1] < len ? tb[1] : len;
+                most = hi[h] - pos[h] > most ? hi[h] - pos[h] : most;
+            }
+        }
+        for (int step = most > 0 ? 1 << (31 - __clz(most)) : 0; step > 0; step >>= 1)
+#pragma unroll
+            for (int h = 0; h < 4; ++h) {
+                if (pos[h] + step > hi[h]) continue;
+                const uint32_t k = skey[(u + h) * kRunCap + pos[h] + step - 1];
+                if (k < K || (k == K && u + h < own)) pos[h] += step;
+            }
+        rank += (pos[0] + pos[1]) + (pos[2] + pos[3]);
+    }
+    return rank;
+}
+// RUNS: the movers are sorted in runs of kRunCap only (tbound: their bounds)
+template <bool RUNS>
 __device__ __forceinline__ void place_movers(const MoverSet& M, int m, int gid, int threads, const OldTables& tb,
                                              bool use_tables, uint32_t* __restrict__ okeys,
-                                             uint32_t* __restrict__ perm) {
+                                             uint32_t* __restrict__ perm, const int* __restrict__ tbound, int tiles) {
     const int n = M.n;
     if (use_tables) {
         const int np = *tb.num_page;
@@ -610,7 +648,7 @@ __device__ __forceinline__ void place_movers(const MoverSet& M, int m, int gid, 
         if (use_tables) all = table_bound(tb, K, !up);
         else all = up ? search_near<kLower>(M.old, nullptr, n, K, 0u, i + 1) : search_near<kUpper>(M.old, nullptr, n, K, 0u, i - 1);
         all = all < 0 ? 0 : (all > n ? n : all);
-        const int pos = r + all - movers_before(M.cpre, M.cmask, all, n, m);
+        const int pos = (RUNS ? rank_in_runs(M.skey, m, r, K, all, tbound, tiles) : r) + all - movers_before(M.cpre, M.cmask, all, n, m);
         if (pos < 0 || pos >= n) continue;   // only if the previous keys were not sorted
         okeys[pos] = K;
         perm[pos] = (uint32_t)i;
@@ -635,7 +673,7 @@ __global__ __launch_bounds__(kRsThreads) void k_place_movers(MoverSet M, const i
     } else if (tq == tiles) {
         tbound[tiles] = m;
     }
-    place_movers(M, m, gid, gridDim.x * blockDim.x, tb, use_tables, okeys, perm);
+    place_movers<false>(M, m, gid, gridDim.x * blockDim.x, tb, use_tables, okeys, perm, tbound, tiles);
 }
 
 // The stayers' places: stayer i (key k, m_i movers in slots before it) comes
@@ -716,9 +754,49 @@ __global__ __launch_bounds__(kRsThreads) void k_place_stayers(MoverSet M, const 
     m = m < M.n ? m : M.n;
     place_stayers(M, cur, m, (int)blockIdx.x, toff, tbound, okeys, perm, sm);
 }
+// the same over the movers' sorted runs: each run's entries between the
+// tile's bounds in it are searched for the thread's eight slots together
+__device__ __forceinline__ void place_stayers_runs(const MoverSet& M, const uint32_t* __restrict__ cur, int m, int tile,
+                                                   int tiles, const int* __restrict__ toff,
+                                                   const int* __restrict__ tbound, uint32_t* __restrict__ okeys,
+                                                   uint32_t* __restrict__ perm, int* lds4) {
+    const int n = M.n, base = tile * kRsTile;
+    uint32_t ko[kRsItems], kn[kRsItems];
+    const unsigned bits = mover_bits(M.old, cur, base, n, ko, kn);
+    int mr[2], total, before[kRsItems], c[kRsItems];
+    half_ranks(bits, toff[tile], mr, total, lds4);
+#pragma unroll
+    for (int j = 0; j < kRsItems; ++j) {
+        before[j] = mr[j / 4] + __popc((bits >> (j & 4)) & ((1u << (j & 3)) - 1u));
+        c[j] = 0;
+    }
+    for (int u = 0; u * kRunCap < m; ++u) {
+        const int b = u * kRunCap, len = m - b < kRunCap ? m - b : kRunCap;
+        const int lo = tbound[(int64_t)u * (tiles + 1) + tile];
+        int hi = tbound[(int64_t)u * (tiles + 1) + tile + 1];
+        hi = hi < len ? hi : len;
+        int pos[kRsItems] = {};
+        if (hi > lo)
+            for (int step = 1 << (31 - __clz(hi - lo)); step > 0; step >>= 1)
+#pragma unroll
+                for (int j = 0; j < kRsItems; ++j)
+                    if (lo + pos[j] + step <= hi &&
+                        below<kPair>(M.skey + b, M.sr0 + b, lo + pos[j] + step - 1, ko[j], (uint32_t)before[j]))
+                        pos[j] += step;
+#pragma unroll
+        for (int j = 0; j < kRsItems; ++j) c[j] += lo + pos[j];
+    }
+#pragma unroll
+    for (int j = 0; j < kRsItems; ++j) {
+        const int i = item_slot(base, j), pos = i - before[j] + c[j];
+        if (i >= n || ((bits >> j) & 1u) || pos < 0 || pos >= n) continue;
+        okeys[pos] = ko[j];
+        perm[pos] = (uint32_t)i;
+    }
+}
 // both placements in one launch, where the tiles' bounds came with the sort
 // of the movers (k_mover_sort): workgroups [0, tiles) the stayers' tiles, the
-// rest the movers
+// rest the movers; with more than one run every workgroup takes movers
 __global__ __launch_bounds__(kRsThreads) void k_place(MoverSet M, const uint32_t* __restrict__ cur, const int* m_dev,
                                                       const int* __restrict__ toff, const int* __restrict__ tbound,
                                                       int tiles, OldTables tb, bool use_tables,
@@ -726,34 +804,39 @@ __global__ __launch_bounds__(kRsThreads) void k_place(MoverSet M, const uint32_t
     __shared__ StayerLds sm;
     int m = *m_dev;
     m = m < M.n ? m : M.n;
-    if ((int)blockIdx.x < tiles)
-        place_stayers(M, cur, m, (int)blockIdx.x, toff, tbound, okeys, perm, sm);
-    else
-        place_movers(M, m, (int)((blockIdx.x - tiles) * blockDim.x + threadIdx.x),
-                     (int)((gridDim.x - tiles) * blockDim.x), tb, use_tables, okeys, perm);
+    const int wg = (int)blockIdx.x, all = (int)(gridDim.x * blockDim.x);
+    if (m > kRunCap) {
+        if (wg < tiles) place_stayers_runs(M, cur, m, wg, tiles, toff, tbound, okeys, perm, sm.lds4);
+        place_movers<true>(M, m, wg * (int)blockDim.x + (int)threadIdx.x, all, tb, use_tables, okeys, perm, tbound,
+                           tiles);
+    } else if (wg < tiles) {
+        place_stayers(M, cur, m, wg, toff, tbound, okeys, perm, sm);
+    } else {
+        place_movers<false>(M, m, (wg - tiles) * (int)blockDim.x + (int)threadIdx.x, all - tiles * (int)blockDim.x, tb,
+                            use_tables, okeys, perm, tbound, tiles);
+    }
 }
 
-// ---- few movers: the whole sort in one workgroup ----
+// ---- the movers' sort in runs ----
 // The general path takes 3 launches per digit, each a few microseconds of
-// dependent launch latency for a few thousand keys; one workgroup of 16 waves
-// sorts up to kMsCap movers in registers and LDS instead.  Wave w owns items
+// dependent launch latency for a few thousand keys; here a workgroup of 16
+// waves sorts kRunCap movers in registers and LDS.  Wave w owns items
 // [64 w per, 64 (w + 1) per), per = items per thread, so (wave, round, lane)
 // order is index order; it ranks its items with private digit counters (peers
 // by eight ballots, no barriers), the counters are scanned digit-major over
-// the waves, and the items change places through LDS.  Larger counts, which
-// the caller's last published count did not foresee, go through the same
-// ranking tile by tile with the passes' output in global memory: slow, and
-// the next sort takes the general path.  list is one of the output buffers
-// (kb0 or kb1): the first pass reads it before anything overwrites it.
-// Finally each tile of slots gets the sorted movers that precede its first
-// slot (tbound), by search.
+// the waves, and the items change places through LDS.  Workgroup u sorts
+// movers [u kRunCap, (u + 1) kRunCap) into a run of their own and leaves at
+// once where the list ends before them; k_place merges the runs by searching
+// each of them between the bounds of a tile of slots.  Those bounds, the sorted
+// movers of the run that precede each tile's first slot (tbound[run][tile]), are
+// found here.  The host need not know the count.
 constexpr int kMsThreads = 1024;
 constexpr int kMsItems = 16;
-constexpr int kMsCap = kMsThreads * kMsItems;
+static_assert(kMsThreads * kMsItems == kRunCap, "a run per workgroup");
 struct MsLds {
-    uint32_t key[kMsCap], val[kMsCap];
+    uint32_t key[kRunCap], val[kRunCap];
     uint32_t wcnt[kMsThreads / 64][256];
-    uint32_t base[256], run[256];
+    uint32_t base[256];
     int lds4[4];
 };
 // the wave's LDS writes before it are seen by all its lanes after it (the
@@ -821,109 +904,67 @@ __device__ __forceinline__ void ms_scan256(MsLds& L, int v) {
     }
     __syncthreads();
 }
-__global__ __launch_bounds__(kMsThreads) void k_mover_sort(const uint32_t* list, const int* m_dev, int n,
-                                                           int passes, uint32_t* kb0, uint32_t* vb0, uint32_t* kb1,
-                                                           uint32_t* vb1, const uint32_t* __restrict__ old,
+__global__ __launch_bounds__(kMsThreads) void k_mover_sort(const uint32_t* __restrict__ list, const int* m_dev, int n,
+                                                           int passes, uint32_t* __restrict__ okey,
+                                                           uint32_t* __restrict__ oidx,
+                                                           const uint32_t* __restrict__ old,
                                                            const int* __restrict__ toff, int tiles,
                                                            int* __restrict__ tbound) {
     __shared__ MsLds L;
     int m = *m_dev;
     m = m < n ? m : n;
+    const int b0 = (int)blockIdx.x * kRunCap;
+    if (b0 > 0 && b0 >= m) return;   // the first workgroup stays: the tiles' bounds are zero without movers
+    m = m - b0 < kRunCap ? m - b0 : kRunCap;
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
     uint32_t k[kMsItems], v[kMsItems], rank[kMsItems];
-    const bool small = m <= kMsCap;
-    if (small) {
-        const int per = (m + kMsThreads - 1) / kMsThreads, first = w * 64 * per;
+    const int per = (m + kMsThreads - 1) / kMsThreads, first = w * 64 * per;
 #pragma unroll
-        for (int r = 0; r < kMsItems; ++r) {
-            const int i = first + r * 64 + lane;
-            const bool in = r < per && i < m;
-            k[r] = in ? list[i] : 0u;
-            v[r] = (uint32_t)i;
-        }
-        for (int p = 0; p < passes; ++p) {
-            ms_rank(k, rank, per, first, m, 8 * p, L.wcnt[w]);
-            __syncthreads();
-            int mine;
-            ms_offsets(L, mine);
-            ms_scan256(L, mine);
+    for (int r = 0; r < kMsItems; ++r) {
+        const int i = first + r * 64 + lane;
+        const bool in = r < per && i < m;
+        k[r] = in ? list[b0 + i] : 0u;
+        v[r] = (uint32_t)(b0 + i);
+    }
+    for (int p = 0; p < passes; ++p) {
+        ms_rank(k, rank, per, first, m, 8 * p, L.wcnt[w]);
+        __syncthreads();
+        int mine;
+        ms_offsets(L, mine);
+        ms_scan256(L, mine);
 #pragma unroll
-            for (int r = 0; r < kMsItems; ++r)
-                if (r < per && first + r * 64 + lane < m) {
-                    const uint32_t d = (k[r] >> (8 * p)) & 255u;
-                    const uint32_t pos = L.base[d] + L.wcnt[w][d] + rank[r];
-                    L.key[pos] = k[r];
-                    L.val[pos] = v[r];
-                }
-            __syncthreads();
-            if (p + 1 < passes) {
-#pragma unroll
-                for (int r = 0; r < kMsItems; ++r) {
-                    const int i = first + r * 64 + lane;
-                    if (r < per && i < m) {
-                        k[r] = L.key[i];
-                        v[r] = L.val[i];
-                    }
-                }
-                __syncthreads();
+        for (int r = 0; r < kMsItems; ++r)
+            if (r < per && first + r * 64 + lane < m) {
+                const uint32_t d = (k[r] >> (8 * p)) & 255u;
+                const uint32_t pos = L.base[d] + L.wcnt[w][d] + rank[r];
+                L.key[pos] = k[r];
+                L.val[pos] = v[r];
             }
-        }
-        for (int i = tid; i < m; i += kMsThreads) {
-            kb1[i] = L.key[i];
-            vb1[i] = L.val[i];
-        }
-    } else {
-        for (int p = 0; p < passes; ++p) {
-            const int o = (passes - 1 - p) % 2 == 0 ? 1 : 0;   // the last pass writes kb1, vb1
-            const uint32_t* ki = p == 0 ? list : (o ? kb0 : kb1);
-            const uint32_t* vi = o ? vb0 : vb1;
-            uint32_t* ko = o ? kb1 : kb0;
-            uint32_t* vo = o ? vb1 : vb0;
-            // digit starts of the whole list
-            if (tid < 256) L.run[tid] = 0u;
-            __syncthreads();
-            for (int i = tid; i < m; i += kMsThreads) atomicAdd(&L.run[(ki[i] >> (8 * p)) & 255u], 1u);
-            __syncthreads();
-            ms_scan256(L, tid < 256 ? (int)L.run[tid] : 0);
-            for (int t0 = 0; t0 < m; t0 += kMsCap) {
-                const int cnt = m - t0 < kMsCap ? m - t0 : kMsCap;
-                const int per = (cnt + kMsThreads - 1) / kMsThreads, first = w * 64 * per;
+        __syncthreads();
+        if (p + 1 < passes) {
 #pragma unroll
-                for (int r = 0; r < kMsItems; ++r) {
-                    const int i = first + r * 64 + lane;
-                    const bool in = r < per && i < cnt;
-                    k[r] = in ? ki[t0 + i] : 0u;
-                    v[r] = in ? (p == 0 ? (uint32_t)(t0 + i) : vi[t0 + i]) : 0u;
+            for (int r = 0; r < kMsItems; ++r) {
+                const int i = first + r * 64 + lane;
+                if (r < per && i < m) {
+                    k[r] = L.key[i];
+                    v[r] = L.val[i];
                 }
-                ms_rank(k, rank, per, first, cnt, 8 * p, L.wcnt[w]);
-                __syncthreads();
-                int mine;
-                ms_offsets(L, mine);
-                __syncthreads();
-#pragma unroll
-                for (int r = 0; r < kMsItems; ++r)
-                    if (r < per && first + r * 64 + lane < cnt) {
-                        const uint32_t d = (k[r] >> (8 * p)) & 255u;
-                        const uint32_t pos = L.base[d] + L.wcnt[w][d] + rank[r];
-                        ko[pos] = k[r];
-                        vo[pos] = v[r];
-                    }
-                __syncthreads();
-                if (tid < 256) L.base[tid] += (uint32_t)mine;
-                __syncthreads();
             }
+            __syncthreads();
         }
     }
-    __syncthreads();
-    const uint32_t* sk = small ? L.key : kb1;
-    const uint32_t* sv = small ? L.val : vb1;
+    for (int i = tid; i < m; i += kMsThreads) {
+        okey[b0 + i] = L.key[i];
+        oidx[b0 + i] = L.val[i];
+    }
+    tbound += (int64_t)blockIdx.x * (tiles + 1);
     for (int t = tid; t <= tiles; t += kMsThreads) {
         int a = 0, b = m;
         if (t < tiles) {
             const uint32_t K = old[t * kRsTile], r0 = (uint32_t)toff[t];
             while (a < b) {
                 const int mid = (a + b) >> 1;
-                if (below<kPair>(sk, sv, mid, K, r0)) a = mid + 1;
+                if (below<kPair>(L.key, L.val, mid, K, r0)) a = mid + 1;
                 else b = mid;
             }
         } else {
@@ -1071,21 +1112,29 @@ static hipError_t sort_radix(mpmx_ctx* c) {
 static hipError_t sort_movers(mpmx_ctx* c) {
     const int n = (int)c->n;
     const int tiles = c->sort_tiles;
+    // In runs or by radix passes, whole sort in us (a lattice in flight; share of
+    // the particles that change cell 0.5 / 5 / 20 / 100 %): 64,000 particles 34 / 43 /
+    // 67 / 110 and 80 / 97 / 114 / 90, 512,000 38 / 79 / 97 / 164 and 83 / 101 / 106 /
+    // 104, 1,728,000 66 / 105 / 135 / 358 and 115 / 130 / 139 / 174, 2,097,152 74 /
+    // 108 / 147 / 488 and 113 / 124 / 148 / 181.  Above a quarter every key is sorted
+    // anyway (choose_sort_path); the merge grows with movers times runs, so not
+    // beyond 2,097,152 particles.
+    const bool runs = n <= kRunsMaxParticles;
     k_mover_count<<<tiles, kRsThreads, 0, c->stream>>>(c->keys, c->keys_next, n, c->mv_tcount);
-    // the movers' radix passes end in mv_key[1] / mv_val[1]; the list goes
-    // to the buffer that the first pass does not write
+    // the sorted movers go to mv_key[1] / mv_val[1]; the list to the buffer that
+    // the first pass of the radix sort does not write, or that the runs do not
     const int passes = (c->key_bits + 7) / 8;
-    uint32_t* const list = c->mv_key[(passes - 1) % 2 == 0 ? 0 : 1];
+    uint32_t* const list = c->mv_key[runs || (passes - 1) % 2 == 0 ? 0 : 1];
     k_mover_list<<<tiles, kRsThreads, 0, c->stream>>>(c->keys, c->keys_next, n, c->mv_tcount, c->mv_toff,
                                                       &c->dc->movers, list, c->mv_old, c->mv_slot, c->mv_cpre,
                                                       c->mv_cmask);
     const OldTables tb{c->pmask, c->wcount, c->page2particle, c->cell_start, &c->dc->num_page, c->cap_p};
     const MoverSet M{c->keys, n, c->mv_key[1], c->mv_val[1], c->mv_old, c->mv_slot, c->mv_cpre, c->mv_cmask};
-    if (c->few_movers) {
-        k_mover_sort<<<1, kMsThreads, 0, c->stream>>>(list, &c->dc->movers, n, passes, c->mv_key[0], c->mv_val[0],
-                                                      c->mv_key[1], c->mv_val[1], c->keys, c->mv_toff, tiles,
-                                                      c->mv_tbound);
-        const int mwg = std::max(1, std::min(tiles, kMsCap / kRsThreads));
+    if (runs) {
+        k_mover_sort<<<most_runs(n), kMsThreads, 0, c->stream>>>(list, &c->dc->movers, n, passes, c->mv_key[1],
+                                                                 c->mv_val[1], c->keys, c->mv_toff, tiles,
+                                                                 c->mv_tbound);
+        const int mwg = std::max(1, std::min(tiles, kRunCap / kRsThreads));
         k_place<<<tiles + mwg, kRsThreads, 0, c->stream>>>(M, c->keys_next, &c->dc->movers, c->mv_toff, c->mv_tbound,
                                                            tiles, tb, c->tables_match_keys, c->keys_alt, c->vals_alt);
         c->gather_perm = c->vals_alt;
@@ -1106,18 +1155,8 @@ static hipError_t sort_movers(mpmx_ctx* c) {
     return hipGetLastError();
 }
 
-// Which path the next sort takes.  few_movers: the movers' own sort in one
-// workgroup, where the last published count (or n itself) leaves room for
-// growth by a third up to its capacity; a count not published yet (-1, the
-// first sorts after an upload) is taken as large unless n is small.  A count
-// that jumps past the capacity (a lattice crossing its cells at once) takes that
-// workgroup about 10 ns a mover, 6 ms on the 8M impact: so not above 2,097,152
-// particles, and after such a jump not for as many sorts as make up for it.
+// Which path the next sort takes.
 void choose_sort_path(mpmx_ctx* c) {
-    const int64_t now = c->sorts + c->substeps;
-    if (c->few_movers && c->hc->movers > kMsCap) c->few_after = now + 64 * std::max<int64_t>(1, c->n >> 18);
-    const int64_t bound = c->hc->movers < 0 ? c->n : std::min<int64_t>(c->n, (int64_t)c->hc->movers * 4 / 3);
-    c->few_movers = bound <= kMsCap && (c->n <= kMsCap || (c->n <= (1 << 21) && now >= c->few_after));
     if (c->cfg.sort_variant != 0) {
         c->sort_by_movers = c->cfg.sort_variant == 2;
         return;
@@ -1133,7 +1172,6 @@ void choose_sort_path(mpmx_ctx* c) {
 // sort's keys, so the first sort after an upload takes the radix path.
 hipError_t sort_keys(mpmx_ctx* c) {
     choose_sort_path(c);
-    ++c->sorts;
     const bool movers = c->sort_by_movers && c->old_keys_sorted;
     hipError_t e = movers ? sort_movers(c) : sort_radix(c);
     if (e != hipSuccess) return e;

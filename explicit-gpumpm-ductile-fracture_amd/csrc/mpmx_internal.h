@@ -37,6 +37,12 @@
 
 namespace mpmx {
 
+// The movers' sort in runs (k_mover_sort): movers per run, the particles up to
+// which it is used, and its runs if every particle moves
+constexpr int kRunCap = 16384;
+constexpr int64_t kRunsMaxParticles = 1 << 21;
+constexpr int most_runs(int64_t n) { return n <= kRunsMaxParticles ? (int)((n + kRunCap - 1) / kRunCap) : 1; }
+
 constexpr int kGridCh = 8;       // channels per page in the grid slab
 constexpr int kPageFloats = kGridCh * 64;
 constexpr int kTile = 6;         // 6^3 node tile of one page's particles
@@ -227,11 +233,9 @@ struct mpmx_ctx {
     uint32_t* mv_slot = nullptr;
     bool sort_by_movers = true;   // the path the next sort takes (mpmx_config.sort_variant 0: from
                                   // the last published mover count)
-    bool few_movers = false;      // the movers are few enough for the one-workgroup sort
-    int64_t sorts = 0, few_after = 0;   // sorts made; sorts + substeps from which few_movers may be set again
     bool old_keys_sorted = false; // keys holds a sort's output (the mover path's precondition)
     bool tables_match_keys = false;   // the page tables were built from keys (the mover path uses them)
-    int* mv_tbound = nullptr;     // [sort_tiles + 1] sorted movers before each tile's first slot
+    int* mv_tbound = nullptr;     // [most_runs][sort_tiles + 1] sorted movers (of each run) before each tile's first slot
     int* mv_cpre = nullptr;       // [n / 64 + 1] movers before each 64-slot chunk
     uint64_t* mv_cmask = nullptr; // [n / 64 + 1] movers of each chunk
     // keys of the particles in their current slots
@@ -284,7 +288,6 @@ struct mpmx_ctx {
         int iters = 0;
         int64_t blocks = 0;
         bool by_movers = false;   // the sort path captured
-        bool few_movers = false;
     } graphs[2];
     int cg_recent[8] = {0, 0, 0, 0, 0, 0, 0, 0};   // PCG iterations of the last substeps
     int* bcount = nullptr;           // [mask_words] per-word block counts, then their scan

@@ -1,0 +1,110 @@
+"""The movers' sort in runs: the order of the radix sort at its largest particle
+count (128 runs when every particle moves) and past it, and a bounded cost: the
+count of movers may jump, or grow inside one long call without a solve (whose
+substeps the host never looks at), or come and go in captured substeps.
+
+The times are compared with the radix sort of every key in the same scene;
+both sides were measured before the limits were set: the sort in runs takes 1.1,
+3.0 and 0.9 times as long, one that goes by an old count 4.3, 50 and 2.8 times."""
+import time
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+DT = 1e-3
+
+
+def lattice(mpmx, edge, N, jitter, n=None):
+    """A corotated block of edge^3 cells, eight particles each, at rest."""
+    rng = np.random.default_rng(1)
+    g = np.stack(np.meshgrid(*[np.arange(2 * edge)] * 3, indexing="ij"), -1).reshape(-1, 3)[:n]
+    x = (N // 2 - edge // 2 + (g + 0.5) * 0.5 + rng.uniform(-jitter, jitter, g.shape)) / N
+    p = mpmx.default_params(N=N, model=0, E=100.0, nu=0.3, V0=0.125 / N ** 3, gravity=(0.0, 0.0, 0.0))
+    return p, x.astype(np.float32).astype(np.float64), np.full(len(x), 125.0 / N ** 3)
+
+
+def fly(ctx, cells, N):
+    """cells per substep along x, free of stress"""
+    ctx.set("v", np.tile([cells / N / DT, 0.0, 0.0], (ctx.n, 1)))
+    ctx.set("B", np.zeros((ctx.n, 3, 3)))
+    ctx.set("F", np.tile(np.eye(3), (ctx.n, 1, 1)))
+
+
+def resting(mpmx, scene, variant, graph=0):
+    p, x, m = scene
+    ctx = mpmx.Context(p, mpmx.default_config(sort_variant=variant, use_graph=graph))
+    ctx.set_particles(x, np.zeros_like(x), m)
+    ctx.run(4, DT)
+    ctx.sync()
+    return ctx
+
+
+@pytest.mark.parametrize("n", [2097152, 2097153])
+def test_order_of_many_runs(mpmx, n):
+    scene = lattice(mpmx, 65, 256, 0.24, n)
+    for cells in (0.1, 1.0):
+        got = []
+        for variant in (1, 2):
+            ctx = resting(mpmx, scene, variant)
+            fly(ctx, cells, 256)
+            ctx.run(2, DT)
+            ctx.bin_sort()
+            got.append(ctx.order())
+            ctx.close()
+        assert np.array_equal(got[0][1], got[1][1]), cells
+        assert np.array_equal(got[0][0], got[1][0]), cells
+
+
+def test_cost_when_no_count_is_published(mpmx):
+    """30 substeps in one call, a quarter of the particles moving in each."""
+    scene = lattice(mpmx, 50, 256, 0.24)
+    best = {}
+    for variant in (1, 2):
+        for _ in range(2):
+            ctx = resting(mpmx, scene, variant)
+            fly(ctx, 0.25, 256)
+            ctx.sync()
+            t0 = time.perf_counter()
+            ctx.run(30, DT)
+            ctx.sync()
+            best[variant] = min(best.get(variant, 1e9), time.perf_counter() - t0)
+            ctx.close()
+    assert best[2] < 2 * best[1], best
+
+
+def test_cost_of_a_jump(mpmx):
+    """Every particle changes cell in one substep, none did before."""
+    scene = lattice(mpmx, 50, 256, 0.24)
+    best = {}
+    for variant in (1, 2):
+        for _ in range(2):
+            ctx = resting(mpmx, scene, variant)
+            fly(ctx, 1.0, 256)
+            ctx.run(1, DT)
+            ctx.timing_begin()
+            ctx.run(1, DT)
+            best[variant] = min(best.get(variant, 1e9), ctx.timing_end()["sort"][1])
+            ctx.close()
+    assert best[2] < 8 * best[1], best
+
+
+def test_captured_substeps_with_bursts_of_movers(mpmx):
+    """A lattice without jitter changes cells in bursts, 13,500 of 27,000 particles
+    every third substep and none between: the captured substeps stay."""
+    scene = lattice(mpmx, 15, 128, 0.0)
+    best, x = {}, {}
+    for variant in (1, 2):
+        for _ in range(2):
+            ctx = resting(mpmx, scene, variant, graph=1)
+            fly(ctx, 0.17, 128)
+            ctx.run(8, DT)
+            ctx.sync()
+            t0 = time.perf_counter()
+            ctx.run(100, DT)
+            ctx.sync()
+            best[variant] = min(best.get(variant, 1e9), time.perf_counter() - t0)
+            x[variant] = ctx.get("x")
+            ctx.close()
+    assert np.array_equal(x[1], x[2])
+    assert best[2] < 2 * best[1], best
