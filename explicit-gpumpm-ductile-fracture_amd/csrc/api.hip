@@ -432,7 +432,7 @@ static void free_particles(mpmx_ctx* c) {
         dfree(m.mass); dfree(m.id);
     }
     dfree(c->sigma); dfree(c->FP); dfree(c->vol); dfree(c->cg_col); dfree(c->payload); dfree(c->pbound); dfree(c->cbound);
-    dfree(c->keys); dfree(c->keys_alt); dfree(c->keys_next); dfree(c->vals); dfree(c->vals_alt); dfree(c->hist); dfree(c->hist2);
+    dfree(c->keys); dfree(c->keys_alt); dfree(c->keys_next); dfree(c->vals); dfree(c->vals_alt); dfree(c->hist);
     dfree(c->mv_tcount); dfree(c->mv_toff); dfree(c->mv_old); dfree(c->mv_slot);
     dfree(c->mv_tbound); dfree(c->mv_cpre); dfree(c->mv_cmask);
     for (int b = 0; b < 2; ++b) { dfree(c->mv_key[b]); dfree(c->mv_val[b]); }
@@ -808,7 +808,6 @@ static mpmx_status upload_particles(mpmx_ctx* c, const int64_t* counts, const st
     HIPCHK(c, dalloc(&c->vals_alt, n));
     c->sort_tiles = (int)((n + 2047) / 2048);
     HIPCHK(c, dalloc(&c->hist, (int64_t)256 * c->sort_tiles));
-    HIPCHK(c, dalloc(&c->hist2, (int64_t)256 * c->sort_tiles));
     HIPCHK(c, dalloc(&c->mv_tcount, c->sort_tiles));
     HIPCHK(c, dalloc(&c->mv_toff, c->sort_tiles));
     HIPCHK(c, dalloc(&c->mv_old, n));

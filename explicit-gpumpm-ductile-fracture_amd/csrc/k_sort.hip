@@ -153,42 +153,6 @@ hipError_t scan_exclusive(mpmx_ctx* c, const int* in, int* out, int64_t n_cap, c
     return hipGetLastError();
 }
 
-// One launch, out of place, for a device count of a few dozen tiles: every tile
-// adds up all entries before it itself (16-byte loads, at most 32 per thread
-// for the last of 32 tiles) instead of waiting for a launch of tile sums.
-// Above that the sums' launch is the cheaper one (radix_passes).
-__global__ __launch_bounds__(256) void k_scan_direct(const int* __restrict__ in, int* __restrict__ out,
-                                                     const int* __restrict__ n_dev, int64_t cap) {
-    __shared__ int lds4[4];
-    int64_t n = *n_dev;
-    n = n < cap ? n : cap;
-    const int64_t base = (int64_t)blockIdx.x * kScanTile;
-    if (base >= n) return;
-    int pre = 0;
-    const int4* in4 = reinterpret_cast<const int4*>(in);   // base is a multiple of a tile
-#pragma unroll 4
-    for (int i = threadIdx.x; i < (int)(base >> 2); i += 256) {
-        const int4 q = in4[i];
-        pre += (q.x + q.y) + (q.z + q.w);
-    }
-    int offset, total;
-    (void)block_excl_scan256(pre, offset, lds4);
-    int v[kScanPer], local = 0;
-#pragma unroll
-    for (int q = 0; q < kScanPer; ++q) {
-        const int64_t i = base + (int64_t)threadIdx.x * kScanPer + q;
-        v[q] = (i < n) ? in[i] : 0;
-        local += v[q];
-    }
-    int off = block_excl_scan256(local, total, lds4) + offset;
-#pragma unroll
-    for (int q = 0; q < kScanPer; ++q) {
-        const int64_t i = base + (int64_t)threadIdx.x * kScanPer + q;
-        if (i < n) out[i] = off;
-        off += v[q];
-    }
-}
-
 // up to three scans of n entries each in the same two launches (in place
 // allowed); array y uses the tile sums at sums + y * tiles
 __global__ __launch_bounds__(256) void k_scan_reduce3(ScanSet3 a, int* sums, int64_t n) {
@@ -1061,26 +1025,16 @@ static hipError_t radix_passes(mpmx_ctx* c, const uint32_t* k_in, const uint32_t
                                uint32_t* const (&vb)[2], RsSize z, int grid, int* hist_n) {
     const int passes = (c->key_bits + 7) / 8;
     const int64_t hist_cap = (int64_t)256 * c->sort_tiles;
-    // a device count is scanned in one launch while the last published mover
-    // count keeps the histogram within 32 scan tiles: the 8M impact (570,000
-    // movers, 70 tiles) took 57 us a pass that way and takes 9 in two launches
-    const bool direct = z.n_dev && c->hc->movers >= 0 && c->hc->movers <= 32 * kScanTile / 256 * kRsTile;
-    uint32_t* const offs = direct ? c->hist2 : c->hist;
     const uint32_t* ki = k_in;
     const uint32_t* vi = vals_in;
     for (int p = 0; p < passes; ++p) {
         const int o = (passes - 1 - p) % 2 == 0 ? 1 : 0;
         k_radix_hist<<<grid, kRsThreads, 0, c->stream>>>(ki, z, 8 * p, c->hist, hist_n);
-        hipError_t e = hipSuccess;
-        if (direct)
-            k_scan_direct<<<(int)((hist_cap + kScanTile - 1) / kScanTile), 256, 0, c->stream>>>(
-                (const int*)c->hist, (int*)c->hist2, hist_n, hist_cap);
-        else
-            e = z.n_dev ? scan_exclusive(c, (const int*)c->hist, (int*)c->hist, hist_cap, hist_n, hist_cap, nullptr)
+        hipError_t e = z.n_dev ? scan_exclusive(c, (const int*)c->hist, (int*)c->hist, hist_cap, hist_n, hist_cap, nullptr)
                                : scan_exclusive(c, (const int*)c->hist, (int*)c->hist, (int64_t)256 * z.tiles,
                                                 nullptr, (int64_t)256 * z.tiles, nullptr);
         if (e != hipSuccess) return e;
-        k_radix_scatter<<<grid, kRsThreads, 0, c->stream>>>(ki, vi, kb[o], vb[o], z, 8 * p, offs);
+        k_radix_scatter<<<grid, kRsThreads, 0, c->stream>>>(ki, vi, kb[o], vb[o], z, 8 * p, c->hist);
         ki = kb[o];
         vi = vb[o];
     }

@@ -218,7 +218,6 @@ struct mpmx_ctx {
     uint32_t* vals = nullptr;
     uint32_t* vals_alt = nullptr;
     uint32_t* hist = nullptr;
-    uint32_t* hist2 = nullptr;   // scanned histogram of the movers' radix passes
     int sort_tiles = 0;
     int key_bits = 0;
     bool sorted = false;     // particles gathered to the order of `keys`
