@@ -645,14 +645,17 @@ mpmx_status mpmx_create_batch(int num_scenes, const mpmx_params* ps, const mpmx_
     }
     if (hipMalloc((void**)&c->dc, sizeof(DevCounts)) != hipSuccess ||
         hipHostMalloc((void**)&c->hc, sizeof(DevCounts), hipHostMallocDefault) != hipSuccess ||
-        hipHostMalloc((void**)&c->pub, sizeof(DevCounts), hipHostMallocCoherent) != hipSuccess) {
+        hipHostMalloc((void**)&c->pub, sizeof(DevCounts), hipHostMallocCoherent) != hipSuccess ||
+        hipHostMalloc((void**)&c->seen, 2 * sizeof(int), hipHostMallocCoherent) != hipSuccess) {
         if (c->dc) (void)hipFree(c->dc);
         if (c->hc) (void)hipHostFree(c->hc);
+        if (c->pub) (void)hipHostFree(c->pub);
         delete c;
         return MPMX_ERR_HIP;
     }
     std::memset(c->hc, 0, sizeof(DevCounts));
     std::memset(c->pub, 0, sizeof(DevCounts));
+    c->seen[0] = c->seen[1] = 0;
     (void)hipMemcpy(c->dc, c->hc, sizeof(DevCounts), hipMemcpyHostToDevice);
     if (hipMalloc((void**)&c->scene_dp, sizeof(DevParams) * num_scenes) != hipSuccess ||
         hipMalloc((void**)&c->scg, sizeof(SceneCG) * num_scenes) != hipSuccess ||
@@ -690,6 +693,7 @@ mpmx_status mpmx_destroy(mpmx_ctx* c) {
     if (c->dc) (void)hipFree(c->dc);
     if (c->hc) (void)hipHostFree(c->hc);
     if (c->pub) (void)hipHostFree(c->pub);
+    if (c->seen) (void)hipHostFree(c->seen);
     if (c->stream) (void)hipStreamDestroy(c->stream);
     delete c;
     return MPMX_OK;
@@ -874,7 +878,8 @@ static mpmx_status upload_particles(mpmx_ctx* c, const int64_t* counts, const st
     else k_upload_fp32<<<(int)((n + 255) / 256), 256, 0, c->stream>>>(c->ps[0], dx_, dv_, dm_, (int)n);
     HIPCHK(c, hipGetLastError());
     std::memset(c->hc, 0, sizeof(DevCounts));
-    c->hc->movers = -1;   // not counted yet
+    c->hc->movers = c->seen[0] = -1;   // not counted yet
+    c->seen[1] = 0;
     HIPCHK(c, hipMemcpyAsync(c->dc, c->hc, sizeof(DevCounts), hipMemcpyHostToDevice, c->stream));
     // keys, first canonical sort, first tables (with the bound as capacity)
     HIPCHK(c, compute_keys(c));
@@ -1045,8 +1050,7 @@ mpmx_status mpmx_substep(mpmx_ctx* c, double dt) {
 // afterwards; replays set it themselves.
 static mpmx_status capture_substep(mpmx_ctx* c, double dt, int iters) {
     const int p = c->cur;
-    choose_sort_path(c);
-    const bool by_movers = c->sort_by_movers && c->old_keys_sorted;   // the path sort_keys takes
+    const bool old_keys_sorted = c->old_keys_sorted;
     uint32_t* const keys0 = c->keys;
     uint32_t* const keys1 = c->keys_alt;
     auto& G = c->graphs[p];
@@ -1095,7 +1099,7 @@ static mpmx_status capture_substep(mpmx_ctx* c, double dt, int iters) {
     G.valid = true;
     G.dt = (float)dt;
     G.iters = iters;
-    G.by_movers = by_movers;
+    G.by_movers = c->sort_by_movers && old_keys_sorted;   // the path sort_keys took
     G.blocks = c->hc->num_blocks;
     return MPMX_OK;
 }

@@ -129,7 +129,7 @@ __global__ void k_page_keys(DevParams dp, const uint64_t* __restrict__ pmask, co
                             const int* __restrict__ wpre, const int* __restrict__ spre,
                             const int* __restrict__ bpre, int64_t words, int per, uint32_t* page_key, int64_t cap_p,
                             int64_t cap_tp, uint32_t* __restrict__ block_key, int64_t cap_blocks,
-                            SceneCG* __restrict__ scg, DevCounts* dc) {
+                            SceneCG* __restrict__ scg, int* __restrict__ seen, DevCounts* dc) {
     // a wave per `per` (<= 64) consecutive words: one lane per word finds the words that
     // hold a page (a batch's page space is mostly empty), then the wave takes
     // those words one at a time with one lane per bit: a set bit's id is the
@@ -145,6 +145,10 @@ __global__ void k_page_keys(DevParams dp, const uint64_t* __restrict__ pmask, co
         const int total = num_page + dc->num_supp;
         dc->num_total = total;
         if (num_page > cap_p || total > cap_tp) atomicOr(&dc->err, kErrCapacity);
+        if (seen) {   // host memory
+            __hip_atomic_store(&seen[0], dc->movers, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+            __hip_atomic_store(&seen[1], dc->num_blocks, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        }
     }
     if (t < dp.num_scenes) scene_counts_of(dp, (int)t, wpre, spre, scg, dc);
     const int64_t w0 = (t >> 6) * per;   // the wave's first word
@@ -362,7 +366,7 @@ hipError_t build_tables(mpmx_ctx* c) {
     const int per = words <= (1 << 17) ? 8 : 32;
     k_page_keys<<<(int)((words + 4 * per - 1) / (4 * per)), 256, 0, c->stream>>>(
         c->dp, c->pmask, c->nmask, c->wcount, c->scount, c->bcount, words, per, c->page_key, c->cap_p, c->cap_tp,
-        c->block_key, c->tp_bound, c->scg, c->dc);
+        c->block_key, c->tp_bound, c->scg, c->dp.phase_field ? nullptr : c->seen, c->dc);
     k_page_heads<<<(n + 256 * kHeadItems - 1) / (256 * kHeadItems), 256, 0, c->stream>>>(c->keys, n, c->pmask, c->nmask, c->wcount, c->scount,
                                                           c->page2particle, c->cell_start, c->cap_p, c->dc);
     c->vpages_valid = false;

@@ -314,6 +314,8 @@ struct mpmx_ctx {
     mpmx::DevCounts* hc = nullptr;   // pinned host mirror
     mpmx::DevCounts* pub = nullptr;  // coherent pinned copy the device publishes to (counts_to_host)
     unsigned pub_seq = 0;
+    int* seen = nullptr;             // coherent pinned: movers and blocks of the last table build that has run,
+                                     // for scenes without a solve, whose counts nothing else brings to the host
     // scans
     int* scan_tmp = nullptr;
     int64_t scan_tmp_cap = 0;
