@@ -373,6 +373,10 @@ __device__ __forceinline__ unsigned long long to_fix_scaled(float xs) {
 __device__ __forceinline__ unsigned long long to_fix_scaled_nonneg(float xs) {
     return (unsigned long long)(unsigned)(int)xs;
 }
+// the sum of two such integers in 32 bits: exact for terms of finite sources
+// (their weights leave room for two), while the term of an infinite one, the
+// largest integer, stays there instead of wrapping round to a small value
+__device__ __forceinline__ int add_fix(int a, int b) { return __builtin_elementwise_add_sat(a, b); }
 __device__ __forceinline__ float from_fix(unsigned long long v, int e) {
     return (float)ldexp((double)(long long)v, -e);
 }

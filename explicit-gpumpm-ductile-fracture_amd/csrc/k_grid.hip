@@ -185,7 +185,7 @@ __device__ __forceinline__ void p2g_fix(const P2GTerms (&T)[2], const int (&s)[3
                     }
                     const float v[kP2GCh] = {wt * t.m, pr[0], pr[1], pr[2], wt * t.cphase, wt * sc5, wt * t.V, wt * t.VF};
 #pragma unroll
-                    for (int k = 0; k < kP2GCh; ++k) add[k] = h == 0 ? (int)v[k] : add[k] + (int)v[k];
+                    for (int k = 0; k < kP2GCh; ++k) add[k] = h == 0 ? (int)v[k] : add_fix(add[k], (int)v[k]);
                 }
                 unsigned long long* a = acc + (ii * SX + jj * SY + kk);
                 // the weights are >= 0, so channel 5 needs no sign extension

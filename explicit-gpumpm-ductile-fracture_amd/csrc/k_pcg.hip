@@ -335,7 +335,7 @@ __device__ __forceinline__ void cgq_pair(const DevParams& sp, const ST& s, int i
                 if (kk >= cnt[2]) break;
                 int add = 0;
 #pragma unroll
-                for (int h = 0; h < 2; ++h) add += (int)fmaf(w[h][2][kk], rA[h], gw[h][2][kk] * rB[h]);
+                for (int h = 0; h < 2; ++h) add = add_fix(add, (int)fmaf(w[h][2][kk], rA[h], gw[h][2][kk] * rB[h]));
                 atomicAdd(az[kk] + (ii * A::kX + jj * A::kZ), (unsigned long long)(long long)add);
             }
         }
