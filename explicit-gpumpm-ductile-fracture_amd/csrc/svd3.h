@@ -289,7 +289,11 @@ __device__ __forceinline__ void jacobi_columns(double (&G)[3][3]) {
             const double a = fma(G[2][p], G[2][p], fma(G[1][p], G[1][p], G[0][p] * G[0][p]));
             const double b = fma(G[2][q], G[2][q], fma(G[1][q], G[1][q], G[0][q] * G[0][q]));
             const double c = fma(G[2][p], G[2][q], fma(G[1][p], G[1][q], G[0][p] * G[0][q]));
-            if (c * c > tol2 * (a * b)) {
+            // below 2^-48 of the other's length a column is rounding noise (of a
+            // matrix of lower rank): more rotations would only take it on to
+            // lengths far below that
+            const bool noise = abs(__double2hiint(a) - __double2hiint(b)) >= 96 << 20;
+            if (c * c > tol2 * (a * b) && !noise) {
                 // tan 2t = 2c / (b - a); cos t >= sqrt(1/2)
                 const double d = b - a, r = rsqrt_acc(fma(d, d, 4.0 * (c * c)));
                 const double h = fma(0.5 * fabs(d), r, 0.5), rh = rsqrt_acc(h);
@@ -360,9 +364,11 @@ __device__ __forceinline__ void across(const double (&u)[3], double (&v)[3]) {
 __device__ __forceinline__ double pick(const double (&x)[3], int i) { return i == 0 ? x[0] : (i == 1 ? x[1] : x[2]); }
 
 // where principal_axes returned false: the smallest singular value's directions,
-// u and v alike, completed to right-handed bases from the other two (of a lower
-// rank: any vectors across).  R as principal_axes left it (0 for S = 0); i is the
-// smallest, (i, j, k) cyclic.
+// u and v alike, completed to right-handed bases from the other two; of those the
+// smaller one's v orthogonal to the larger one's, or, where it too is rounding
+// noise of the larger (a lower rank: u not across the larger one's, or F^T u not
+// S long and across), any vectors across.  R as principal_axes left it (0 for S =
+// 0); i is the smallest, (i, j, k) cyclic.
 __device__ __forceinline__ void principal_axes_singular(const float (&F)[3][3], const double (&R)[3],
                                                         double (&U)[3][3], double (&V)[3][3]) {
     double S[3];
@@ -370,38 +376,52 @@ __device__ __forceinline__ void principal_axes_singular(const float (&F)[3][3], 
     for (int a = 0; a < 3; ++a) S[a] = R[a] != 0.0 ? 1.0 / fabs(R[a]) : 0.0;
     const int i = S[0] <= S[1] && S[0] <= S[2] ? 0 : (S[1] <= S[2] ? 1 : 2), j = i == 2 ? 0 : i + 1,
               k = j == 2 ? 0 : j + 1;
-    const double sj = pick(S, j), sk = pick(S, k);
-    double uj[3], uk[3], vj[3], vk[3], ui[3], vi[3];
-    double nj = 0.0, nk = 0.0;
+    const bool kl = pick(S, k) >= pick(S, j);   // k is the larger of the two
+    const double sl = pick(S, kl ? k : j), ss = pick(S, kl ? j : k);
+    double ul[3], us[3], vl[3], vs[3];
+    double nl = 0.0, ns = 0.0, d = 0.0, e = 0.0;
 #pragma unroll
     for (int r = 0; r < 3; ++r) {
-        uj[r] = pick(U[r], j);
-        uk[r] = pick(U[r], k);
+        ul[r] = pick(U[r], kl ? k : j);
+        us[r] = pick(U[r], kl ? j : k);
+    }
+    if (!(sl > 0.0)) {   // F = 0
+        ul[0] = 1.0;
+        ul[1] = ul[2] = 0.0;
     }
 #pragma unroll
     for (int c = 0; c < 3; ++c) {
-        vj[c] = F[0][c] * uj[0] + F[1][c] * uj[1] + F[2][c] * uj[2];
-        vk[c] = F[0][c] * uk[0] + F[1][c] * uk[1] + F[2][c] * uk[2];
-        nj += vj[c] * vj[c];
-        nk += vk[c] * vk[c];
+        vl[c] = sl > 0.0 ? F[0][c] * ul[0] + F[1][c] * ul[1] + F[2][c] * ul[2] : ul[c];
+        vs[c] = F[0][c] * us[0] + F[1][c] * us[1] + F[2][c] * us[2];
+        nl += vl[c] * vl[c];
     }
-    nj = rsqrt_acc(nj);
-    nk = rsqrt_acc(nk);
+    nl = rsqrt_acc(nl);
 #pragma unroll
     for (int c = 0; c < 3; ++c) {
-        vj[c] *= nj;
-        vk[c] *= nk;
+        vl[c] *= nl;
+        d += vs[c] * vl[c];
+        e += us[c] * ul[c];
     }
-    if (!(sj > 0.0 || sk > 0.0)) {
-        uj[0] = vj[0] = 1.0;
-        uj[1] = uj[2] = vj[1] = vj[2] = 0.0;
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+        vs[c] -= d * vl[c];
+        ns += vs[c] * vs[c];
     }
-    if (!(sk > 0.0)) {
-        across(uj, uk);
-        across(vj, vk);
-    } else if (!(sj > 0.0)) {
-        across(uk, uj);
-        across(vk, vj);
+    if (fabs(e) < 1e-10 && fabs(d) <= 1e4 * ss && ns > 0.25 * (ss * ss)) {
+        ns = rsqrt_acc(ns);
+#pragma unroll
+        for (int c = 0; c < 3; ++c) vs[c] *= ns;
+    } else {
+        across(ul, us);
+        across(vl, vs);
+    }
+    double uj[3], uk[3], vj[3], vk[3], ui[3], vi[3];
+#pragma unroll
+    for (int r = 0; r < 3; ++r) {
+        uj[r] = kl ? us[r] : ul[r];
+        uk[r] = kl ? ul[r] : us[r];
+        vj[r] = kl ? vs[r] : vl[r];
+        vk[r] = kl ? vl[r] : vs[r];
     }
     ui[0] = uj[1] * uk[2] - uj[2] * uk[1];
     ui[1] = uj[2] * uk[0] - uj[0] * uk[2];
