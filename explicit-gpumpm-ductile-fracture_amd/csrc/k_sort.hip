@@ -414,9 +414,9 @@ __device__ __forceinline__ uint64_t spread4(uint64_t x) {
 // the movers in slot order: new key, previous key, slot; per 64 slots, the
 // movers before them (cpre) and which of them move (cmask), so that the movers
 // before any slot s are cpre[s / 64] + popcount(cmask[s / 64] below bit s %
-// 64).  Each tile adds up the counts of the tiles before it itself (toff keeps
-// the sum; a few loads per thread even at 13 M particles) instead of waiting
-// for two scan launches; the last tile leaves the total in *m_dev.
+// 64).  With tcount set each tile adds up the counts of the tiles before it
+// itself (toff keeps the sum) instead of waiting for two scan launches, and the
+// last tile leaves the total in *m_dev; without, toff holds the sums already.
 __global__ __launch_bounds__(kRsThreads) void k_mover_list(const uint32_t* __restrict__ old,
                                                            const uint32_t* __restrict__ cur, int n,
                                                            const int* __restrict__ tcount, int* __restrict__ toff,
@@ -428,11 +428,15 @@ __global__ __launch_bounds__(kRsThreads) void k_mover_list(const uint32_t* __res
     const int base = blockIdx.x * kRsTile;
     const unsigned bits = mover_bits(old, cur, base, n, ko, kn);
     int pre = 0, before;
-    for (int t = threadIdx.x; t < (int)blockIdx.x; t += kRsThreads) pre += tcount[t];
-    (void)block_excl_scan256(pre, before, lds4);
+    if (tcount) {
+        for (int t = threadIdx.x; t < (int)blockIdx.x; t += kRsThreads) pre += tcount[t];
+        (void)block_excl_scan256(pre, before, lds4);
+    } else {
+        before = toff[blockIdx.x];
+    }
     int mr[2], total;
     half_ranks(bits, before, mr, total, lds4);
-    if (threadIdx.x == 0) {
+    if (tcount && threadIdx.x == 0) {
         toff[blockIdx.x] = before;
         if (blockIdx.x == gridDim.x - 1) *m_dev = before + total;
     }
@@ -1079,9 +1083,18 @@ static hipError_t sort_movers(mpmx_ctx* c) {
     // the first pass of the radix sort does not write, or that the runs do not
     const int passes = (c->key_bits + 7) / 8;
     uint32_t* const list = c->mv_key[runs || (passes - 1) % 2 == 0 ? 0 : 1];
-    k_mover_list<<<tiles, kRsThreads, 0, c->stream>>>(c->keys, c->keys_next, n, c->mv_tcount, c->mv_toff,
-                                                      &c->dc->movers, list, c->mv_old, c->mv_slot, c->mv_cpre,
-                                                      c->mv_cmask);
+    // the sums over the tiles in the list kernel grow with their square: whole
+    // sort with them and with a scan of two launches, 2 % of the particles moving,
+    // 8,000,000 particles 187 / 187 us, 13,144,256 251 / 247, 32,768,000 498 / 465,
+    // 128,024,064 1,960 / 1,590
+    const bool scan = tiles > 4096;
+    if (scan) {
+        hipError_t e = scan_exclusive(c, c->mv_tcount, c->mv_toff, tiles, nullptr, tiles, &c->dc->movers);
+        if (e != hipSuccess) return e;
+    }
+    k_mover_list<<<tiles, kRsThreads, 0, c->stream>>>(c->keys, c->keys_next, n, scan ? nullptr : c->mv_tcount,
+                                                      c->mv_toff, &c->dc->movers, list, c->mv_old, c->mv_slot,
+                                                      c->mv_cpre, c->mv_cmask);
     const OldTables tb{c->pmask, c->wcount, c->page2particle, c->cell_start, &c->dc->num_page, c->cap_p};
     const MoverSet M{c->keys, n, c->mv_key[1], c->mv_val[1], c->mv_old, c->mv_slot, c->mv_cpre, c->mv_cmask};
     if (runs) {
