@@ -153,7 +153,8 @@ __device__ __forceinline__ void neo_hookean(const DevParams& dp, const StressIn&
     out.alpha = in.alpha;
     const T J = S[0] * S[1] * S[2];
     const T ln_J = log(J);
-    const T J_bar = exp(-T(2.0f / 3.0f) * ln_J);
+    // FP64: from the logarithm at hand; FP32: pow, whose result is the closer one
+    const T J_bar = std::is_same<T, float>::value ? pow(J, -T(2.0f / 3.0f)) : exp(-T(2.0f / 3.0f) * ln_J);
     T be[3];
 #pragma unroll
     for (int a = 0; a < 3; ++a) be[a] = J_bar * S[a] * S[a];
