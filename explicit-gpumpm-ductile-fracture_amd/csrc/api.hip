@@ -201,12 +201,14 @@ int particle_blocks(const mpmx_ctx* c) {
 
 // the captured substeps no longer match the context (buffers, capacities or
 // launch shapes changed)
+static void destroy_graph(mpmx_ctx::SubstepGraph& g) {
+    if (g.a) (void)hipGraphExecDestroy(g.a);
+    if (g.b) (void)hipGraphExecDestroy(g.b);
+    g = mpmx_ctx::SubstepGraph{};
+}
 void destroy_graphs(mpmx_ctx* c) {
-    for (auto& g : c->graphs) {
-        if (g.a) (void)hipGraphExecDestroy(g.a);
-        if (g.b) (void)hipGraphExecDestroy(g.b);
-        g = mpmx_ctx::SubstepGraph{};
-    }
+    for (auto& parity : c->graphs)
+        for (auto& g : parity) destroy_graph(g);
 }
 
 void note_cg_iters(mpmx_ctx* c, int iters) {
@@ -1046,17 +1048,15 @@ mpmx_status mpmx_substep(mpmx_ctx* c, double dt) {
 // Captures the substep that starts from the current parity (particles
 // unsorted in buffer c->cur) as graph A (sort, tables, stress, P2G + grid
 // update, `iters` PCG iterations, the counter copy to the host) and graph B
-// (G2P).  The host-side state the stages update during capture is put back
-// afterwards; replays set it themselves.
-static mpmx_status capture_substep(mpmx_ctx* c, double dt, int iters) {
+// (G2P), kept by parity and the sort path that was captured (kept: where).  The
+// host-side state the stages update during capture is put back afterwards;
+// replays set it themselves.
+static mpmx_status capture_substep(mpmx_ctx* c, double dt, int iters, mpmx_ctx::SubstepGraph** kept) {
     const int p = c->cur;
     const bool old_keys_sorted = c->old_keys_sorted;
     uint32_t* const keys0 = c->keys;
     uint32_t* const keys1 = c->keys_alt;
-    auto& G = c->graphs[p];
-    if (G.a) (void)hipGraphExecDestroy(G.a);
-    if (G.b) (void)hipGraphExecDestroy(G.b);
-    G = mpmx_ctx::SubstepGraph{};
+    mpmx_ctx::SubstepGraph G;
     hipGraph_t ga = nullptr, gb = nullptr;
     mpmx_status s = MPMX_OK;
     HIPCHK(c, hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
@@ -1091,16 +1091,16 @@ static mpmx_status capture_substep(mpmx_ctx* c, double dt, int iters) {
     c->gather_perm = nullptr;
     c->vb_perm = nullptr;
     if (s != MPMX_OK) {
-        if (G.a) (void)hipGraphExecDestroy(G.a);
-        if (G.b) (void)hipGraphExecDestroy(G.b);
-        G = mpmx_ctx::SubstepGraph{};
+        destroy_graph(G);
         return s;
     }
     G.valid = true;
     G.dt = (float)dt;
     G.iters = iters;
-    G.by_movers = c->sort_by_movers && old_keys_sorted;   // the path sort_keys took
     G.blocks = c->hc->num_blocks;
+    *kept = &c->graphs[p][c->sort_by_movers && old_keys_sorted ? 1 : 0];
+    destroy_graph(**kept);
+    **kept = G;
     return MPMX_OK;
 }
 
@@ -1110,15 +1110,14 @@ static mpmx_status substep_graph(mpmx_ctx* c, double dt) {
     int want = 1;
     for (int q : c->cg_recent) want = std::max(want, q);
     want = std::min(want, std::max(1, c->P.cg_max_iter));
-    auto& G = c->graphs[p];
     choose_sort_path(c);
-    const bool by_movers = c->sort_by_movers && c->old_keys_sorted;
-    if (!G.valid || G.dt != (float)dt || G.iters != want || c->hc->num_blocks > G.blocks + G.blocks / 4 + 64 ||
-        G.by_movers != by_movers) {
-        mpmx_status s = capture_substep(c, dt, want);
+    auto* G = &c->graphs[p][c->sort_by_movers && c->old_keys_sorted ? 1 : 0];
+    if (!G->valid || G->dt != (float)dt || G->iters != want ||
+        c->hc->num_blocks > G->blocks + G->blocks / 4 + 64) {
+        mpmx_status s = capture_substep(c, dt, want, &G);
         if (s != MPMX_OK) return s;
     }
-    HIPCHK(c, hipGraphLaunch(G.a, c->stream));
+    HIPCHK(c, hipGraphLaunch(G->a, c->stream));
     c->cur = 1 - p;
     std::swap(c->keys, c->keys_alt);   // what the captured sort did
     c->sorted = true;
@@ -1126,8 +1125,8 @@ static mpmx_status substep_graph(mpmx_ctx* c, double dt) {
     if (c->cfg.p2g_variant != 1) c->vb_perm = c->vals_alt;   // graph A's gather left v and B to graph B
     hipError_t e = hipStreamSynchronize(c->stream);          // graph A copied the counters to the host
     if (e == hipSuccess && c->dp.phase_field) {
-        if (!c->hc->cg_done && G.iters < c->P.cg_max_iter)
-            e = launch_pcg_from(c, G.iters, c->cfg.cg_check_every > 0 ? c->cfg.cg_check_every : 1);
+        if (!c->hc->cg_done && G->iters < c->P.cg_max_iter)
+            e = launch_pcg_from(c, G->iters, c->cfg.cg_check_every > 0 ? c->cfg.cg_check_every : 1);
         c->cg_spec = c->hc->cg_iters > 0 ? c->hc->cg_iters : 1;
         note_cg_iters(c, c->hc->cg_iters);
     }
@@ -1135,7 +1134,7 @@ static mpmx_status substep_graph(mpmx_ctx* c, double dt) {
         (void)finish_carry_vb(c);
         return hipfail(c, e, "substep between its graphs");
     }
-    HIPCHK(c, hipGraphLaunch(G.b, c->stream));
+    HIPCHK(c, hipGraphLaunch(G->b, c->stream));
     c->vb_perm = nullptr;
     c->sorted = false;
     ++c->substeps;

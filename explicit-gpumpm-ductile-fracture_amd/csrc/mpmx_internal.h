@@ -278,16 +278,16 @@ struct mpmx_ctx {
     int particle_wg = 256;           // threads per workgroup of the per-particle kernels
     int p2g_pct = 100, g2p_pct = 100, cg_pct = 100;   // block-kernel workgroups, % of the block count
     // captured substeps (mpmx_config.use_graph), one pair per parity of the
-    // double-buffered particle state: A = sort .. PCG (k_graph iterations) +
-    // the counter copy, B = G2P
+    // double-buffered particle state and sort path (0 every key, 1 the movers), so
+    // that a change of path captures nothing anew: A = sort .. PCG (k_graph
+    // iterations) + the counter copy, B = G2P
     struct SubstepGraph {
         hipGraphExec_t a = nullptr, b = nullptr;
         bool valid = false;
         float dt = 0.f;
         int iters = 0;
         int64_t blocks = 0;
-        bool by_movers = false;   // the sort path captured
-    } graphs[2];
+    } graphs[2][2];
     int cg_recent[8] = {0, 0, 0, 0, 0, 0, 0, 0};   // PCG iterations of the last substeps
     int* bcount = nullptr;           // [mask_words] per-word block counts, then their scan
     // grid + PCG
