@@ -1053,7 +1053,7 @@ mpmx_status mpmx_substep(mpmx_ctx* c, double dt) {
 // replays set it themselves.
 static mpmx_status capture_substep(mpmx_ctx* c, double dt, int iters, mpmx_ctx::SubstepGraph** kept) {
     const int p = c->cur;
-    const bool old_keys_sorted = c->old_keys_sorted;
+    const bool old_keys_sorted = c->old_keys_sorted, tables = c->tables_match_keys;
     uint32_t* const keys0 = c->keys;
     uint32_t* const keys1 = c->keys_alt;
     mpmx_ctx::SubstepGraph G;
@@ -1098,6 +1098,7 @@ static mpmx_status capture_substep(mpmx_ctx* c, double dt, int iters, mpmx_ctx::
     G.dt = (float)dt;
     G.iters = iters;
     G.blocks = c->hc->num_blocks;
+    G.tables = tables;
     *kept = &c->graphs[p][c->sort_by_movers && old_keys_sorted ? 1 : 0];
     destroy_graph(**kept);
     **kept = G;
@@ -1112,18 +1113,23 @@ static mpmx_status substep_graph(mpmx_ctx* c, double dt) {
     want = std::min(want, std::max(1, c->P.cg_max_iter));
     choose_sort_path(c);
     auto* G = &c->graphs[p][c->sort_by_movers && c->old_keys_sorted ? 1 : 0];
-    if (!G->valid || G->dt != (float)dt || G->iters != want ||
+    if (!G->valid || G->dt != (float)dt || G->iters != want || G->tables != c->tables_match_keys ||
         c->hc->num_blocks > G->blocks + G->blocks / 4 + 64) {
         mpmx_status s = capture_substep(c, dt, want, &G);
         if (s != MPMX_OK) return s;
     }
     HIPCHK(c, hipGraphLaunch(G->a, c->stream));
     c->cur = 1 - p;
-    std::swap(c->keys, c->keys_alt);   // what the captured sort did
+    // what the captured stages set: the sort, the tables, the stress and P2G
+    std::swap(c->keys, c->keys_alt);
     c->sorted = true;
-    c->grid_fused = c->cfg.p2g_variant != 1;
-    if (c->cfg.p2g_variant != 1) c->vb_perm = c->vals_alt;   // graph A's gather left v and B to graph B
-    hipError_t e = hipStreamSynchronize(c->stream);          // graph A copied the counters to the host
+    c->old_keys_sorted = c->tables_match_keys = true;
+    const bool scatter = c->cfg.p2g_variant == 1;
+    c->vpages_valid = scatter;
+    c->stress_fields = scatter || c->cfg.store_stress != 0;
+    c->grid_fused = c->order_ok = !scatter;
+    if (!scatter) c->vb_perm = c->vals_alt;           // graph A's gather left v and B to graph B
+    hipError_t e = hipStreamSynchronize(c->stream);   // graph A copied the counters to the host
     if (e == hipSuccess && c->dp.phase_field) {
         if (!c->hc->cg_done && G->iters < c->P.cg_max_iter)
             e = launch_pcg_from(c, G->iters, c->cfg.cg_check_every > 0 ? c->cfg.cg_check_every : 1);

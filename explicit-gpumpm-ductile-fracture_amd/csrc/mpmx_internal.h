@@ -287,6 +287,7 @@ struct mpmx_ctx {
         float dt = 0.f;
         int iters = 0;
         int64_t blocks = 0;
+        bool tables = false;   // captured with page tables of the previous keys (the movers' places come from them)
     } graphs[2][2];
     int cg_recent[8] = {0, 0, 0, 0, 0, 0, 0, 0};   // PCG iterations of the last substeps
     int* bcount = nullptr;           // [mask_words] per-word block counts, then their scan
