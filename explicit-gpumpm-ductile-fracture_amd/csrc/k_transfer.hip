@@ -376,9 +376,9 @@ static Tables tables_of(mpmx_ctx* c) {
 }
 
 // workgroups for the 2x2x2-block kernels: pct % of the last block count the
-// host saw (refreshed at every PCG check) plus a margin, a multiple of 8.  The
-// kernels stride over the device-side count, so a stale hint or any pct
-// changes only the balance, never the results.
+// host saw (refreshed at every PCG check, without a solve at every sort) plus a
+// margin, a multiple of 8.  The kernels stride over the device-side count, so a
+// stale hint or any pct changes only the balance, never the results.
 int block_grid(mpmx_ctx* c, int pct) {
     int64_t nb = c->hc->num_blocks;
     // no count seen yet (the first build): enough workgroups to fill the GPU,
