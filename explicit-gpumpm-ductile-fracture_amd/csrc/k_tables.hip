@@ -272,7 +272,7 @@ __global__ void k_page_heads(const uint32_t* __restrict__ keys, int n, const uin
 __global__ void k_page_topology(const uint32_t* __restrict__ page_key, const int* __restrict__ page2particle,
                                 const uint64_t* __restrict__ pmask, const uint64_t* __restrict__ nmask,
                                 const int* __restrict__ wpre, const int* __restrict__ spre, int* adj,
-                                int* nvp, int64_t cap_p, int vpage, DevCounts* dc) {
+                                int* nvp, int64_t cap_p, int vpage, int slot_shift, DevCounts* dc) {
     const int p = blockIdx.x * blockDim.x + threadIdx.x;
     int num_page = dc->num_page;
     num_page = num_page < cap_p ? num_page : (int)cap_p;
@@ -280,9 +280,12 @@ __global__ void k_page_topology(const uint32_t* __restrict__ page_key, const int
     const uint32_t pk = page_key[p];
 #pragma unroll
     for (int q = 0; q < 7; ++q) {
-        // -1 only past the edge of a batched scene's page space, which no
-        // node of the scene reaches
-        adj[(int64_t)q * cap_p + p] = page_rank(neighbor_key(pk, q), pmask, nmask, wpre, spre, dc->num_page);
+        // -1 only past the edge of a batched scene's page space (its slot), which
+        // no node of the scene reaches; that key lies in another slot or past
+        // the bitmaps of the batch
+        const uint32_t nk = neighbor_key(pk, q);
+        adj[(int64_t)q * cap_p + p] =
+            (nk >> slot_shift) == (pk >> slot_shift) ? page_rank(nk, pmask, nmask, wpre, spre, dc->num_page) : -1;
     }
     const int cnt = page2particle[p + 1] - page2particle[p];
     nvp[p] = (cnt + vpage - 1) / vpage;
@@ -337,7 +340,7 @@ hipError_t build_vpage_tables(mpmx_ctx* c) {
     const int pblocks = (int)((c->cap_p + 255) / 256);
     k_page_topology<<<pblocks, 256, 0, c->stream>>>(c->page_key, c->page2particle, c->pmask, c->nmask,
                                                      c->wcount, c->scount, c->adj, c->nvp, c->cap_p,
-                                                     c->P.vpage, c->dc);
+                                                     c->P.vpage, c->dp.slot_shift, c->dc);
     if ((e = scan_exclusive(c, c->nvp, c->vpo, c->cap_p, &c->dc->num_page, 0, &c->dc->num_vp)) != hipSuccess)
         return e;
     k_vtargets<<<pblocks, 256, 0, c->stream>>>(c->vpo, c->target, c->cap_p, c->cap_vp, c->dc);
