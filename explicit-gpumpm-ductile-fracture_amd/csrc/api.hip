@@ -201,14 +201,15 @@ int particle_blocks(const mpmx_ctx* c) {
 
 // the captured substeps no longer match the context (buffers, capacities or
 // launch shapes changed)
-static void destroy_graph(mpmx_ctx::SubstepGraph& g) {
+static void destroy_graph(mpmx_ctx* c, mpmx_ctx::SubstepGraph& g) {
+    if (g.valid) (void)hipStreamSynchronize(c->stream);   // its last replay may still be running
     if (g.a) (void)hipGraphExecDestroy(g.a);
     if (g.b) (void)hipGraphExecDestroy(g.b);
     g = mpmx_ctx::SubstepGraph{};
 }
 void destroy_graphs(mpmx_ctx* c) {
     for (auto& parity : c->graphs)
-        for (auto& g : parity) destroy_graph(g);
+        for (auto& g : parity) destroy_graph(c, g);
 }
 
 void note_cg_iters(mpmx_ctx* c, int iters) {
@@ -1091,7 +1092,7 @@ static mpmx_status capture_substep(mpmx_ctx* c, double dt, int iters, mpmx_ctx::
     c->gather_perm = nullptr;
     c->vb_perm = nullptr;
     if (s != MPMX_OK) {
-        destroy_graph(G);
+        destroy_graph(c, G);
         return s;
     }
     G.valid = true;
@@ -1100,7 +1101,7 @@ static mpmx_status capture_substep(mpmx_ctx* c, double dt, int iters, mpmx_ctx::
     G.blocks = c->hc->num_blocks;
     G.tables = tables;
     *kept = &c->graphs[p][c->sort_by_movers && old_keys_sorted ? 1 : 0];
-    destroy_graph(**kept);
+    destroy_graph(c, **kept);
     **kept = G;
     return MPMX_OK;
 }
